@@ -6,15 +6,15 @@
 // gfx950 layout: one wave64 integrates one time block; lane l holds the four
 // consecutive sections 4l..4l+3 in registers.  The Jacobi pressure sweep
 // exchanges the two lane-boundary pressures with DPP wave shifts, the three
-// step-control reductions run as DPP butterflies plus four readlanes, and
-// accept/reject is a lane-uniform decision.  No LDS, no barriers.  The same
+// step-control reductions run interleaved as DPP trees, and accept/reject is a
+// lane-uniform decision.  No LDS, no barriers.  The same
 // functions also run a block over a workgroup of 2 or 4 waves (2 or 1
 // sections per lane), exchanging wave-boundary values through LDS (Lay<N>
 // below); results are identical in every layout.
 //
 // Arithmetic contract (shared with the CPU oracle): FP32, every operation
 // IEEE-rounded, no contraction (built with -ffp-contract=off), IEEE division
-// where the reference uses __fdividef, tanh by cm_tanhf below, and the fixed
+// where the reference uses __fdividef, tanh by tanh_slots below, and the fixed
 // reduction tree (s0+s1)+(s2+s3) -> xor 1,2,4,8 -> (r0+r16)+(r32+r48).
 #ifndef CM_BM_DEVICE_H
 #define CM_BM_DEVICE_H
@@ -46,29 +46,47 @@ __device__ __forceinline__ float exp_reduced(float y) {
   return __builtin_ldexpf(p, (int)k);
 }
 
-// tanh: odd series below 0.55, 1 - 2/(e^{2a}+1) below 10, 1 beyond.
-__device__ __forceinline__ float cm_tanhf(float x) {
-  float a = __builtin_fabsf(x);
-  float r;
-  if (a < 0.55f) {
-    float z = a * a;
-    float q = -2.39129114e-04f;
-    q = __builtin_fmaf(q, z, 5.90027441e-04f);
-    q = __builtin_fmaf(q, z, -1.45583438e-03f);
-    q = __builtin_fmaf(q, z, 3.59212812e-03f);
-    q = __builtin_fmaf(q, z, -8.86323989e-03f);
-    q = __builtin_fmaf(q, z, 2.18694881e-02f);
-    q = __builtin_fmaf(q, z, -5.39682540e-02f);
-    q = __builtin_fmaf(q, z, 1.33333340e-01f);
-    q = __builtin_fmaf(q, z, -3.33333343e-01f);
-    r = __builtin_fmaf(a * z, q, a);
-  } else if (a < 10.0f) {
-    float e = exp_reduced(a + a);
-    r = 1.0f - 2.0f / (e + 1.0f);
-  } else {
-    r = 1.0f;
+// tanh of a lane's N values: odd series below 0.55, 1 - 2/(e^{2a}+1) below 10,
+// 1 beyond.  The series runs for all N values together (independent chains, no
+// branch per value; odd, so it needs no sign handling); the exponential form
+// follows only when some lane of the wave holds an argument of 0.55 or more.
+// There the divisor e + 1 lies in [2, 5e8], so the division is the correctly
+// rounded sequence of reciprocal, Newton step and two residual corrections
+// without range scaling.  (A NaN may leave as a NaN or, as beyond 10, as 1; it
+// meets the same NaN again in psi's own term of the same sum.)
+template <int N>
+__device__ __forceinline__ void tanh_slots(const float (&x)[N], float (&r)[N]) {
+  float q[N], z[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    z[j] = x[j] * x[j];
+    q[j] = __builtin_fmaf(-2.39129114e-04f, z[j], 5.90027441e-04f);
   }
-  return __builtin_copysignf(r, x);
+  constexpr float c[7] = {-1.45583438e-03f, 3.59212812e-03f, -8.86323989e-03f, 2.18694881e-02f,
+                          -5.39682540e-02f, 1.33333340e-01f, -3.33333343e-01f};
+#pragma unroll
+  for (int i = 0; i < 7; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) q[j] = __builtin_fmaf(q[j], z[j], c[i]);
+  float m = __builtin_fabsf(x[0]);
+#pragma unroll
+  for (int j = 1; j < N; ++j) m = fmaxf(m, __builtin_fabsf(x[j]));
+#pragma unroll
+  for (int j = 0; j < N; ++j) r[j] = __builtin_fmaf(x[j] * z[j], q[j], x[j]);
+  if (__builtin_amdgcn_ballot_w64(!(m < 0.55f)) != 0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float a = __builtin_fabsf(x[j]);
+      const float d = exp_reduced(a + a) + 1.0f;
+      float y = __builtin_amdgcn_rcpf(d);
+      y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+      float t = 2.0f * y;
+      t = __builtin_fmaf(__builtin_fmaf(-d, t, 2.0f), y, t);
+      t = __builtin_fmaf(__builtin_fmaf(-d, t, 2.0f), y, t);
+      const float big = a < 10.0f ? 1.0f - t : 1.0f;
+      r[j] = a < 0.55f ? r[j] : __builtin_copysignf(big, x[j]);
+    }
+  }
 }
 
 // ------------------------------------------------------------ DPP ------
@@ -106,18 +124,45 @@ __device__ __forceinline__ float tree_sum(float x0, float x1, float x2, float x3
   s = s + row_bcast31(s);
   return readlane(s, 63);
 }
-__device__ __forceinline__ float tree_max(float x0, float x1, float x2, float x3) {
-  float s = fmaxf(fmaxf(x0, x1), fmaxf(x2, x3));
-  s = fmaxf(s, quad_xor1(s));
-  s = fmaxf(s, quad_xor2(s));
-  s = fmaxf(s, row_half_mirror(s));
-  s = fmaxf(s, row_mirror(s));
-  s = fmaxf(s, row_bcast15(s));
-  s = fmaxf(s, row_bcast31(s));
-  return readlane(s, 63);
+// The cross-lane part of the tree for three (or two) per-lane values at once.
+// A DPP operand needs two other instructions after the one that wrote it, so
+// one tree alone waits in every step; three interleaved trees never do.  One
+// asm block, because the compiler keeps the trees apart and, for the maximum,
+// adds a canonicalising move and operation per step (values here come from
+// arithmetic, so no operand is a signalling NaN).
+#define CM_TREE3(op0, op1, op2, ctrl)                                   \
+  op0 " %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  op1 " %1, %1, %1 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  op2 " %2, %2, %2 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define CM_TREE2(ctrl)                                                          \
+  "v_add_f32_dpp %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  "v_add_f32_dpp %1, %1, %1 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  "s_nop 0\n\t"
+#define CM_TREE_STEPS(step) \
+  step("quad_perm:[1,0,3,2]") step("quad_perm:[2,3,0,1]") step("row_half_mirror") step("row_mirror") \
+      step("row_bcast:15") step("row_bcast:31")
+#define CM_TREE_MAX_SUM_SUM(ctrl) CM_TREE3("v_max_f32_dpp", "v_add_f32_dpp", "v_add_f32_dpp", ctrl)
+#define CM_TREE_SUM3(ctrl) CM_TREE3("v_add_f32_dpp", "v_add_f32_dpp", "v_add_f32_dpp", ctrl)
+#define CM_TREE_READ3 \
+  "v_readlane_b32 %3, %0, 63\n\tv_readlane_b32 %4, %1, 63\n\tv_readlane_b32 %5, %2, 63"
+__device__ __forceinline__ void tree_max_sum_sum(float &x, float &y, float &z) {
+  float a, b, c;
+  asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE_MAX_SUM_SUM) CM_TREE_READ3
+      : "+&v"(x), "+&v"(y), "+&v"(z), "=s"(a), "=s"(b), "=s"(c));
+  x = a; y = b; z = c;
 }
-
-
+__device__ __forceinline__ void tree_sum3(float &x, float &y, float &z) {
+  float a, b, c;
+  asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE_SUM3) CM_TREE_READ3
+      : "+&v"(x), "+&v"(y), "+&v"(z), "=s"(a), "=s"(b), "=s"(c));
+  x = a; y = b; z = c;
+}
+__device__ __forceinline__ void tree_sum2(float &x, float &y) {
+  float a, b;
+  asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE2) "v_readlane_b32 %2, %0, 63\n\tv_readlane_b32 %3, %1, 63"
+      : "+&v"(x), "+&v"(y), "=s"(a), "=s"(b));
+  x = a; y = b;
+}
 
 #define UNROLL _Pragma("unroll")
 
@@ -249,13 +294,43 @@ struct Lay {
   __device__ __forceinline__ void reduce3(const float (&ex)[N], const float (&ey)[N], const float (&ez)[N],
                                           float &emax, float &esum, float &fsum) {
     if constexpr (N == 4) {
-      emax = tree_max(ex[0], ex[1], ex[2], ex[3]);
-      esum = tree_sum(ey[0], ey[1], ey[2], ey[3]);
-      fsum = tree_sum(ez[0], ez[1], ez[2], ez[3]);
+      emax = fmaxf(fmaxf(ex[0], ex[1]), fmaxf(ex[2], ex[3]));
+      esum = (ey[0] + ey[1]) + (ey[2] + ey[3]);
+      fsum = (ez[0] + ez[1]) + (ez[2] + ez[3]);
+      tree_max_sum_sum(emax, esum, fsum);
     } else {
       float v[3] = {part_max(ex), part_sum(ey), part_sum(ez)};
       combine<3>(v, 1u);
       emax = v[0]; esum = v[1]; fsum = v[2];
+    }
+  }
+  // sums of the squares of two or three vectors
+  __device__ __forceinline__ void sum_sq2(const float (&x)[N], const float (&y)[N], float &sx, float &sy) {
+    float a[N], b[N];
+    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; }
+    if constexpr (N == 4) {
+      sx = (a[0] + a[1]) + (a[2] + a[3]);
+      sy = (b[0] + b[1]) + (b[2] + b[3]);
+      tree_sum2(sx, sy);
+    } else {
+      float v[2] = {part_sum(a), part_sum(b)};
+      combine<2>(v, 0u);
+      sx = v[0]; sy = v[1];
+    }
+  }
+  __device__ __forceinline__ void sum_sq3(const float (&x)[N], const float (&y)[N], const float (&z)[N], float &sx,
+                                          float &sy, float &sz) {
+    float a[N], b[N], c[N];
+    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; c[j] = z[j] * z[j]; }
+    if constexpr (N == 4) {
+      sx = (a[0] + a[1]) + (a[2] + a[3]);
+      sy = (b[0] + b[1]) + (b[2] + b[3]);
+      sz = (c[0] + c[1]) + (c[2] + c[3]);
+      tree_sum3(sx, sy, sz);
+    } else {
+      float v[3] = {part_sum(a), part_sum(b), part_sum(c)};
+      combine<3>(v, 0u);
+      sx = v[0]; sy = v[1]; sz = v[2];
     }
   }
   // section 0's value (slot 0 of the lane that holds it) in every lane
@@ -305,17 +380,29 @@ struct ItemConstN {
 
 // Scalars shared by all lanes (uniform).
 struct ItemScal {
-  float w_ohc, alpha_r, Ts, al, Gme, a1, sigma_ow, eta1, eta2, dt_min, dt_max, tso, mtt, mmspt;
-  float al_over_as, dxdx, dxa0, neg_a1, neg_a2, neg_w, neg_as, span;
+  float w_ohc, alpha_r, Ts, al, Gme, a1, eta1, eta2, dt_min, dt_max, tso, mtt, mmspt;
+  float al_over_as, dxdx, dxa0, neg_a2, neg_as, span;
+  double inv_sigma_ow;
 };
 
-// Integration state of an item (include/cochlea.cuh:13620-13700 names in comments).
+// One side of an integration step (include/cochlea.cuh:13620-13700 names:
+// displacement, velocity, acceleration, psi, its derivative, xi's derivative
+// and xi per section, and the oval window's displacement, velocity and
+// acceleration).
+template <int N>
+struct HalfN {
+  float d[N], v[N], a[N], psi[N], psid[N], xis[N], xi[N];
+  float ow_d, ow_v, ow_a;
+};
+
+// Integration state of an item: two sides, the committed one and the one the
+// passes of a step work on.  Which is which alternates from step to step, so
+// a commit copies nothing.
 template <int N>
 struct ItemStateN {
-  float pd[N], pv[N], pa[N], ppsi[N], ppsid[N], pxis[N], pxi[N];    // committed
-  float nd[N], nv[N], na[N], npsi[N], npsid[N], nxis[N], nxi[N], Ptm[N];
+  HalfN<N> A, B;
+  float Ptm[N];
   float p[N];                                                          // resident pressure
-  float ow_pd, ow_pv, ow_pa, ow_nd, ow_nv, ow_na;                      // oval window
   float dt, t, sx0, sx1;
   int in_s;
   float c_fail, c_dt, c_steps, c_passes;                               // sx[11], sx[12], sx[13], sx[15]
@@ -325,6 +412,7 @@ struct ItemStateN {
 };
 using ItemConst = ItemConstN<4>;
 using ItemState = ItemStateN<4>;
+using Half = HalfN<4>;
 
 // The functions below take the per-lane section constants as K: ItemConstN<N>
 // (every row in registers) or a type with the same members whose rarely read
@@ -355,40 +443,96 @@ __device__ __forceinline__ void jacobi_sweep(Lay<N> &L, const float (&Y)[N], con
     q[j] = (Y[j] - coupling<N>(j, k.low, pl, pr)) * k.rsm[j];
   }
 }
+// Sweeps of the one-wave layout in asm: 12 VALU instructions per sweep and no
+// wait.  t <- sweep(p) reads p through DPP in its first two instructions, and
+// the products that feed them (slots 0 and 3) come first among the previous
+// sweep's last four, so every DPP operand is at least two instructions old;
+// the compiler's loop took 13 and a wait.  The 13th was slot 3's coupling:
+// l_255 = 0 and no section follows 255, so there it is l p_254 + 0, which does
+// not change from sweep to sweep; %[a3]'s lane 63 holds it, and the shift
+// without bound_ctrl leaves that lane alone.  (p_254 only enters it as 0 times
+// itself; a non-finite p_254 still makes it NaN from the next call on.)
+#define CM_SWEEP(p0, p1, p2, p3, t0, t1, t2, t3)                                                      \
+  "v_add_f32_dpp %[" t0 "], %[" p3 "], %[" p1 "] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  "v_add_f32_dpp %[a3], %[" p0 "], %[" p2 "] wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"              \
+  "v_add_f32 %[" t1 "], %[" p0 "], %[" p2 "]\n\t"                                                    \
+  "v_fma_f32 %[" t2 "], %[low], %[" p1 "], %[" p3 "]\n\t"                                            \
+  "v_sub_f32 %[" t0 "], %[Y0], %[" t0 "]\n\t"                                                        \
+  "v_sub_f32 %[" t3 "], %[Y3], %[a3]\n\t"                                                            \
+  "v_sub_f32 %[" t1 "], %[Y1], %[" t1 "]\n\t"                                                        \
+  "v_sub_f32 %[" t2 "], %[Y2], %[" t2 "]\n\t"                                                        \
+  "v_mul_f32 %[" t0 "], %[r0], %[" t0 "]\n\t"                                                        \
+  "v_mul_f32 %[" t3 "], %[r3], %[" t3 "]\n\t"                                                        \
+  "v_mul_f32 %[" t1 "], %[r1], %[" t1 "]\n\t"                                                        \
+  "v_mul_f32 %[" t2 "], %[r2], %[" t2 "]\n\t"
+#define CM_SWEEP_PT CM_SWEEP("p0", "p1", "p2", "p3", "t0", "t1", "t2", "t3")
+#define CM_SWEEP_TP CM_SWEEP("t0", "t1", "t2", "t3", "p0", "p1", "p2", "p3")
+#define CM_SWEEP_IN                                                                                     \
+  [Y0] "v"(Y[0]), [Y1] "v"(Y[1]), [Y2] "v"(Y[2]), [Y3] "v"(Y[3]), [r0] "v"(r[0]), [r1] "v"(r[1]),       \
+      [r2] "v"(r[2]), [r3] "v"(r[3]), [low] "v"(low)
+// J >= 0 sweeps; PAIRS (1 or 2) pairs per trip of the loop.
+template <int PAIRS>
+__device__ __forceinline__ void sweeps_asm(const float (&Y)[4], const float (&r)[4], float low, float (&p)[4], int J) {
+  float a3 = low * p[2] + 0.0f;
+  float t0, t1, t2, t3;
+  int n = J / (2 * PAIRS);
+  if (n > 0) {
+    if constexpr (PAIRS == 1)
+      asm("s_nop 1\n"
+          "1:\n\t" CM_SWEEP_PT CM_SWEEP_TP
+          "s_sub_i32 %[n], %[n], 1\n\ts_cmp_lg_u32 %[n], 0\n\ts_cbranch_scc1 1b\n\t"
+          : [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [p2] "+&v"(p[2]), [p3] "+&v"(p[3]), [a3] "+&v"(a3), [n] "+&s"(n),
+            [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
+          : CM_SWEEP_IN
+          : "scc");
+    else
+      asm("s_nop 1\n"
+          "1:\n\t" CM_SWEEP_PT CM_SWEEP_TP CM_SWEEP_PT CM_SWEEP_TP
+          "s_sub_i32 %[n], %[n], 1\n\ts_cmp_lg_u32 %[n], 0\n\ts_cbranch_scc1 1b\n\t"
+          : [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [p2] "+&v"(p[2]), [p3] "+&v"(p[3]), [a3] "+&v"(a3), [n] "+&s"(n),
+            [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
+          : CM_SWEEP_IN
+          : "scc");
+  }
+  if (PAIRS == 2 && (J & 2))
+    asm("s_nop 1\n\t" CM_SWEEP_PT CM_SWEEP_TP
+        : [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [p2] "+&v"(p[2]), [p3] "+&v"(p[3]), [a3] "+&v"(a3), [t0] "=&v"(t0),
+          [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
+        : CM_SWEEP_IN);
+  if (J & 1) {
+    asm("s_nop 1\n\t" CM_SWEEP_PT
+        : [a3] "+&v"(a3), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
+        : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), CM_SWEEP_IN);
+    p[0] = t0; p[1] = t1; p[2] = t2; p[3] = t3;
+  }
+}
+
 // J is wave-uniform: the count goes to a scalar register.  U (1, 2 or 4) is
-// the unroll of the sweep loop, a launch knob of the autotuner: with U >= 2
-// sweeps come in pairs so the two iterates alternate between register sets
-// instead of being copied back each sweep; U = 4 runs two pairs per loop trip.
-// Every U performs the same sweeps in the same order, so results are identical.
+// the unroll of the sweep loop, a launch knob of the autotuner: sweeps come in
+// pairs (U = 2) or two pairs (U = 4) per trip, so the two iterates alternate
+// between register sets; U = 1 copies the iterate back each sweep.  Every U
+// performs the same sweeps in the same order, so results are identical.
 template <int U = 2, int N, class K>
 __device__ __forceinline__ void jacobi_sweeps(Lay<N> &L, const float (&Y)[N], const K &k, float (&p)[N],
                                               int J) {
   static_assert(U == 1 || U == 2 || U == 4, "unroll 1, 2 or 4");
   J = __builtin_amdgcn_readfirstlane(J);
-  float q[N];
-  if (U == 1) {
-    for (int i = 0; i < J; ++i) {
+  if constexpr (N == 4 && U != 1) {
+    const float r[4] = {k.rsm[0], k.rsm[1], k.rsm[2], k.rsm[3]};
+    sweeps_asm<U / 2>(Y, r, k.low, p, J);
+  } else {
+    float q[N];
+    int i = 0;
+    if (U != 1) {
+      for (; i + 2 <= J; i += 2) {
+        jacobi_sweep(L, Y, k, p, q);
+        jacobi_sweep(L, Y, k, q, p);
+      }
+    }
+    for (; i < J; ++i) {
       jacobi_sweep(L, Y, k, p, q);
       UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
     }
-    return;
-  }
-  int i = 0;
-  if (U == 4) {
-    for (; i + 4 <= J; i += 4) {
-      jacobi_sweep(L, Y, k, p, q);
-      jacobi_sweep(L, Y, k, q, p);
-      jacobi_sweep(L, Y, k, p, q);
-      jacobi_sweep(L, Y, k, q, p);
-    }
-  }
-  for (; i + 2 <= J; i += 2) {
-    jacobi_sweep(L, Y, k, p, q);
-    jacobi_sweep(L, Y, k, q, p);
-  }
-  if (J & 1) {
-    jacobi_sweep(L, Y, k, p, q);
-    UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
   }
 }
 
@@ -412,11 +556,21 @@ __device__ __forceinline__ float resid2(Lay<N> &L, const float (&Y)[N], const K 
   UNROLL for (int j = 0; j < N; ++j) r[j] = r[j] * r[j];
   return L.sum(r);
 }
-template <int N>
-__device__ __forceinline__ float sum_sq(Lay<N> &L, const float (&x)[N]) {
-  float q[N];
-  UNROLL for (int j = 0; j < N; ++j) q[j] = x[j] * x[j];
-  return L.sum(q);
+// Squared residual of p and, from the same couplings, the next sweep's iterate q.
+template <int N, class K>
+__device__ __forceinline__ float resid2_sweep(Lay<N> &L, const float (&Y)[N], const K &k, const float (&p)[N],
+                                              float (&q)[N]) {
+  float left, right, r[N];
+  L.nbrs(p[N - 1], p[0], left, right);
+  UNROLL for (int j = 0; j < N; ++j) {
+    const float pl = j == 0 ? left : p[j - 1];
+    const float pr = j == N - 1 ? right : p[j + 1];
+    const float c = coupling<N>(j, k.low, pl, pr);
+    r[j] = Y[j] - (c + k.mf[j] * p[j]);
+    r[j] = r[j] * r[j];
+    q[j] = (Y[j] - c) * k.rsm[j];
+  }
+  return L.sum(r);
 }
 
 template <bool TOL, int N>
@@ -450,21 +604,22 @@ __device__ __forceinline__ void item_setup(const BmLaunch &a, const cm_bm_item &
 
   c.w_ohc = sc.w_ohc; c.alpha_r = sc.alpha_r; c.Ts = sc.Ts;
   c.al = sc.alpha_l; c.Gme = sc.Gme; c.a1 = sc.a1;
-  c.sigma_ow = sc.sigma_ow; c.eta1 = sc.eta1; c.eta2 = sc.eta2;
+  c.eta1 = sc.eta1; c.eta2 = sc.eta2;
   c.dt_min = sc.dt_min; c.dt_max = sc.dt_max; c.tso = sc.time_step_out;
   c.mtt = it.tol; c.mmspt = it.m1tol;
   c.al_over_as = sc.alpha_l / sc.alpha_s;
   c.dxdx = sc.delta_x * sc.delta_x;
   c.dxa0 = sc.delta_x * sc.a0;
-  c.neg_a1 = -sc.a1; c.neg_a2 = -sc.a2; c.neg_w = -sc.w_ohc; c.neg_as = -sc.alpha_s;
+  c.neg_a2 = -sc.a2; c.neg_as = -sc.alpha_s;
   c.span = (float)(it.mesi - it.mosi);
+  c.inv_sigma_ow = 1.0 / (double)sc.sigma_ow;
 
   UNROLL for (int j = 0; j < N; ++j) {
-    s.pd[j] = 0; s.pv[j] = 0; s.pa[j] = 0; s.ppsi[j] = 0; s.ppsid[j] = 0; s.pxis[j] = 0; s.pxi[j] = 0;
-    s.nd[j] = 0; s.nv[j] = 0; s.na[j] = 0; s.npsi[j] = 0; s.npsid[j] = 0; s.nxis[j] = 0; s.nxi[j] = 0;
+    s.A.d[j] = 0; s.A.v[j] = 0; s.A.a[j] = 0; s.A.psi[j] = 0; s.A.psid[j] = 0; s.A.xis[j] = 0; s.A.xi[j] = 0;
     s.Ptm[j] = 0; s.p[j] = 0;
   }
-  s.ow_pd = 0; s.ow_pv = 0; s.ow_pa = 0; s.ow_nd = 0; s.ow_nv = 0; s.ow_na = 0;
+  s.A.ow_d = 0; s.A.ow_v = 0; s.A.ow_a = 0;
+  s.B = s.A;
   s.dt = sc.time_step;
   s.t = 0.0f;
   s.in_s = it.start;
@@ -476,143 +631,174 @@ __device__ __forceinline__ void item_setup(const BmLaunch &a, const cm_bm_item &
   s.ctb = 0.f; s.clb = 0.f; s.cjb = 0.f;
 }
 
-// Predictor (Euler) or corrector (trapezoid) update, :13770-13820.
+// Predictor (Euler) update of side n from the committed side o, :13770-13820.
+// The trapezoids keep their own halving, ((a + b) 0.5) dt: folding it into
+// 0.5 dt would save an instruction each and rounds alike except for sums below
+// 2^-125, but the tails of decaying signals reach those.
 template <int N>
-__device__ __forceinline__ void pass_begin(ItemStateN<N> &s, bool predictor) {
-  const float dt = s.dt;
-  if (predictor) {
-    UNROLL for (int j = 0; j < N; ++j) {
-      s.nxi[j] = s.pxis[j] * dt + s.pxi[j];
-      s.nv[j] = s.pa[j] * dt + s.pv[j];
-      s.nd[j] = ((s.pv[j] + s.nv[j]) * 0.5f) * dt + s.pd[j];
-      s.npsi[j] = s.ppsid[j] * dt + s.ppsi[j];
-    }
-    s.ow_nd = s.ow_pv * dt + s.ow_pd;
-    s.ow_nv = s.ow_pa * dt + s.ow_pv;
-  } else {
-    UNROLL for (int j = 0; j < N; ++j) {
-      s.nv[j] = ((s.pa[j] + s.na[j]) * 0.5f) * dt + s.pv[j];
-      s.nd[j] = ((s.pv[j] + s.nv[j]) * 0.5f) * dt + s.pd[j];
-      s.nxi[j] = ((s.pxis[j] + s.nxis[j]) * 0.5f) * dt + s.pxi[j];
-      s.npsi[j] = ((s.ppsid[j] + s.npsid[j]) * 0.5f) * dt + s.ppsi[j];
-    }
-    s.ow_nd = ((s.ow_pv + s.ow_nv) * 0.5f) * dt + s.ow_pd;
-    s.ow_nv = ((s.ow_pa + s.ow_na) * 0.5f) * dt + s.ow_pv;
+__device__ __forceinline__ void predict(const HalfN<N> &o, HalfN<N> &n, float dt) {
+  UNROLL for (int j = 0; j < N; ++j) {
+    n.xi[j] = o.xis[j] * dt + o.xi[j];
+    n.v[j] = o.a[j] * dt + o.v[j];
+    n.d[j] = ((o.v[j] + n.v[j]) * 0.5f) * dt + o.d[j];
+    n.psi[j] = o.psid[j] * dt + o.psi[j];
   }
+  n.ow_d = o.ow_v * dt + o.ow_d;
+  n.ow_v = o.ow_a * dt + o.ow_v;
+}
+// Corrector (trapezoid) update.
+template <int N>
+__device__ __forceinline__ void correct(const HalfN<N> &o, HalfN<N> &n, float dt) {
+  UNROLL for (int j = 0; j < N; ++j) {
+    n.v[j] = ((o.a[j] + n.a[j]) * 0.5f) * dt + o.v[j];
+    n.d[j] = ((o.v[j] + n.v[j]) * 0.5f) * dt + o.d[j];
+    n.xi[j] = ((o.xis[j] + n.xis[j]) * 0.5f) * dt + o.xi[j];
+    n.psi[j] = ((o.psid[j] + n.psid[j]) * 0.5f) * dt + o.psi[j];
+  }
+  n.ow_d = ((o.ow_v + n.ow_v) * 0.5f) * dt + o.ow_d;
+  n.ow_v = ((o.ow_a + n.ow_a) * 0.5f) * dt + o.ow_v;
 }
 
-// TM/OHC block (passes < 2, :13839-13898), G (:13905-13909) and the right-hand
-// side with its boundaries (:13925-13954).  Returns the forcing s(t).
-template <int N, class K>
-__device__ __forceinline__ float pass_rhs(const K &k, const ItemScal &c, ItemStateN<N> &s, bool aux_pass,
-                                          const Lay<N> &L, float (&od)[N], float (&G)[N], float (&Y)[N]) {
+// Forcing s(t), the same for every pass of a step.
+template <int N>
+__device__ __forceinline__ float forcing(const ItemScal &c, const ItemStateN<N> &s) {
+  const float delta = s.t / c.Ts;
+  return s.sx1 * delta + s.sx0 * (1.0f - delta);
+}
+
+// Terms of a pass that its end (pass_finish) uses again.
+template <int N>
+struct PassTerms {
+  float eod[N];    // eta1 (xi - d)
+  float wpsi[N];   // w_ohc psi
+  float G[N];
+};
+
+// TM/OHC block (AUX: passes < 2, :13839-13898), G (:13905-13909) and the
+// right-hand side with its boundaries (:13925-13954).
+template <bool AUX, int N, class K>
+__device__ __forceinline__ void pass_rhs(const K &k, const ItemScal &c, HalfN<N> &n, float (&Ptm)[N], float sf,
+                                         const Lay<N> &L, PassTerms<N> &T, float (&Y)[N]) {
+  UNROLL for (int j = 0; j < N; ++j) T.wpsi[j] = c.w_ohc * n.psi[j];
+  float od[N];
   UNROLL for (int j = 0; j < N; ++j) {
-    od[j] = s.nxi[j] - s.nd[j];
-    const float ohc_p = (k.gam[j] * k.Sohc[j]) * od[j];
-    if (aux_pass) {
-      float aux = cm_tanhf(c.al_over_as * s.npsi[j]);
-      const float dL = c.neg_as * aux;
-      aux = aux * aux - 1.0f;
-      aux = c.al * aux;
-      float n = (c.eta2 * s.nv[j] + c.eta1 * od[j]) - c.w_ohc * s.npsi[j];
-      n = k.Stm[j] * dL + (n * k.Rtm[j]) * aux;
-      const float ptmp = k.Stm[j] * s.nxi[j] + ohc_p;
-      n = ptmp - k.gam[j] * n;
+    od[j] = n.xi[j] - n.d[j];
+    T.eod[j] = c.eta1 * od[j];
+  }
+  if constexpr (AUX) {
+    float x[N], th[N];
+    UNROLL for (int j = 0; j < N; ++j) x[j] = c.al_over_as * n.psi[j];
+    tanh_slots<N>(x, th);
+    UNROLL for (int j = 0; j < N; ++j) {
+      const float ohc_p = (k.gam[j] * k.Sohc[j]) * od[j];
+      const float dL = c.neg_as * th[j];
+      const float aux = c.al * (th[j] * th[j] - 1.0f);
+      float m = (c.eta2 * n.v[j] + T.eod[j]) - T.wpsi[j];
+      m = k.Stm[j] * dL + (m * k.Rtm[j]) * aux;
+      const float sxi = k.Stm[j] * n.xi[j];
+      m = (sxi + ohc_p) - k.gam[j] * m;
       float den = (k.gam[j] * aux) * c.eta2 - 1.0f;
       den = k.Rtm[j] * den;
-      s.nxis[j] = n / den;
-      s.Ptm[j] = k.Rtm[j] * s.nxis[j] + k.Stm[j] * s.nxi[j];
+      n.xis[j] = m / den;
+      Ptm[j] = k.Rtm[j] * n.xis[j] + sxi;
     }
-    float g = s.nv[j] * s.nv[j];
-    g = k.R[j] * (c.alpha_r * g + 1.0f);
-    g = g * s.nv[j] + k.S[j] * s.nd[j];
-    G[j] = -g - s.Ptm[j];
-    Y[j] = (c.dxdx * G[j]) * k.Q[j];
   }
-  const float delta = s.t / c.Ts;
-  const float sf = s.sx1 * delta + s.sx0 * (1.0f - delta);
-  const float Y0 = c.dxa0 * (((c.neg_a2 * s.ow_nv) - c.a1 * s.ow_nd) + c.Gme * sf);
-  if (L.sec0()) Y[0] = Y0;
-  if (L.last()) Y[N - 1] = 0.0f;
-  return sf;
+  UNROLL for (int j = 0; j < N; ++j) {
+    float g = n.v[j] * n.v[j];
+    g = k.R[j] * (c.alpha_r * g + 1.0f);
+    g = g * n.v[j] + k.S[j] * n.d[j];
+    T.G[j] = -g - Ptm[j];
+    Y[j] = (c.dxdx * T.G[j]) * k.Q[j];
+  }
+  const float Y0 = c.dxa0 * (((c.neg_a2 * n.ow_v) - c.a1 * n.ow_d) + c.Gme * sf);
+  Y[0] = L.sec0() ? Y0 : Y[0];
+  Y[N - 1] = L.last() ? 0.0f : Y[N - 1];
 }
 
 // Jacobi until |Y - A p|_2 <= tol |Y|_2 (checked every check_every sweeps,
 // capped at max_sweeps); returns the sweeps done.  rr is |Y - A p|_2^2 of the
-// incoming p (the guess selection has already computed it).
+// incoming p (the guess selection has already computed it).  A check shares
+// its couplings with the sweep that follows when it fails, and that sweep's
+// other instructions fill the reduction's waits.
 template <int U = 2, int N, class K>
 __device__ __forceinline__ int jacobi_tol(Lay<N> &L, const cm_bm_scalars &sc, const K &k,
                                           const float (&Y)[N], float yy, float (&p)[N], float rr) {
   const float tau2 = sc.tol_rel * sc.tol_rel;
+  const float lim = tau2 * yy;
   int J = 0;
+  if (rr <= lim || J >= sc.max_sweeps) return J;
+  int kk = sc.check_every < sc.max_sweeps ? sc.check_every : sc.max_sweeps;
+  jacobi_sweeps<U>(L, Y, k, p, kk);
   for (;;) {
-    if (rr <= tau2 * yy || J >= sc.max_sweeps) break;
-    const int kk = sc.check_every < sc.max_sweeps - J ? sc.check_every : sc.max_sweeps - J;
-    jacobi_sweeps<U>(L, Y, k, p, kk);
     J += kk;
-    rr = resid2(L, Y, k, p);
+    float q[N];
+    rr = resid2_sweep(L, Y, k, p, q);
+    if (rr <= lim || J >= sc.max_sweeps) return J;
+    kk = sc.check_every < sc.max_sweeps - J ? sc.check_every : sc.max_sweeps - J;
+    UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
+    jacobi_sweeps<U>(L, Y, k, p, kk - 1);
   }
-  return J;
 }
 
 // Acceleration, oval-window acceleration and psi derivative, :13989-14013.
+// The oval window's division by the constant sigma_ow is a product with its
+// reciprocal in FP64: a quotient of two floats is at least 2^-49 (relative)
+// from the midpoint of two floats, the product within 2^-52 of the quotient,
+// so it rounds to the same float (in the normal range).
 template <int N, class K>
-__device__ __forceinline__ void pass_finish(Lay<N> &L, const K &k, const ItemScal &c, ItemStateN<N> &s,
-                                            const float (&od)[N], const float (&G)[N], float sf) {
-  UNROLL for (int j = 0; j < N; ++j) s.na[j] = (s.p[j] + G[j]) * k.rmass[j];
+__device__ __forceinline__ void pass_finish(Lay<N> &L, const K &k, const ItemScal &c, HalfN<N> &n,
+                                            const float (&p)[N], const PassTerms<N> &T, float sf) {
+  UNROLL for (int j = 0; j < N; ++j) n.a[j] = (p[j] + T.G[j]) * k.rmass[j];
   {
-    const float p0 = L.sec0_value(s.p[0]);
-    const float NN1 = c.neg_a2 * s.ow_nv;
+    const float p0 = L.sec0_value(p[0]);
+    const float NN1 = c.neg_a2 * n.ow_v;
     const float NN2 = c.Gme * sf + p0;
-    const float NN3 = c.neg_a1 * s.ow_nd;
-    s.ow_na = ((NN1 + NN2) + NN3) / c.sigma_ow;
+    const float x = (NN1 + NN2) - c.a1 * n.ow_d;
+    n.ow_a = (float)((double)x * c.inv_sigma_ow);
   }
   UNROLL for (int j = 0; j < N; ++j)
-    s.npsid[j] = (c.eta1 * od[j] + c.eta2 * (s.nxis[j] - s.nv[j])) + c.neg_w * s.npsi[j];
+    n.psid[j] = (T.eod[j] + c.eta2 * (n.xis[j] - n.v[j])) - T.wpsi[j];
 }
 
-// Step control (:14021-14088) and the pass counter; Q1 lane-0 semantics.
+// Step control (:14021-14088); Q1 lane-0 semantics.  Returns whether the step
+// needs another pass.  L = (emax dt) / esum only meets 6 and 0.5, so it is not
+// divided out: the float quotient is above 6 where the exact one is above the
+// midpoint 6 + 2^-22 (a tie rounds to 6), and below 0.5 where the exact one is
+// below 0.5 - 2^-26; esum times either bound is exact in FP64.
 template <int N>
-__device__ __forceinline__ void pass_control(Lay<N> &L, const cm_bm_scalars &sc, const ItemScal &c,
-                                             ItemStateN<N> &s, const float (&vref)[N], const float (&aref)[N],
-                                             int &out_loop, int &reset, int &another) {
-  if (reset == 0) {
-    float ex[N], ey[N], ez[N];
-    UNROLL for (int j = 0; j < N; ++j) {
-      ex[j] = __builtin_fabsf(aref[j] - s.na[j]);
-      ey[j] = __builtin_fabsf(s.nv[j] - vref[j]);
-      ez[j] = ey[j] - fmaxf(c.mtt, s.nv[j] * s.dt);
-    }
-    float emax, esum, fsum;
-    L.reduce3(ex, ey, ez, emax, esum, fsum);
-    if (sc.decision_mode == 1) { emax = 0.f; esum = 0.f; fsum = 0.f; }
-    float Lr;
-    if (esum > c.mmspt) { Lr = emax * s.dt; Lr = Lr / esum; } else Lr = 0.0f;
-    if (Lr > 6.0f) {
-      s.dt = s.dt * 0.5f;
-      if (s.dt < c.dt_min) s.dt = c.dt_min;
-      another = 0; reset = 1;
-    } else if (fsum > 0.0f) {
-      another = 1; reset = 0;
-    } else if (Lr < 0.5f) {
-      s.dt = s.dt * 2.0f;
-      if (s.dt > c.dt_max) s.dt = c.dt_max;
-      another = 0; reset = 1;
-    } else {
-      another = 1; reset = 0;
-    }
-  } else {
-    another = 1; reset = 0;
+__device__ __forceinline__ bool pass_control(Lay<N> &L, const cm_bm_scalars &sc, const ItemScal &c, float &dt,
+                                             const HalfN<N> &n, const float (&vref)[N], const float (&aref)[N]) {
+  float ex[N], ey[N], ez[N];
+  UNROLL for (int j = 0; j < N; ++j) {
+    ex[j] = __builtin_fabsf(aref[j] - n.a[j]);
+    ey[j] = __builtin_fabsf(n.v[j] - vref[j]);
+    ez[j] = ey[j] - fmaxf(c.mtt, n.v[j] * dt);
   }
-  out_loop++;
-  if (out_loop >= sc.max_passes) { another = 0; reset = 1; s.c_fail = 1.f; }
+  float emax, esum, fsum;
+  L.reduce3(ex, ey, ez, emax, esum, fsum);
+  if (sc.decision_mode == 1) { emax = 0.f; esum = 0.f; fsum = 0.f; }
+  bool above = false, below = true;   // L > 6, L < 0.5
+  if (esum > c.mmspt) {
+    const double e = esum, q = emax * dt;
+    above = q > e * (6.0 + 0x1p-22);
+    below = q < e * (0.5 - 0x1p-26);
+  }
+  if (above) {
+    dt = dt * 0.5f;
+    if (dt < c.dt_min) dt = c.dt_min;
+    return false;
+  }
+  if (fsum > 0.0f || !below) return true;
+  dt = dt * 2.0f;
+  if (dt > c.dt_max) dt = c.dt_max;
+  return false;
 }
 
-// Commit of a step: counters, sample advance with output row (:14130-14203),
-// state shift and local time (:14212-14230).
+// Commit of a step whose passes left side n: counters, sample advance with
+// output row (:14130-14203) and local time (:14212-14230).
 template <int N>
 __device__ __forceinline__ void step_commit(const BmLaunch &a, const cm_bm_item &it, const ItemScal &c,
-                                            ItemStateN<N> &s, int out_loop, const Lay<N> &L) {
+                                            ItemStateN<N> &s, const HalfN<N> &n, int out_loop, const Lay<N> &L) {
   s.c_steps += 1.0f;
   s.c_dt += s.dt;
   s.c_passes += (float)out_loop;
@@ -632,9 +818,9 @@ __device__ __forceinline__ void step_commit(const BmLaunch &a, const cm_bm_item 
           // store costs it a spill)
           if constexpr (N == 4)
             *reinterpret_cast<float4 *>(a.speeds + (int64_t)s.in_s * CM_SECTIONS + 4 * L.lane) =
-                make_float4(s.nv[0], s.nv[1], s.nv[2], s.nv[3]);
+                make_float4(n.v[0], n.v[1], n.v[2], n.v[3]);
           else
-            st_slots<N>(a.speeds + (int64_t)s.in_s * CM_SECTIONS + L.base(), s.nv);
+            st_slots<N>(a.speeds + (int64_t)s.in_s * CM_SECTIONS + L.base(), n.v);
         }
         if (L.sec0()) {
           if (a.failed_nodes) a.failed_nodes[s.in_s] = (int32_t)s.c_fail;
@@ -651,11 +837,6 @@ __device__ __forceinline__ void step_commit(const BmLaunch &a, const cm_bm_item 
     s.c_fail = 0.f; s.c_dt = 0.f; s.c_steps = 0.f; s.c_passes = 0.f;
     s.in_s++;
   }
-  UNROLL for (int j = 0; j < N; ++j) {
-    s.pd[j] = s.nd[j]; s.pv[j] = s.nv[j]; s.pa[j] = s.na[j]; s.ppsi[j] = s.npsi[j];
-    s.ppsid[j] = s.npsid[j]; s.pxis[j] = s.nxis[j]; s.pxi[j] = s.nxi[j];
-  }
-  s.ow_pd = s.ow_nd; s.ow_pv = s.ow_nv; s.ow_pa = s.ow_na;
   s.t += s.dt;
 }
 
@@ -679,23 +860,102 @@ __device__ __forceinline__ void item_final(const BmLaunch &a, const ItemStateN<N
 // that lowers the residual (ties keep the previous pressure).  The previous
 // step's pressure and dt_prev live in LDS (pold[lane], first N floats, and
 // pold[64].x, one copy per wave).  Returns the squared residual of the plain
-// guess; *rre gets the extrapolation's, and p holds the extrapolation on
-// return when keep_lin, else the choice.
+// guess; rre gets the extrapolation's and yy |Y|^2, and p holds the
+// extrapolation on return when keep_lin, else the choice.
 template <int N, class K>
 __device__ __forceinline__ float extrapolate_guess(Lay<N> &L, const K &k, const float (&Y)[N], float dt,
-                                                   float4 *pold, float (&p)[N], float &rre, bool keep_lin) {
+                                                   float4 *pold, float (&p)[N], float &rre, float &yy,
+                                                   bool keep_lin) {
   float *dt_prev = reinterpret_cast<float *>(pold + 64);
   float *mine = reinterpret_cast<float *>(pold + L.lane);
   const float rho = dt / *dt_prev;
-  const float rr0 = resid2(L, Y, k, p);
-  float po[N];
+  float po[N], r0[N], r1[N];
   ld_slots<N>(mine, po);
   st_slots<N>(mine, p);
+  resid_vec(L, Y, k, p, r0);
   UNROLL for (int j = 0; j < N; ++j) p[j] = p[j] + rho * (p[j] - po[j]);
-  rre = resid2(L, Y, k, p);
+  resid_vec(L, Y, k, p, r1);
+  float rr0;
+  L.sum_sq3(r0, r1, Y, rr0, rre, yy);
   if (!keep_lin && !(rre < rr0)) ld_slots<N>(mine, p);
   if (L.lane == 0) *dt_prev = dt;
   return rr0;
+}
+
+// The pressure solve of a corrector pass: fixed sweeps, or to the tolerance
+// from the resident pressure.
+template <bool TOL, int U, int N, class K>
+__device__ __forceinline__ int solve_pass(Lay<N> &L, const cm_bm_scalars &sc, const K &k, const float (&Y)[N],
+                                          float (&p)[N], int J_fixed) {
+  if constexpr (TOL) {
+    float r[N], yy, rr;
+    resid_vec(L, Y, k, p, r);
+    L.sum_sq2(r, Y, rr, yy);
+    return jacobi_tol<U>(L, sc, k, Y, yy, p, rr);
+  } else {
+    jacobi_sweeps<U>(L, Y, k, p, J_fixed);
+    return J_fixed;
+  }
+}
+
+// One integration step, include/cochlea.cuh:13760-14230: committed side o to
+// side n.  The predictor pass, the first corrector pass (which repeats the
+// TM/OHC block) and the further ones are written out one after another, so
+// that none carries the others' branches and selections.
+// Bound: instruction issue.  One wave per SIMD issues an instruction every 5 to
+// 6 cycles whatever it depends on; three reach about 3 cycles (FP32) and 4.2
+// (DPP, FP64).  So the step is written for few instructions: per block-step of
+// the reference method 1589 VALU and 122 SALU, where one pass loop for all
+// kinds of pass, a branch per tanh, divided-out step control and copied states
+// took 1793 and 246 (600 tones of 200 ms, 20-90 dB).  5 blocks: 141 -> 111 ms;
+// 610 blocks, extrapolated guess: 183 -> 143 ms; 6000 blocks: 408 -> 380 ms.
+template <int N, bool TOL, int WS, int U>
+__device__ __forceinline__ void step(const BmLaunch &a, const cm_bm_item &it, Lay<N> &L, const ItemConstN<N> &k,
+                                     const ItemScal &c, ItemStateN<N> &s, const HalfN<N> &o, HalfN<N> &n,
+                                     float4 *pold) {
+  const float sf = forcing(c, s);
+  PassTerms<N> T;
+  float Y[N];
+  int J;
+  predict(o, n, s.dt);
+  pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
+  if constexpr (TOL && WS == 1) {
+    float rre, yy;
+    const float rr0 = extrapolate_guess(L, k, Y, s.dt, pold, s.p, rre, yy, false);
+    J = jacobi_tol<U>(L, a.sc, k, Y, yy, s.p, rre < rr0 ? rre : rr0);   // residual of the guess kept
+  } else {
+    J = solve_pass<TOL, U>(L, a.sc, k, Y, s.p, a.sc.j_slow);
+  }
+  s.n_sweeps += J;
+  pass_finish(L, k, c, n, s.p, T, sf);
+  int passes = 1;
+  bool another = passes < a.sc.max_passes;
+  if (another) {
+    float vref[N], aref[N];
+    UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
+    correct(o, n, s.dt);
+    pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
+    J = solve_pass<TOL, U>(L, a.sc, k, Y, s.p, a.sc.j_slow);
+    s.n_sweeps += J;
+    pass_finish(L, k, c, n, s.p, T, sf);
+    another = pass_control(L, a.sc, c, s.dt, n, vref, aref);
+    passes = 2;
+    if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
+    while (another) {
+      UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
+      correct(o, n, s.dt);
+      pass_rhs<false>(k, c, n, s.Ptm, sf, L, T, Y);
+      J = solve_pass<TOL, U>(L, a.sc, k, Y, s.p, a.sc.j_fast);
+      s.n_sweeps += J;
+      pass_finish(L, k, c, n, s.p, T, sf);
+      another = pass_control(L, a.sc, c, s.dt, n, vref, aref);
+      ++passes;
+      if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
+    }
+  } else {
+    s.c_fail = 1.f;
+  }
+  step_commit(a, it, c, s, n, passes, L);
 }
 
 // One time block, include/cochlea.cuh:13620-14232.  TOL selects the
@@ -713,38 +973,11 @@ __device__ void run_item(const BmLaunch &a, int item_index, Lay<N> &L, float4 *p
     pold[L.lane] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (L.lane == 0) reinterpret_cast<float *>(pold + 64)[0] = s.dt;
   }
-
+  // two steps per trip: the sides change roles without a copy
   while (s.in_s < it.mesi) {
-    int out_loop = 0, reset = 1, another = 1;
-    while (another) {
-      float vref[N], aref[N];
-      UNROLL for (int j = 0; j < N; ++j) { vref[j] = s.nv[j]; aref[j] = s.na[j]; }
-      const bool predictor = out_loop == 0 || reset;
-      if (predictor) out_loop = 0;
-      pass_begin(s, predictor);
-      float od[N], G[N], Y[N];
-      const float sf = pass_rhs(k, c, s, out_loop < 2, L, od, G, Y);
-      int J;
-      if (TOL) {
-        const float yy = sum_sq(L, Y);
-        float rr;
-        if (WS == 1 && out_loop == 0) {
-          float rre;
-          const float rr0 = extrapolate_guess(L, k, Y, s.dt, pold, s.p, rre, false);
-          rr = rre < rr0 ? rre : rr0;   // residual of the guess kept
-        } else {
-          rr = resid2(L, Y, k, s.p);
-        }
-        J = jacobi_tol<U>(L, a.sc, k, Y, yy, s.p, rr);
-      } else {
-        J = out_loop < 2 ? a.sc.j_slow : a.sc.j_fast;
-        jacobi_sweeps<U>(L, Y, k, s.p, J);
-      }
-      s.n_sweeps += J;
-      pass_finish(L, k, c, s, od, G, sf);
-      pass_control(L, a.sc, c, s, vref, aref, out_loop, reset, another);
-    }
-    step_commit(a, it, c, s, out_loop, L);
+    step<N, TOL, WS, U>(a, it, L, k, c, s, s.A, s.B, pold);
+    if (s.in_s >= it.mesi) break;
+    step<N, TOL, WS, U>(a, it, L, k, c, s, s.B, s.A, pold);
   }
   item_final(a, s, item_index, L);
 }

@@ -255,6 +255,7 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
     k.rmass = t + 1536; k.rsm = t + 1792; k.mf = t + 2048;
     k.gam = (const CM_LDS float *)(gam_lds + wave * 64 + lane);
   }
+  Half &o = s.A, &n = s.B;                   // committed side, side of the current step
   pold[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
   if (lane == 0) reinterpret_cast<float *>(pold + 64)[0] = s.dt;
   __syncthreads();
@@ -266,14 +267,17 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
     const bool net_round = w.use_net && (round % w.net_every) == 0;
     float rr0 = 0.f, rre = 0.f, rr_scale = 0.f;
     if (active) {
-      float od[4], G4[4], Y[4];
-      pass_begin(s, true);
-      const float sf = pass_rhs(k, c, s, true, L, od, G4, Y);
-      keep[lane] = make_float4(G4[0], G4[1], G4[2], G4[3]);
-      keep[64 + lane] = make_float4(s.nxis[0], s.nxis[1], s.nxis[2], s.nxis[3]);
+      PassTerms<4> T;
+      float Y[4];
+      predict(o, n, s.dt);
+      const float sf = forcing(c, s);
+      pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
+      keep[lane] = make_float4(T.G[0], T.G[1], T.G[2], T.G[3]);
+      keep[64 + lane] = make_float4(n.xis[0], n.xis[1], n.xis[2], n.xis[3]);
       keep[128 + lane] = make_float4(s.Ptm[0], s.Ptm[1], s.Ptm[2], s.Ptm[3]);
-      if (lane == 0) reinterpret_cast<float *>(pold + 64)[1] = sf;
-      rr0 = extrapolate_guess(L, k, Y, s.dt, pold, s.p, rre, true);   // s.p = p_lin
+      float yy;
+      rr0 = extrapolate_guess(L, k, Y, s.dt, pold, s.p, rre, yy, true);   // s.p = p_lin
+      if (lane == 0) reinterpret_cast<float2 *>(pold + 64)[1] = make_float2(sf, yy);
       rr_scale = __builtin_amdgcn_sqrtf(rre * inv_256) + 1e-30f;
       if (net_round || w.capture) {
       float r[4];
@@ -281,14 +285,14 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
       const float4 pk = pold[lane];   // plain guess (previous pressure)
       // the scales only normalise BF16 network inputs: the hardware reciprocal
       // (1 ulp) stands in for an IEEE division
-      const float inv_d = __builtin_amdgcn_rcpf(rms256(s.nd[0], s.nd[1], s.nd[2], s.nd[3]));
-      const float inv_v = __builtin_amdgcn_rcpf(rms256(s.nv[0], s.nv[1], s.nv[2], s.nv[3]));
+      const float inv_d = __builtin_amdgcn_rcpf(rms256(n.d[0], n.d[1], n.d[2], n.d[3]));
+      const float inv_v = __builtin_amdgcn_rcpf(rms256(n.v[0], n.v[1], n.v[2], n.v[3]));
       const float inv_r = __builtin_amdgcn_rcpf(rr_scale);
       const float inv_p = __builtin_amdgcn_rcpf(rms256(pk.x, pk.y, pk.z, pk.w));
       float f[13];
       UNROLL for (int j = 0; j < 4; ++j) {
-        f[j] = s.nd[j] * inv_d;
-        f[4 + j] = s.nv[j] * inv_v;
+        f[j] = n.d[j] * inv_d;
+        f[4 + j] = n.v[j] * inv_v;
         f[8 + j] = r[j] * inv_r;
       }
       f[12] = sf * inv_p;
@@ -338,27 +342,29 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
       __syncthreads();
     }
     if (active) {
-      // the predictor state again (same inputs, same values), G, nxis and Ptm
-      // from LDS, and od and Y formed from them as pass_rhs formed them (same
-      // operations on the same values): cheaper than holding any of it in
-      // registers across the network
-      float od[4], G4[4], Y[4];
-      pass_begin(s, true);
-      const float sf = reinterpret_cast<const float *>(pold + 64)[1];
+      // the predictor state again (same inputs, same values), G, xis and Ptm
+      // from LDS, and the pass's other terms and Y formed from them as pass_rhs
+      // formed them (same operations on the same values): cheaper than holding
+      // any of it in registers across the network
+      PassTerms<4> T;
+      float Y[4];
+      predict(o, n, s.dt);
+      const float2 sf_yy = reinterpret_cast<const float2 *>(pold + 64)[1];
+      const float sf = uniform(sf_yy.x), yy = uniform(sf_yy.y);
       {
         const float4 g = keep[lane], x = keep[64 + lane], t = keep[128 + lane];
-        G4[0] = g.x; G4[1] = g.y; G4[2] = g.z; G4[3] = g.w;
-        s.nxis[0] = x.x; s.nxis[1] = x.y; s.nxis[2] = x.z; s.nxis[3] = x.w;
+        T.G[0] = g.x; T.G[1] = g.y; T.G[2] = g.z; T.G[3] = g.w;
+        n.xis[0] = x.x; n.xis[1] = x.y; n.xis[2] = x.z; n.xis[3] = x.w;
         s.Ptm[0] = t.x; s.Ptm[1] = t.y; s.Ptm[2] = t.z; s.Ptm[3] = t.w;
-        for (int j = 0; j < 4; ++j) {
-          od[j] = s.nxi[j] - s.nd[j];
-          Y[j] = (c.dxdx * G4[j]) * k.Q[j];
+        UNROLL for (int j = 0; j < 4; ++j) {
+          T.wpsi[j] = c.w_ohc * n.psi[j];
+          T.eod[j] = c.eta1 * (n.xi[j] - n.d[j]);
+          Y[j] = (c.dxdx * T.G[j]) * k.Q[j];
         }
-        const float Y0 = c.dxa0 * (((c.neg_a2 * s.ow_nv) - c.a1 * s.ow_nd) + c.Gme * sf);
-        if (lane == 0) Y[0] = Y0;
-        if (lane == 63) Y[3] = 0.0f;
+        const float Y0 = c.dxa0 * (((c.neg_a2 * n.ow_v) - c.a1 * n.ow_d) + c.Gme * sf);
+        Y[0] = lane == 0 ? Y0 : Y[0];
+        Y[3] = lane == 63 ? 0.0f : Y[3];
       }
-      const float yy = tree_sum(Y[0] * Y[0], Y[1] * Y[1], Y[2] * Y[2], Y[3] * Y[3]);
       float rr_sel = rre;   // residual of the guess kept (p_lin unless replaced below)
       if (net_round) {
         // learned guess: p_lin + rms(r_lin) c_out S(y), S = [1,2,1]/4 (edges replicated)
@@ -391,31 +397,27 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
         rr_sel = rr0;
       }
       // rest of the predictor pass, then the corrector passes of this step
-      int out_loop = 0, reset = 1, another = 1;
-      {
-        const int J = jacobi_tol(L, a.sc, k, Y, yy, s.p, rr_sel);
-        s.n_sweeps += J;
-        pass_finish(L, k, c, s, od, G4, sf);
-        float vref[4], aref[4];   // unused: step control is skipped on the predictor pass
-        UNROLL for (int j = 0; j < 4; ++j) { vref[j] = 0.f; aref[j] = 0.f; }
-        pass_control(L, a.sc, c, s, vref, aref, out_loop, reset, another);
-      }
-      // vref/aref of the first corrector pass are the predictor pass's values
+      s.n_sweeps += jacobi_tol(L, a.sc, k, Y, yy, s.p, rr_sel);
+      pass_finish(L, k, c, n, s.p, T, sf);
+      int passes = 1;
+      bool another = passes < a.sc.max_passes;
+      if (!another) s.c_fail = 1.f;
       while (another) {
         float vref[4], aref[4];
-        UNROLL for (int j = 0; j < 4; ++j) { vref[j] = s.nv[j]; aref[j] = s.na[j]; }
-        const bool predictor = out_loop == 0 || reset;
-        if (predictor) out_loop = 0;
-        pass_begin(s, predictor);
-        float od2[4], G2[4], Y2[4];
-        const float sf2 = pass_rhs(k, c, s, out_loop < 2, L, od2, G2, Y2);
-        const float yy2 = tree_sum(Y2[0] * Y2[0], Y2[1] * Y2[1], Y2[2] * Y2[2], Y2[3] * Y2[3]);
-        const int J = jacobi_tol(L, a.sc, k, Y2, yy2, s.p, resid2(L, Y2, k, s.p));
-        s.n_sweeps += J;
-        pass_finish(L, k, c, s, od2, G2, sf2);
-        pass_control(L, a.sc, c, s, vref, aref, out_loop, reset, another);
+        UNROLL for (int j = 0; j < 4; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
+        correct(o, n, s.dt);
+        if (passes < 2)
+          pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
+        else
+          pass_rhs<false>(k, c, n, s.Ptm, sf, L, T, Y);
+        s.n_sweeps += solve_pass<true, 2>(L, a.sc, k, Y, s.p, 0);
+        pass_finish(L, k, c, n, s.p, T, sf);
+        another = pass_control(L, a.sc, c, s.dt, n, vref, aref);
+        ++passes;
+        if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
       }
-      step_commit(a, it, c, s, out_loop, L);
+      step_commit(a, it, c, s, n, passes, L);
+      o = n;   // one copy per round: the group's code is not doubled for two roles
     }
   }
   if (valid) item_final(a, s, idx, L);
