@@ -66,17 +66,14 @@ struct StageHolder {
 };
 StageHolder g_st;
 
-// Device scratch of cm_ihc_lambda_run_noalloc: the interval table and the
-// zero-padded AC and DC tap tables, staged in a fixed array of this code
-// object instead of allocated memory.  Every GPU holds its own copy for the
-// life of the process; host code reaches it only through the per-device
+// Device scratch of cm_ihc_lambda_run_noalloc: the interval table of a call
+// whose table does not travel with its launch, staged in a fixed array of this
+// code object instead of allocated memory.  Every GPU holds its own copy for
+// the life of the process; host code reaches it only through the per-device
 // address from hipGetSymbolAddress, never through the array's name.
 constexpr int kNoallocIntervals = 4096;
-constexpr int kNoallocAcTaps = 512;    // a multiple of 16 (the FIR chunk)
-constexpr int kNoallocDcTaps = 112;    // 97 used at most, padded to 16
-constexpr size_t kNoallocIvBytes = (size_t)kNoallocIntervals * sizeof(cm_ihc_interval);
-constexpr size_t kNoallocBytes =
-    kNoallocIvBytes + (size_t)kNoallocAcTaps * sizeof(double) + (size_t)kNoallocDcTaps * sizeof(double);
+constexpr int kNoallocAcTaps = 512;
+constexpr size_t kNoallocBytes = (size_t)kNoallocIntervals * sizeof(cm_ihc_interval);
 static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 
 constexpr int kMaxDevices = 64;
@@ -96,12 +93,6 @@ static unsigned char *noalloc_scratch() {
     g_scratch_dev[dev] = static_cast<unsigned char *>(p);
   }
   return g_scratch_dev[dev];
-}
-
-// dst[i] = src[i] for i < n, 0 up to npad (a fill kernel rather than a memset)
-__global__ void pad_taps_kernel(double *dst, const double *src, int n, int npad) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < npad) dst[i] = i < n ? src[i] : 0.0;
 }
 
 }  // namespace cm
@@ -206,6 +197,19 @@ static int pad_taps(Buf<double> &dst, const double *d_src, int n) {
                "pad taps");
 }
 
+// What a launch of cm_launch_ihc_lambda reads besides the caller's buffers:
+// the interval table in device memory unless it travels with the launch, and
+// zero-padded taps for the two-pass kernels.
+static int prepare_tables(const cm_ihc_interval *h_ivs, int n_ivs, const double *d_ac_b, int n_ac, const double *d_dc,
+                          int n_dc, const cm_ihc_interval **d_ivs) {
+  *d_ivs = nullptr;
+  if (ihc_table_inline(h_ivs, n_ivs, n_dc)) return 0;
+  if (g_st.ivs.upload(h_ivs, n_ivs)) return -1;
+  *d_ivs = g_st.ivs.ptr;
+  if (ihc_one_pass(h_ivs, n_ivs, n_dc)) return 0;
+  return pad_taps(g_st.ac_bpad, d_ac_b, n_ac) || pad_taps(g_st.dcpad, d_dc, n_dc) ? -1 : 0;
+}
+
 static void build_intervals(int rows, std::vector<cm_ihc_interval> &fir, std::vector<cm_ihc_interval> &iir) {
   const int DF = g_st.decouple;
   const int L = DF > 0 ? g_st.interval_nodes * DF : rows;
@@ -240,13 +244,14 @@ int RunIHCKernel(float *host_backup, int Show_Run_Time, int save_lambda, int bac
   }
   std::vector<cm_ihc_interval> fir, iir;
   build_intervals(rows, fir, iir);
-  if (g_st.ivs.upload(fir.data(), fir.size()) || g_st.iir_ivs.upload(iir.data(), iir.size())) return -1;
+  const cm_ihc_interval *d_ivs = nullptr;
+  if (prepare_tables(fir.data(), (int)fir.size(), g_st.ac_b.ptr, g_st.n_ac, g_st.dc.ptr, g_st.n_dc, &d_ivs)) return -1;
+  if (g_st.is_iir && g_st.iir_ivs.upload(iir.data(), iir.size())) return -1;
   const size_t plane = (size_t)rows * CM_SECTIONS;
   const int want_stages = backup_stage >= 9 && backup_stage <= 14 && host_backup;
   if (want_stages && g_st.stages.ensure(5 * plane)) return -1;
   if (g_st.lambda.ensure(3 * plane) || g_st.scratch.ensure(2 * plane)) return -1;
-  if (pad_taps(g_st.ac_bpad, g_st.ac_b.ptr, g_st.n_ac) || pad_taps(g_st.dcpad, g_st.dc.ptr, g_st.n_dc)) return -1;
-  int rc = cm_launch_ihc_lambda(bm_speeds_ptr(), rows, g_st.ivs.ptr, fir.data(), (int)fir.size(), g_st.iir_ivs.ptr,
+  int rc = cm_launch_ihc_lambda(bm_speeds_ptr(), rows, d_ivs, fir.data(), (int)fir.size(), g_st.iir_ivs.ptr,
                                 (int)iir.size(), g_st.ac_b.ptr, g_st.ac_bpad.ptr, g_st.is_iir ? g_st.ac_a.ptr : nullptr,
                                 g_st.n_ac, g_st.dc.ptr, g_st.dcpad.ptr, g_st.n_dc, g_st.damage.ptr, g_st.A.ptr, g_st.spont, g_st.sat,
                                 g_st.eta_ac, g_st.eta_dc, g_st.scale, g_st.scratch.ptr, g_st.lambda.ptr,
@@ -401,7 +406,6 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
       set_error("cm_ihc_lambda_run: interval %d outside [0, %lld)", i, (long long)rows);
       return -3;
     }
-  if (g_st.ivs.upload(h_ivs, n_ivs)) return -1;
   if (d_ac_a && (!h_iir_ivs || n_iir_ivs <= 0)) {
     set_error("cm_ihc_lambda_run: IIR filter needs its interval table");
     return -3;
@@ -414,8 +418,9 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
       return -3;
     }
   if (d_ac_a && g_st.iir_ivs.upload(h_iir_ivs, n_iir_ivs)) return -1;
-  if (pad_taps(g_st.ac_bpad, d_ac_b, n_ac) || pad_taps(g_st.dcpad, d_dc, n_dc)) return -1;
-  const int rc = cm_launch_ihc_lambda(d_bm, rows, g_st.ivs.ptr, h_ivs, n_ivs, g_st.iir_ivs.ptr, n_iir_ivs, d_ac_b,
+  const cm_ihc_interval *d_ivs = nullptr;
+  if (prepare_tables(h_ivs, n_ivs, d_ac_b, n_ac, d_dc, n_dc, &d_ivs)) return -1;
+  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, g_st.iir_ivs.ptr, n_iir_ivs, d_ac_b,
                                       g_st.ac_bpad.ptr, d_ac_a, n_ac, d_dc, g_st.dcpad.ptr, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc,
                                       scale_bm, d_scratch, d_lambda, d_stages, stream());
   if (rc) set_error("cm_ihc_lambda_run: launch failed (%d)", rc);
@@ -423,10 +428,10 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
 }
 
 // cm_ihc_lambda_run without allocating: the one-pass kernel (no AC/dS
-// workspace) with its tables staged in the device scratch array.  FIR AC
-// filters only, at most kNoallocIntervals intervals (kbase 0), kNoallocAcTaps
-// AC taps and 97 DC taps.  Calls that overlap on one GPU (other streams or
-// threads) race on the scratch array.
+// workspace), a table too long for its launch staged in the device scratch
+// array.  FIR AC filters only, at most kNoallocIntervals intervals (kbase 0),
+// kNoallocAcTaps AC taps and 97 DC taps.  Calls that overlap on one GPU (other
+// streams or threads) race on the scratch array.
 int cm_ihc_lambda_run_noalloc(const float *d_bm, int64_t rows, const cm_ihc_interval *h_ivs, int n_ivs,
                               const double *d_ac_b, int n_ac, const double *d_dc, int n_dc, const double *d_damage,
                               const float *d_A, const float *spont3, float lambda_sat, float eta_ac, float eta_dc,
@@ -455,20 +460,16 @@ int cm_ihc_lambda_run_noalloc(const float *d_bm, int64_t rows, const cm_ihc_inte
       return -3;
     }
   }
-  unsigned char *base = noalloc_scratch();
-  if (!base) return -1;
-  cm_ihc_interval *d_ivs = reinterpret_cast<cm_ihc_interval *>(base);
-  double *ac_pad = reinterpret_cast<double *>(base + kNoallocIvBytes);
-  double *dc_pad = ac_pad + kNoallocAcTaps;
-  const int ac_np = (n_ac + 15) / 16 * 16, dc_np = (n_dc + 15) / 16 * 16;
-  if (check(hipMemcpyAsync(d_ivs, h_ivs, (size_t)n_ivs * sizeof(cm_ihc_interval), hipMemcpyHostToDevice, stream()),
-            "interval table"))
-    return -1;
-  hipLaunchKernelGGL(pad_taps_kernel, dim3((ac_np + 255) / 256), dim3(256), 0, stream(), ac_pad, d_ac_b, n_ac, ac_np);
-  hipLaunchKernelGGL(pad_taps_kernel, dim3(1), dim3(256), 0, stream(), dc_pad, d_dc, n_dc, dc_np);
-  if (check(hipGetLastError(), "pad taps")) return -1;
-  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, nullptr, 0, d_ac_b, ac_pad, nullptr, n_ac, d_dc,
-                                      dc_pad, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc, scale_bm,
+  cm_ihc_interval *d_ivs = nullptr;
+  if (!ihc_table_inline(h_ivs, n_ivs, n_dc)) {
+    d_ivs = reinterpret_cast<cm_ihc_interval *>(noalloc_scratch());
+    if (!d_ivs) return -1;
+    if (check(hipMemcpyAsync(d_ivs, h_ivs, (size_t)n_ivs * sizeof(cm_ihc_interval), hipMemcpyHostToDevice, stream()),
+              "interval table"))
+      return -1;
+  }
+  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, nullptr, 0, d_ac_b, nullptr, nullptr, n_ac, d_dc,
+                                      nullptr, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc, scale_bm,
                                       nullptr, d_lambda, d_stages, stream());
   if (rc) set_error("cm_ihc_lambda_run_noalloc: launch failed (%d)", rc);
   return rc ? -1 : 0;

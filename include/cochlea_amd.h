@@ -203,10 +203,11 @@ void *getCudaLambda(void);
 void *getCudaBuffer(void);
 void *getCudaMeanRate(void);
 /* batched IHC/lambda over device pointers and an interval table (no
- * reference counterpart); d_scratch holds 2 x rows x 256 floats (AC, dS) for
- * the two-pass kernels.  d_scratch = NULL runs the chain in one pass with no
- * workspace (slower, half the HBM traffic): FIR AC filters only, every
- * interval with kbase 0, at most 97 DC taps.  With an IIR
+ * reference counterpart).  The chain runs in one pass where every interval has
+ * kbase 0 and the DC filter at most 97 taps; d_scratch (2 x rows x 256 floats)
+ * holds AC and dS for the two-pass kernels of the other tables, and the AC of
+ * an IIR filter.  d_scratch = NULL is refused where one of these needs it.
+ * Tables of up to 4 intervals travel with the launch (no upload).  With an IIR
  * AC filter (d_ac_a) h_iir_ivs lists the runs the recursion restarts on:
  * rows [row0, row0 + len), period len (CudaIIRFilterDecoupled,
  * src/cochlea.cu:2885-2908).  n_ivs = 0 is a no-op; negative counts and
@@ -220,8 +221,8 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
 /* cm_ihc_lambda_run without any device allocation (no reference counterpart;
  * for callers that cannot allocate: code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  The same inputs and outputs with
- * no workspace: the chain runs in one pass, its interval table and padded tap
- * tables staged in a fixed device array of the library (133 KiB per GPU, held
+ * no workspace: the chain runs in one pass, an interval table of more than 4
+ * entries staged in a fixed device array of the library (128 KiB per GPU, held
  * until the process ends).  Limits: FIR AC filters, at most 4096 intervals
  * (kbase 0), 512 AC taps, 97 DC taps; larger requests return -3.  Every call on
  * one GPU shares that array: calls that overlap on a GPU (several streams or
