@@ -105,7 +105,7 @@ int cm_post_bm_graph_create(const float *d_bm, int64_t rows, const cm_ihc_interv
   a.FisherAISum = d_FisherAISum;
   if (check(hipStreamBeginCapture(g->capture, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
     return fail(-1);
-  int rc = cm_launch_ihc_lambda(d_bm, rows, g->d_ivs, h_ivs, n_ivs, nullptr, 0, d_ac_b, g->d_ac_bpad, nullptr, n_ac,
+  int rc = cm_launch_ihc_lambda(d_bm, rows, g->d_ivs, h_ivs, n_ivs, nullptr, nullptr, 0, d_ac_b, g->d_ac_bpad, nullptr, n_ac,
                                 d_dc, g->d_dcpad, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc, scale_bm,
                                 d_scratch, d_lambda, nullptr, g->capture);
   if (!rc) rc = cm_launch_jnd(&a, g->capture);

@@ -252,7 +252,7 @@ int RunIHCKernel(float *host_backup, int Show_Run_Time, int save_lambda, int bac
   if (want_stages && g_st.stages.ensure(5 * plane)) return -1;
   if (g_st.lambda.ensure(3 * plane) || g_st.scratch.ensure(2 * plane)) return -1;
   int rc = cm_launch_ihc_lambda(bm_speeds_ptr(), rows, d_ivs, fir.data(), (int)fir.size(), g_st.iir_ivs.ptr,
-                                (int)iir.size(), g_st.ac_b.ptr, g_st.ac_bpad.ptr, g_st.is_iir ? g_st.ac_a.ptr : nullptr,
+                                iir.data(), (int)iir.size(), g_st.ac_b.ptr, g_st.ac_bpad.ptr, g_st.is_iir ? g_st.ac_a.ptr : nullptr,
                                 g_st.n_ac, g_st.dc.ptr, g_st.dcpad.ptr, g_st.n_dc, g_st.damage.ptr, g_st.A.ptr, g_st.spont, g_st.sat,
                                 g_st.eta_ac, g_st.eta_dc, g_st.scale, g_st.scratch.ptr, g_st.lambda.ptr,
                                 want_stages ? g_st.stages.ptr : nullptr, stream());
@@ -420,7 +420,7 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
   if (d_ac_a && g_st.iir_ivs.upload(h_iir_ivs, n_iir_ivs)) return -1;
   const cm_ihc_interval *d_ivs = nullptr;
   if (prepare_tables(h_ivs, n_ivs, d_ac_b, n_ac, d_dc, n_dc, &d_ivs)) return -1;
-  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, g_st.iir_ivs.ptr, n_iir_ivs, d_ac_b,
+  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, g_st.iir_ivs.ptr, h_iir_ivs, n_iir_ivs, d_ac_b,
                                       g_st.ac_bpad.ptr, d_ac_a, n_ac, d_dc, g_st.dcpad.ptr, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc,
                                       scale_bm, d_scratch, d_lambda, d_stages, stream());
   if (rc) set_error("cm_ihc_lambda_run: launch failed (%d)", rc);
@@ -468,7 +468,7 @@ int cm_ihc_lambda_run_noalloc(const float *d_bm, int64_t rows, const cm_ihc_inte
               "interval table"))
       return -1;
   }
-  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, nullptr, 0, d_ac_b, nullptr, nullptr, n_ac, d_dc,
+  const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, nullptr, nullptr, 0, d_ac_b, nullptr, nullptr, n_ac, d_dc,
                                       nullptr, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc, scale_bm,
                                       nullptr, d_lambda, d_stages, stream());
   if (rc) set_error("cm_ihc_lambda_run_noalloc: launch failed (%d)", rc);

@@ -62,3 +62,25 @@ def test_windows_that_restart_inside_an_interval(oracle, rows, L, frdp):
     lo = oracle.ihc_lambda(bm, L, frdp, b, stages.dc_filter(FS), stages.ihc_damage(8.0), stages.aihc_table(),
                            np.array(stages.SPONT_DEFAULT, np.float32), threads=8)
     np.testing.assert_array_equal(lam.cpu().numpy(), lo)
+
+
+@pytest.mark.parametrize("taps", [2, 3, 5, 9, 10])
+def test_iir_orders_and_lengths(oracle, taps):
+    """The IIR AC filter of every register form and of the general one, over
+    intervals around its blocks of 16 rows: the same values as the oracle's."""
+    import torch
+    from scipy.signal import butter
+    from cochlearmodel_amd import stages
+    print(f"case: IIR AC filter of {taps} taps", flush=True)
+    lens = [1, 2, 15, 16, 17, 33, 700]
+    b, a = butter(taps - 1, 0.3)
+    starts = np.cumsum([0] + lens[:-1])
+    bm = _field(sum(lens), 7)
+    ivs = stages.signal_intervals(starts, lens)
+    lam, st = stages.BatchedIHC(FS, ac=(b, a)).run(torch.from_numpy(bm).cuda(), sum(lens), ivs, ivs, stages=True)
+    for s0, n in zip(starts, lens):
+        lo, so = oracle.ihc_lambda(bm[s0:s0 + n], n, n + 1, b, stages.dc_filter(FS), stages.ihc_damage(8.0),
+                                   stages.aihc_table(), np.array(stages.SPONT_DEFAULT, np.float32), stages=True,
+                                   threads=8, ac_a=a)
+        np.testing.assert_array_equal(st[:, s0:s0 + n].cpu().numpy(), so, err_msg=f"stages, {n} rows")
+        np.testing.assert_array_equal(lam[:, s0:s0 + n].cpu().numpy(), lo, err_msg=f"{n} rows")
