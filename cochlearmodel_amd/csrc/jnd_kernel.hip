@@ -1,10 +1,9 @@
 // JND reductions of CudaCalculateJND (src/cochlea.cu:3703-4065) in one
 // kernel: per-interval mean rate (GlobalCalculateMeanRate :3741-3771) and the
 // Fisher AI / rate terms reduced over the 256 sections (GlobalCalculateJND
-// :3773-3944).  One workgroup = 256 sections of one (interval, fiber group);
-// time sums run down the section-fastest lambda planes, so every step is a
-// coalesced 1 KB read.  The section reduction keeps the reference's halving
-// tree (stride 128, 64, ..., 1) so the CPU oracle agrees bit for bit.
+// :3773-3944).  One workgroup = 256 sections of one (interval, fiber group).
+// The section reduction keeps the reference's halving tree (stride 128, 64,
+// ..., 1) so the CPU oracle agrees bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "cm_internal.h"
@@ -13,11 +12,12 @@ namespace cm {
 
 
 
-__device__ __forceinline__ float halving_tree(float *sh, float v, int s) {
-  sh[s] = v;
-  for (int t = CM_SECTIONS >> 1; t >= 1; t >>= 1) {
+// v of the threads 0..255 summed; every thread of the workgroup calls it.
+__device__ __forceinline__ float halving_tree(float *sh, float v, int t) {
+  if (t < CM_SECTIONS) sh[t] = v;
+  for (int k = CM_SECTIONS >> 1; k >= 1; k >>= 1) {
     __syncthreads();
-    if (s < t) sh[s] = sh[s] + sh[s + t];
+    if (t < k) sh[t] = sh[t] + sh[t + k];
   }
   __syncthreads();
   const float r = sh[0];
@@ -25,81 +25,211 @@ __device__ __forceinline__ float halving_tree(float *sh, float v, int s) {
   return r;
 }
 
+// Rows of one section, [row, row + N) of a run of `rows` rows from `base`;
+// rows past it read as 0.
+template <int N>
+__device__ __forceinline__ void load_rows(const float *base, int64_t row, int64_t rows, int s, float (&x)[N]) {
+  const int64_t left = rows - row;
+  const auto desc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base) + row * CM_SECTIONS, 0,
+                                                      (int)(left < N ? (left > 0 ? left : 0) : N) * (CM_SECTIONS * 4),
+                                                      0x00027000);
+#pragma unroll
+  for (int m = 0; m < N; ++m)
+    x[m] = __builtin_bit_cast(float,
+                              __builtin_amdgcn_raw_buffer_load_b32(desc, 4 * s + m * (CM_SECTIONS * 4), 0, 0));
+}
+
+// N / D as the compiler's correctly rounded FP64 division computes it, without
+// its range scaling: for D within 2^+-200 and N a finite float, where nothing
+// over- or underflows.
+__device__ __forceinline__ double div_in_range(double n, double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
 // One pass over the interval body of (interval, fiber group) and of its
 // reference: both mean rates (FP64 sums in time order, as
-// GlobalCalculateMeanRate takes them) and the AI Fisher sum, then the rate
-// term and the two section reductions.  The reference's mean rate is summed
-// again by every interval that uses it, in the same order, so it is the value
-// its own workgroup writes; fusing the mean-rate pass saves one read of every
-// interval body.
-__global__ __launch_bounds__(256) void jnd_kernel(JndArgs a) {
+// GlobalCalculateMeanRate takes them) and the AI Fisher sum (float, in time
+// order), then the rate term and the two section reductions.  The reference's
+// mean rate is summed again by every interval that uses it, in the same order,
+// so it is the value its own workgroup writes.
+//
+// The three sums must stay serial in time; the Fisher terms (two divisions
+// each, most of the work) need not.  So each 64 sections have 4 waves: all of
+// them form the terms of a 32-row tile and put them into LDS, while one adds up
+// the tile before it and two add up the rates, with fewer rows for these three
+// (rows_of) so that all four reach the barrier together.
+// Bound: instruction issue of one workgroup per CU.  41 intervals of 12.5 k
+// rows: one thread per section doing everything in turn 6.01 ms, this 1.04 ms.
+constexpr int kTileRows = 32;
+constexpr int kMostRows = 10;
+struct JndWave {
+  const JndArgs &a;
+  const float *c, *r;      // interval body, reference body: first row
+  float *node_stage;
+  int L, s, lane, stage;
+  float dA;
+  double inv_dA;
+
+  // Fisher terms of N rows from row0 of the bodies into pre (64 lanes per row)
+  template <int N>
+  __device__ __forceinline__ void terms(const float (&cal)[kMostRows], const float (&ref)[kMostRows], int64_t row0,
+                                        float *pre) const {
+    bool in_range = a.Fs > 0x1p-100 && a.Fs < 0x1p100;
+    float dl[N], sq[N];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+      // (cal - ref) / dA: the FP64 product with the reciprocal rounds to the
+      // same float (a quotient of floats is 2^-49 from any midpoint of two)
+      dl[m] = dA > 0 ? (float)((double)(cal[m] - ref[m]) * inv_dA) : 0.0f;
+      sq[m] = dl[m] * dl[m];
+      in_range = in_range && (ref[m] > 0x1p-100f && ref[m] < 0x1p100f && sq[m] < __builtin_inff());
+    }
+    const bool fast = __builtin_amdgcn_ballot_w64(!in_range) == 0;
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+      const double n = (double)sq[m], d = a.Fs * (double)ref[m];
+      const float p = (float)(fast ? div_in_range(n, d) : n / d);
+      pre[m * 64 + lane] = p;
+      if (node_stage && row0 + m < L) node_stage[(row0 + m) * CM_SECTIONS + s] = stage == 3 ? dl[m] : p;
+    }
+  }
+};
+
+// first row and number of rows of a tile that each of the 4 waves forms
+template <int Q>
+struct RowsOf;
+template <> struct RowsOf<0> { static constexpr int first = 0, n = 8; };     // adds up the Fisher terms
+template <> struct RowsOf<1> { static constexpr int first = 8, n = 7; };     // adds up the interval's rates
+template <> struct RowsOf<2> { static constexpr int first = 15, n = 7; };    // adds up the reference's rates
+template <> struct RowsOf<3> { static constexpr int first = 22, n = 10; };
+
+// The time loop of wave Q of a section group; returns its sum (0: in accv).
+template <int Q>
+__device__ __forceinline__ double jnd_time(const JndWave &w, float *pre, bool ai, float &accv) {
+  constexpr int first = RowsOf<Q>::first, n = RowsOf<Q>::n;
+  const int tiles = (w.L + kTileRows - 1) / kTileRows;
+  constexpr int kHalf = kTileRows / 2;
+  float cal[n], ref[n], rate[2][kHalf];
+  double acc = 0.0;
+  accv = 0.0f;
+  const float *mine = Q == 1 ? w.c : w.r;
+  if (ai) {
+    load_rows(w.c, first, w.L, w.s, cal);
+    load_rows(w.r, first, w.L, w.s, ref);
+  }
+  if (Q == 1 || Q == 2) {
+    load_rows(mine, 0, w.L, w.s, rate[0]);
+    load_rows(mine, kHalf, w.L, w.s, rate[1]);
+  }
+  for (int j = 0; j <= tiles; ++j) {
+    const int64_t row = (int64_t)j * kTileRows;
+    float *buf = pre + (j & 1) * kTileRows * 64;
+    if (j < tiles) {
+      if (ai) {
+        float c0[kMostRows], r0[kMostRows];
+#pragma unroll
+        for (int m = 0; m < n; ++m) { c0[m] = cal[m]; r0[m] = ref[m]; }
+        load_rows(w.c, row + kTileRows + first, w.L, w.s, cal);   // the next tile's, in flight meanwhile
+        load_rows(w.r, row + kTileRows + first, w.L, w.s, ref);
+        w.terms<n>(c0, r0, row + first, buf + first * 64);
+      }
+      if (Q == 1 || Q == 2) {
+        // rows past the body read as 0
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int m = 0; m < kHalf; ++m) acc = acc + (double)rate[h][m];
+          load_rows(mine, row + kTileRows + h * kHalf, w.L, w.s, rate[h]);
+        }
+      }
+    }
+    if (Q == 0 && ai && j > 0) {
+      const float *last = pre + ((j - 1) & 1) * kTileRows * 64 + w.lane;
+      const int64_t left = w.L - (row - kTileRows);
+      if (left >= kTileRows) {
+        float p[kTileRows];
+#pragma unroll
+        for (int m = 0; m < kTileRows; ++m) p[m] = last[m * 64];
+#pragma unroll
+        for (int m = 0; m < kTileRows; ++m) accv += p[m];
+      } else {
+        for (int m = 0; m < left; ++m) accv += last[m * 64];
+      }
+    }
+    if (ai) __syncthreads();
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(1024) void jnd_kernel(JndArgs a) {
+  __shared__ float pre_lds[4][2 * kTileRows * 64];
+  __shared__ double mean_lds[2][CM_SECTIONS];
+  __shared__ float fisher_lds[CM_SECTIONS];
   __shared__ float sh[CM_SECTIONS];
-  const int iv = blockIdx.x, li = blockIdx.y, s = threadIdx.x;
+  const int iv = blockIdx.x, li = blockIdx.y, t = threadIdx.x;
   const int ref = a.ref_index[iv];
   const float dAv = a.dA[iv];
-  const int64_t c = ((int64_t)li * a.rows + (int64_t)iv * a.interval_nodes + a.head_nodes) * CM_SECTIONS + s;
-  const int64_t r = ((int64_t)li * a.rows + (int64_t)ref * a.interval_nodes + a.head_nodes) * CM_SECTIONS + s;
+  const int64_t c = ((int64_t)li * a.rows + (int64_t)iv * a.interval_nodes + a.head_nodes) * CM_SECTIONS;
+  const int64_t r = ((int64_t)li * a.rows + (int64_t)ref * a.interval_nodes + a.head_nodes) * CM_SECTIONS;
   const int L = a.length_nodes;
   const int stage = a.buffer ? a.backup_stage : 0;
   // per-node stages 3 (dLambda) and 4 (preFisherAI) at the body's own lambda nodes
   float *node_stage = (stage == 3 || stage == 4) ? a.buffer + c : nullptr;
-  const int64_t ms = ((int64_t)li * a.n_intervals + iv) * CM_SECTIONS + s;   // mean-rate layout
   float ai = 0.f, rms = 0.f;
   if (a.calc_ai || a.calc_rms) {
-    double acc_c = a.lambda[c], acc_r = a.lambda[r];
-    float accv = 0.0f;
-    if (a.calc_ai) {
-      const float refl = a.lambda[r], cal = a.lambda[c];
-      const float dl = dAv > 0 ? (cal - refl) / dAv : 0.0f;
-      const float pre = (float)((double)(dl * dl) / (a.Fs * (double)refl));
-      accv += pre;
-      if (node_stage) node_stage[0] = stage == 3 ? dl : pre;
-#pragma unroll 4
-      for (int t = 1; t < L; ++t) {
-        const float refl = a.lambda[r + (int64_t)t * CM_SECTIONS];
-        const float cal = a.lambda[c + (int64_t)t * CM_SECTIONS];
-        acc_c = acc_c + cal;
-        acc_r = acc_r + refl;
-        const float dl = dAv > 0 ? (cal - refl) / dAv : 0.0f;
-        const float pre = (float)((double)(dl * dl) / (a.Fs * (double)refl));
-        accv += pre;
-        if (node_stage) node_stage[(int64_t)t * CM_SECTIONS] = stage == 3 ? dl : pre;
-      }
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = wave >> 2, role = wave & 3;
+    const int lane = t & 63, s = group * 64 + lane;
+    const JndWave w{a, a.lambda + c, a.lambda + r, node_stage, L, s, lane, stage, dAv, 1.0 / (double)dAv};
+    float accv;
+    if (role == 0) {
+      jnd_time<0>(w, pre_lds[group], a.calc_ai, accv);
+      fisher_lds[s] = accv;
+    } else if (role == 1) {
+      mean_lds[0][s] = jnd_time<1>(w, pre_lds[group], a.calc_ai, accv);
+    } else if (role == 2) {
+      mean_lds[1][s] = jnd_time<2>(w, pre_lds[group], a.calc_ai, accv);
     } else {
-#pragma unroll 8
-      for (int t = 1; t < L; ++t) {
-        acc_c = acc_c + a.lambda[c + (int64_t)t * CM_SECTIONS];
-        acc_r = acc_r + a.lambda[r + (int64_t)t * CM_SECTIONS];
-      }
+      jnd_time<3>(w, pre_lds[group], a.calc_ai, accv);
     }
-    const float mr = (float)acc_c / (float)L;
-    const float mref = (float)acc_r / (float)L;
-    a.mean_rate[ms] = mr;
-    const float dMR = (mr - mref) / dAv;
+    __syncthreads();
+    const int64_t ms = ((int64_t)li * a.n_intervals + iv) * CM_SECTIONS + t;   // mean-rate layout
+    float mr = 0.0f, dMR = 0.0f, mref = 0.0f;
+    if (t < CM_SECTIONS) {
+      mr = (float)mean_lds[0][t] / (float)L;
+      mref = (float)mean_lds[1][t] / (float)L;
+      a.mean_rate[ms] = mr;
+      dMR = (mr - mref) / dAv;
+      if (stage == 2) a.buffer[ms] = dMR;
+    }
     if (stage == 1 && a.calc_rms) {   // mean over the sections of this interval's mean rate
-      const float sum = halving_tree(sh, mr, s);
-      if (s == 0) a.buffer[(int64_t)li * a.n_intervals + iv] = sum / (float)CM_SECTIONS;
+      const float sum = halving_tree(sh, mr, t);
+      if (t == 0) a.buffer[(int64_t)li * a.n_intervals + iv] = sum / (float)CM_SECTIONS;
     }
-    if (stage == 2) a.buffer[ms] = dMR;
-    if (a.calc_ai) {
-      const float rs = 1.0f / __builtin_sqrtf(accv);
-      ai = (float)((double)(a.T / a.Tlength) * a.nIHC[s] / (double)(rs * rs));
-      if (stage == 5) a.buffer[ms] = ai;
-    }
-    if (a.calc_rms) {
-      const float crlb = 1.0f / __builtin_sqrtf(((a.T / mref) * dMR) * dMR);
-      rms = (float)(a.nIHC[s] / (double)(crlb * crlb));
-      if (stage == 6) a.buffer[ms] = crlb;
+    if (t < CM_SECTIONS) {
+      if (a.calc_ai) {
+        const float rs = 1.0f / __builtin_sqrtf(fisher_lds[t]);
+        ai = (float)((double)(a.T / a.Tlength) * a.nIHC[t] / (double)(rs * rs));
+        if (stage == 5) a.buffer[ms] = ai;
+      }
+      if (a.calc_rms) {
+        const float crlb = 1.0f / __builtin_sqrtf(((a.T / mref) * dMR) * dMR);
+        rms = (float)(a.nIHC[t] / (double)(crlb * crlb));
+        if (stage == 6) a.buffer[ms] = crlb;
+      }
     }
   }
   const int64_t fi = (int64_t)li * a.out_stride + a.out_index[iv];
   if (a.calc_ai) {
-    const float sum = halving_tree(sh, ai, s);
-    if (s == 0) a.FisherAISum[fi] = sum * a.W[li];
+    const float sum = halving_tree(sh, ai, t);
+    if (t == 0) a.FisherAISum[fi] = sum * a.W[li];
   }
   if (a.calc_rms) {
-    const float sum = halving_tree(sh, rms, s);
-    if (s == 0) a.F_RA[fi] = sum * a.W[li];
+    const float sum = halving_tree(sh, rms, t);
+    if (t == 0) a.F_RA[fi] = sum * a.W[li];
   }
 }
 
@@ -125,7 +255,7 @@ extern "C" int cm_launch_jnd(const cm::JndArgs *a, hipStream_t stream) {
   using namespace cm;
   if (a->n_intervals <= 0) return 0;
   if (a->n_intervals > 0x7fffffff) return -3;
-  hipLaunchKernelGGL(jnd_kernel, dim3(a->n_intervals, 3), dim3(256), 0, stream, *a);
+  hipLaunchKernelGGL(jnd_kernel, dim3(a->n_intervals, 3), dim3(1024), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
