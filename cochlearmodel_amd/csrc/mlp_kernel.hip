@@ -3,10 +3,7 @@
 // weights.  No reference counterpart.
 //
 // GEMM: C[M x N] (fp32) = op(A) * op(B) (+ bias[N]) with op = identity or
-// transpose, A/B bf16 row-major with leading dimensions.  A workgroup of 4
-// waves owns a 64 x 64 tile of C (each wave a 32 x 32 quarter = 2 x 2
-// v_mfma_f32_16x16x16_bf16 tiles) and walks K in steps of 16 through LDS.
-// Out-of-range elements load as zero, so any M, N, K works.
+// transpose, A/B bf16 row-major with leading dimensions, any M, N, K.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -15,7 +12,7 @@
 
 namespace cm {
 
-typedef __attribute__((__vector_size__(4 * sizeof(short)))) short bf16x4;
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 __device__ __forceinline__ uint16_t f32_to_bf16(float x) {
@@ -27,55 +24,219 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float x) {
 }
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
-constexpr int TM = 64, TN = 64, TK = 16;
+// A workgroup owns a 64 x TN tile of C and walks K in steps of 128 G: each of its
+// G groups of 4 waves loads 128 of them, and every element of C is one chain of
+// products in the order of k, whatever G is (activations are rounded to BF16
+// after the product: another order of its sum would move some of them by a whole
+// BF16 step).  A step's elements are requested during the products of the step
+// before it and reach LDS after them.  LDS holds both operands with k running
+// along a row, as v_mfma_f32_16x16x32_bf16 takes them (8 consecutive k per lane,
+// one 16-byte read); an operand that is contiguous the other way is loaded two k
+// at a time and stored as pairs.  Words of a row are xor-ed with 8 x the row's
+// block of 8: those stores, 8 rows apart from lane to lane, then reach all banks.
+// Loads are 16 bytes at any alignment (769 inputs make odd leading dimensions), at
+// the edges too, where they are moved inside the matrix and shifted back.
+// Workgroups b, b + 8, ... of a launch share an XCD: they take consecutive tiles,
+// so that its L2 reads few rows of A.
+// Bound: the chain load -> LDS -> product of a step, 1 to 2 us when one wave per
+// SIMD runs it.  The products of a training step have few tiles, so four groups
+// load a 64 x 32 tile (16 waves, a quarter of the steps; eight of them then hold
+// a 16 x 16 tile each) as long as every tile has a CU of its own: 104 KiB of LDS
+// leave no room for a second.  With a tile more than that, 64 x 64 tiles by 4
+// waves are faster.  M x 512 x 769: M = 1024 (256 tiles) 7.5 us against 10.4,
+// M = 1536 (384) 12.9 against 10.6, M = 8192 46.9 against 24.1.
+// Steps of 16 with 2-byte loads took 110 us at M = 1024; the eight products of a
+// training step at batch 1024 take 47 us (713), 4096 x 4096 x 4096 0.32 ms.
+constexpr int TM = 64, KS = 128, KPAD = 8;
+constexpr int kRowWords = (KS + KPAD) / 2;   // 32-bit words per LDS row
+__device__ __forceinline__ int lds_word(int r, int c) { return r * kRowWords + (c ^ ((r >> 3 & 7) << 3)); }
 
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(int transA, int transB, int M, int N, int K,
-                                                        const uint16_t *__restrict__ A, int lda,
-                                                        const uint16_t *__restrict__ B, int ldb, float *__restrict__ C,
-                                                        int ldc, const float *__restrict__ bias, float beta) {
-  __shared__ uint16_t sA[TM][TK + 2];   // sA[m][k]
-  __shared__ uint16_t sB[TK][TN + 2];   // sB[k][n]
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    // load A tile: 64 x 16 elements, 4 per thread
-    for (int e = tid; e < TM * TK; e += 256) {
-      const int mm = e / TK, kk = e % TK;
-      const int gm = m0 + mm, gk = k0 + kk;
-      uint16_t v = 0;
-      if (gm < M && gk < K) v = transA ? A[(int64_t)gk * lda + gm] : A[(int64_t)gm * lda + gk];
-      sA[mm][kk] = v;
+struct alignas(2) Elems8 {   // 8 elements at element alignment
+  uint16_t v[8];
+};
+__device__ __forceinline__ uint4 vec8(const uint16_t *q) {
+  return __builtin_bit_cast(uint4, *reinterpret_cast<const Elems8 *>(q));
+}
+// drop the first d of 8 elements, zeros move in
+__device__ __forceinline__ uint4 drop(uint4 v, unsigned d) {
+  uint64_t lo = (uint64_t)v.y << 32 | v.x, hi = (uint64_t)v.w << 32 | v.z;
+  if (d >= 8) return make_uint4(0, 0, 0, 0);
+  if (d >= 4) {
+    lo = hi;
+    hi = 0;
+  }
+  const unsigned n = 16 * (d & 3);
+  if (n) {
+    lo = lo >> n | hi << (64 - n);
+    hi >>= n;
+  }
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+// One operand's ROWS x KS tile: rows are m (or n), CONTIG_K when k runs along
+// memory rows.  Each of a group's 256 threads holds kPieces pieces of 8 elements:
+// along k, or (two k per thread) along the rows.  Rows past the matrix may hold
+// anything, they reach no stored element; k past it is zero.
+template <int ROWS, bool CONTIG_K>
+struct Operand {
+  static constexpr int kPieces = ROWS * KS / 8 / 256;
+  static constexpr int kLanes = CONTIG_K ? KS / 8 : ROWS / 8;   // pieces along memory
+  const uint16_t *p;
+  int64_t ld;
+  unsigned rows, K, r0;
+  const uint16_t *at[kPieces];   // of the next step, all inside the matrix
+  uint4 x[kPieces];
+
+  __device__ __forceinline__ unsigned row(int i, int tid) const {
+    return CONTIG_K ? r0 + (tid + 256 * i) / kLanes : r0 + 8 * ((tid + 256 * (i >> 1)) % kLanes);
+  }
+  __device__ __forceinline__ unsigned kofs(int i, int tid) const {
+    return CONTIG_K ? 8 * ((tid + 256 * i) % kLanes) : 2 * ((tid + 256 * (i >> 1)) / kLanes) + (i & 1);
+  }
+  __device__ __forceinline__ void start(unsigned k0, int tid) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const unsigned r = row(i, tid), k = k0 + kofs(i, tid);
+      at[i] = CONTIG_K ? p + (int64_t)(r < rows ? r : 0) * ld + k : p + (int64_t)k * ld + r;
     }
-    for (int e = tid; e < TK * TN; e += 256) {
-      const int kk = e / TN, nn = e % TN;
-      const int gk = k0 + kk, gn = n0 + nn;
-      uint16_t v = 0;
-      if (gk < K && gn < N) v = transB ? B[(int64_t)gn * ldb + gk] : B[(int64_t)gk * ldb + gn];
-      sB[kk][nn] = v;
+  }
+  __device__ __forceinline__ void load(unsigned k0, int tid, int64_t advance) {
+    if (k0 + KS <= K && (CONTIG_K || r0 + ROWS <= rows)) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) x[i] = vec8(at[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const unsigned r = row(i, tid), k = k0 + kofs(i, tid);
+        x[i] = edge(CONTIG_K ? (r < rows ? r : 0) : r, k);
+      }
     }
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) at[i] += advance;
+  }
+  // 8 elements from (r, k) along memory, zeros past its end or at k >= K
+  __device__ __forceinline__ uint4 edge(unsigned r, unsigned k) const {
+    const unsigned len = CONTIG_K ? K : rows, j = CONTIG_K ? k : r, line = CONTIG_K ? r : k < K ? k : 0;
+    const uint16_t *q = p + (int64_t)line * ld;
+    uint4 v;
+    if (len >= 8) {
+      const unsigned s = j + 8 <= len ? j : len - 8;
+      v = drop(vec8(q + s), j - s);
+    } else {
+      uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (unsigned e = 0; e < 8; ++e) w[e / 2] |= (j + e < len ? (uint32_t)q[j + e] : 0u) << 16 * (e & 1);
+      v = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    return CONTIG_K || k < K ? v : make_uint4(0, 0, 0, 0);
+  }
+  __device__ __forceinline__ void store(uint32_t *lds, int tid) const {
+    if (CONTIG_K) {
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const int e = tid + 256 * i;
+        *reinterpret_cast<uint4 *>(lds + lds_word(e / kLanes, 4 * (e % kLanes))) = x[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kPieces; i += 2) {
+        const int e = tid + 256 * (i >> 1);
+        uint32_t *q = lds + lds_word(8 * (e % kLanes), e / kLanes);
+        const uint32_t a[4] = {x[i].x, x[i].y, x[i].z, x[i].w}, b[4] = {x[i + 1].x, x[i + 1].y, x[i + 1].z, x[i + 1].w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          q[(2 * j) * kRowWords] = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);       // low halves
+          q[(2 * j + 1) * kRowWords] = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);   // high halves
+        }
+      }
+    }
+  }
+};
+
+template <int TN, int G, bool TA, bool TB>
+__global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned N, unsigned K,
+                                                            const uint16_t *__restrict__ A, int lda,
+                                                            const uint16_t *__restrict__ B, int ldb,
+                                                            float *__restrict__ C, int ldc,
+                                                            const float *__restrict__ bias, float beta) {
+  constexpr int kTileWords = (TM + TN) * kRowWords;
+  // 16 x 16 tiles of a multiplying wave, and those waves' place in the tile
+  constexpr int NI = G == 1 ? 2 : 1, NJ = G == 1 ? TN / 32 : 1, kWavesN = TN / (16 * NJ);
+  constexpr int kWaves = TM / (16 * NI) * kWavesN;
+  static_assert(kWaves <= 4 * G, "one wave per part of the tile");
+  __shared__ __align__(16) uint32_t lds[G * kTileWords];
+  const int tid = threadIdx.x & 255, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = wave >> 2;
+  const unsigned blk = blockIdx.y * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y;
+  const unsigned xcd = blk & 7, rem = tiles & 7;
+  const unsigned tile = xcd * (tiles >> 3) + (xcd < rem ? xcd : rem) + (blk >> 3);
+  const unsigned m0 = tile / gridDim.x * TM, n0 = tile % gridDim.x * TN;
+  const int wm = wave / kWavesN * 16 * NI, wn = wave % kWavesN * 16 * NJ;
+  Operand<TM, !TA> a{A, lda, M, K, m0, {}, {}};
+  Operand<TN, TB> b{B, ldb, N, K, n0, {}, {}};
+  const int64_t adv_a = TA ? (int64_t)G * KS * lda : G * KS, adv_b = TB ? G * KS : (int64_t)G * KS * ldb;
+  f32x4 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint32_t *const mine = lds + g * kTileWords;
+  // lane l: A rows (B columns) l % 16, k = 8 (l / 16) .. + 7
+  const int ar = wm + (lane & 15), br = wn + (lane & 15), kc = 4 * (lane >> 4);
+  unsigned kg = g * KS;   // first k of this group's part of the step
+  a.start(kg, tid);
+  b.start(kg, tid);
+  if (kg < K) {
+    a.load(kg, tid, adv_a);
+    b.load(kg, tid, adv_b);
+  }
+  for (unsigned k0 = 0; k0 < K; k0 += G * KS) {
+    if (kg < K) {
+      a.store(mine, tid);
+      b.store(mine + TM * kRowWords, tid);
+    }
+    kg += G * KS;
     __syncthreads();
-    // lane l: A rows (l%16), k = 4*(l/16)..+3 ; B cols (l%16), same k
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    bf16x4 a[2], b[2];
-    for (int i = 0; i < 2; ++i)
-      for (int q = 0; q < 4; ++q) a[i][q] = (short)sA[wm + 16 * i + r][kq + q];
-    for (int j = 0; j < 2; ++j)
-      for (int q = 0; q < 4; ++q) b[j][q] = (short)sB[kq + q][wn + 16 * j + r];
-    for (int i = 0; i < 2; ++i)
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+    if (kg < K) {
+      a.load(kg, tid, adv_a);
+      b.load(kg, tid, adv_b);
+    }
+    if (wave < kWaves) {
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        if (k0 + h * KS >= K) break;
+        const uint32_t *const ta = lds + h * kTileWords, *const tb = ta + TM * kRowWords;
+#pragma unroll
+        for (int q = 0; q < KS / 32; ++q) {
+          bf16x8 fa[NI], fb[NJ];
+#pragma unroll
+          for (int i = 0; i < NI; ++i)
+            fa[i] =
+                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ta + lds_word(ar + 16 * i, kc + 16 * q)));
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+            fb[j] =
+                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tb + lds_word(br + 16 * j, kc + 16 * q)));
+#pragma unroll
+          for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+        }
+      }
+    }
     __syncthreads();
   }
+  if (wave >= kWaves) return;
   // lane l holds C rows 4*(l/16)..+3, column l%16 of each 16 x 16 tile
   const int cn = lane & 15, cm = (lane >> 4) * 4;
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int gm = m0 + wm + 16 * i + cm + q, gn = n0 + wn + 16 * j + cn;
+        const unsigned gm = m0 + wm + 16 * i + cm + q, gn = n0 + wn + 16 * j + cn;
         if (gm < M && gn < N) {
           float v = acc[i][j][q];
           if (bias) v += bias[gn];
@@ -83,6 +244,15 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(int transA, int transB, 
           *dst = beta != 0.f ? beta * *dst + v : v;
         }
       }
+}
+
+template <int TN, int G>
+void launch_gemm(int transA, int transB, int M, int N, int K, const uint16_t *A, int lda, const uint16_t *B, int ldb,
+                 float *C, int ldc, const float *bias, float beta) {
+  auto kernel = transA ? (transB ? gemm_bf16_kernel<TN, G, true, true> : gemm_bf16_kernel<TN, G, true, false>)
+                       : (transB ? gemm_bf16_kernel<TN, G, false, true> : gemm_bf16_kernel<TN, G, false, false>);
+  const unsigned cols = ((unsigned)N + TN - 1) / TN, rows = ((unsigned)M + TM - 1) / TM;
+  hipLaunchKernelGGL(kernel, dim3(cols, rows), dim3(256 * G), 0, stream(), M, N, K, A, lda, B, ldb, C, ldc, bias, beta);
 }
 
 // GELU (tanh form) with the solver's tanh: g = 0.5 x (1 + tanh(c (x + 0.044715 x^3))).
@@ -117,13 +287,29 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
   if (i < n) y[i] = f32_to_bf16(x[i]);
 }
 
-// column sums of dZ [M x N] -> db [N] (bias gradient)
-__global__ void colsum_kernel(const float *__restrict__ dZ, float *__restrict__ db, int M, int N) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.f;
-  for (int m = 0; m < M; ++m) s += dZ[(int64_t)m * N + n];
-  db[n] = s;
+// column sums of dZ [M x N] -> db [N] (bias gradient).  A workgroup takes 32
+// columns with 32 threads each, which add every 32nd row; their sums are then
+// added in order.  1024 x 512: 235 us with one thread per column -> 3.9 us.
+constexpr int kSumCols = 32, kSumRows = 32;
+__global__ __launch_bounds__(kSumCols * kSumRows) void colsum_kernel(const float *__restrict__ dZ,
+                                                                     float *__restrict__ db, int M, int N) {
+  __shared__ float part[kSumRows][kSumCols + 1];
+  const int c = threadIdx.x % kSumCols, r = threadIdx.x / kSumCols;
+  for (int64_t n0 = (int64_t)blockIdx.x * kSumCols; n0 < N; n0 += (int64_t)gridDim.x * kSumCols) {
+    const int64_t n = n0 + c;
+    float s = 0.f;
+    if (n < N) {
+#pragma unroll 8
+      for (int m = r; m < M; m += kSumRows) s += dZ[(int64_t)m * N + n];
+    }
+    part[r][c] = s;
+    __syncthreads();
+    if (r == 0 && n < N) {
+      for (int k = 1; k < kSumRows; ++k) s += part[k][c];
+      db[n] = s;
+    }
+    __syncthreads();
+  }
 }
 
 // MSE loss gradient: dY = (2/(M*N)) (Y - T), loss partials per row.
@@ -178,9 +364,9 @@ int cm_gemm_bf16(int transA, int transB, int M, int N, int K, const void *A, int
     set_error("cm_gemm_bf16: bad arguments");
     return -3;
   }
-  dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-  hipLaunchKernelGGL(gemm_bf16_kernel, grid, dim3(256), 0, stream(), transA, transB, M, N, K, (const uint16_t *)A,
-                     lda, (const uint16_t *)B, ldb, C, ldc, bias, beta);
+  const int64_t tiles = (((int64_t)M + TM - 1) / TM) * (((int64_t)N + 31) / 32);
+  (tiles <= device_cus() ? launch_gemm<32, 4> : launch_gemm<64, 1>)(
+      transA, transB, M, N, K, (const uint16_t *)A, lda, (const uint16_t *)B, ldb, C, ldc, bias, beta);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -205,7 +391,9 @@ int cm_to_bf16(const float *x, void *y, int64_t n) {
 }
 
 int cm_colsum(const float *dZ, float *db, int M, int N) {
-  hipLaunchKernelGGL(colsum_kernel, dim3((N + 255) / 256), dim3(256), 0, stream(), dZ, db, M, N);
+  const int64_t groups = ((int64_t)N + kSumCols - 1) / kSumCols;
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)(groups < 65536 ? groups : 65536)), dim3(kSumCols * kSumRows), 0,
+                     stream(), dZ, db, M, N);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
