@@ -7,10 +7,10 @@
 // consecutive sections 4l..4l+3 in registers.  The Jacobi pressure sweep
 // exchanges the two lane-boundary pressures with DPP wave shifts, the three
 // step-control reductions run interleaved as DPP trees, and accept/reject is a
-// lane-uniform decision.  No LDS, no barriers.  The same
-// functions also run a block over a workgroup of 2 or 4 waves (2 or 1
-// sections per lane), exchanging wave-boundary values through LDS (Lay<N>
-// below); results are identical in every layout.
+// lane-uniform decision.  No LDS, no barriers.  The same functions also run a
+// block over a workgroup of 4 or 8 waves (2 or 1 sections per lane), which carry
+// their neighbours' sections and exchange pressures and totals through LDS
+// (Lay<N> below); results are identical in every layout.
 //
 // Arithmetic contract (shared with the CPU oracle): FP32, every operation
 // IEEE-rounded, no contraction (built with -ffp-contract=off), IEEE division
@@ -166,6 +166,30 @@ __device__ __forceinline__ void tree_sum2(float &x, float &y) {
 
 #define UNROLL _Pragma("unroll")
 
+// The four steps inside a row of 16 lanes, or the first three of them, for 1 to
+// 3 values (MAX0: the first is a maximum), as above.
+#define CM_TREE1(ctrl) \
+  "s_nop 1\n\tv_add_f32_dpp %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+#define CM_OCT_STEPS(step) step("quad_perm:[1,0,3,2]") step("quad_perm:[2,3,0,1]") step("row_half_mirror")
+#define CM_ROW_STEPS(step) CM_OCT_STEPS(step) step("row_mirror")
+template <int K, bool MAX0, bool ROW>
+__device__ __forceinline__ void tree_row(float (&v)[K]) {
+  static_assert(K >= 1 && K <= 3 && !(MAX0 && K != 3), "one to three sums, or a maximum and two sums");
+  if constexpr (K == 1) {
+    if constexpr (ROW) asm(CM_ROW_STEPS(CM_TREE1) : "+v"(v[0]));
+    else asm(CM_OCT_STEPS(CM_TREE1) : "+v"(v[0]));
+  } else if constexpr (K == 2) {
+    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE2) : "+v"(v[0]), "+v"(v[1]));
+    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE2) : "+v"(v[0]), "+v"(v[1]));
+  } else if constexpr (MAX0) {
+    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_MAX_SUM_SUM) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_MAX_SUM_SUM) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+  } else {
+    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_SUM3) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_SUM3) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+  }
+}
+
 __device__ __forceinline__ float in_at(const BmLaunch &a, int64_t idx) {
   return (idx >= 0 && idx < a.input_len) ? a.input[idx] : 0.0f;
 }
@@ -173,180 +197,6 @@ __device__ __forceinline__ float in_at(const BmLaunch &a, int64_t idx) {
 __device__ __forceinline__ float uniform(float x) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
-
-// ------------------------------------------------ section layouts -------
-// A block's 256 sections over W = 4 / N waves of one workgroup: lane l of wave
-// w holds the N consecutive sections N (64 w + l) .. N (64 w + l) + N - 1.
-//
-// N = 4 is one wave per block: neighbour pressures move by DPP wave shifts,
-// reductions run as DPP butterflies, nothing goes through LDS and there is no
-// barrier.  N = 2 and N = 1 spread a block over 2 or 4 waves, so a wave needs
-// about a half or a quarter of the registers and more blocks fit on a SIMD.
-// The wave-boundary pressures, section 0's pressure and each wave's partial
-// reductions then pass through a small LDS area behind a workgroup barrier.
-// The area has two halves used in turn, so one barrier per exchange suffices:
-// a wave writes a half again only after the next exchange's barrier, which
-// every wave reaches after its reads of that half.  Totals leave an exchange
-// through readfirstlane, so every branch that depends on them is a scalar
-// branch, and every wave of a block forms the same totals bit for bit (the
-// tree below) and takes the same branches: the barriers always match.
-template <int N>
-struct Lay {
-  static_assert(N == 1 || N == 2 || N == 4, "1, 2 or 4 sections per lane");
-  static constexpr int W = 4 / N;
-  int lane;
-  int wave;    // wave of the block (0 when W == 1)
-  float *xa;   // exchange area: 2 halves x W waves x 4 floats (W > 1)
-  int ph;      // half used by the next exchange
-
-  __device__ bool sec0() const { return (W == 1 || wave == 0) && lane == 0; }
-  __device__ bool last() const { return (W == 1 || wave == W - 1) && lane == 63; }
-  __device__ int base() const { return N * (64 * (W == 1 ? 0 : wave) + lane); }
-  // Slots that can hold section 254 or 255, whose lower coupling l_i is 0
-  // (l_i = 1 elsewhere): slots 2 and 3 when N = 4, every slot otherwise.
-  static constexpr bool has_low(int j) { return N == 4 ? j >= 2 : true; }
-  __device__ float low() const {
-    if (N == 4) return lane == 63 ? 0.0f : 1.0f;
-    return base() + N - 1 >= 254 ? 0.0f : 1.0f;
-  }
-
-  // Pressures of the sections just before and after this lane's slots (0 past
-  // either end of the block), from every lane's last and first slot.
-  __device__ __forceinline__ void nbrs(float last_v, float first_v, float &left, float &right) {
-    left = wave_shr1(last_v);
-    right = wave_shl1(first_v);
-    if constexpr (W > 1) {
-      float *h = xa + ph * 4 * W;
-      if (lane == 0) h[4 * wave] = first_v;
-      if (lane == 63) h[4 * wave + 1] = last_v;
-      __syncthreads();
-      const float from_prev = wave > 0 ? h[4 * (wave - 1) + 1] : 0.0f;
-      const float from_next = wave < W - 1 ? h[4 * (wave + 1)] : 0.0f;
-      if (lane == 0) left = from_prev;
-      if (lane == 63) right = from_next;
-      ph ^= 1;
-    }
-  }
-
-  // This wave's part of a reduction (N < 4), the same in every lane.  The
-  // one-wave tree is (s0 + s1) + (s2 + s3) over each lane's four sections,
-  // then xor 1, 2, 4, 8 up to the 64-section sums R_k and (R0 + R1) + (R2 + R3).
-  // Here a group of 4 sections spans 2 lanes (N = 2) or a quad (N = 1); each
-  // step below adds the same two partial sums as the matching one-wave step
-  // (IEEE addition is commutative), ending with R_{2w} + R_{2w+1} (N = 2) or
-  // R_w (N = 1).
-  __device__ __forceinline__ float part_sum(const float (&x)[N]) const {
-    float s = x[0];
-    if constexpr (N == 2) s = x[0] + x[1];
-    s = s + quad_xor1(s);
-    s = s + quad_xor2(s);
-    s = s + row_half_mirror(s);   // xor 4 once quads are uniform
-    s = s + row_mirror(s);        // xor 8 once octets are uniform
-    s = s + row_bcast15(s);       // rows 1 and 3 hold their 16-lane pair's sum
-    return readlane(s, 31) + readlane(s, 63);
-  }
-  __device__ __forceinline__ float part_max(const float (&x)[N]) const {
-    float s = x[0];
-    if constexpr (N == 2) s = fmaxf(x[0], x[1]);
-    s = fmaxf(s, quad_xor1(s));
-    s = fmaxf(s, quad_xor2(s));
-    s = fmaxf(s, row_half_mirror(s));
-    s = fmaxf(s, row_mirror(s));
-    s = fmaxf(s, row_bcast15(s));
-    return fmaxf(readlane(s, 31), readlane(s, 63));
-  }
-
-  // Block totals from the K wave parts in v (bit k of is_max: a maximum, else
-  // a sum) through one exchange: W = 2 adds (R0 + R1) + (R2 + R3) as
-  // part_0 + part_1, W = 4 as (R0 + R1) + (R2 + R3).
-  template <int K>
-  __device__ __forceinline__ void combine(float (&v)[K], unsigned is_max) {
-    static_assert(K <= 4, "4 values per wave and half");
-    float *h = xa + ph * 4 * W;
-    if (lane == 0) {
-      UNROLL for (int k = 0; k < K; ++k) h[4 * wave + k] = v[k];
-    }
-    __syncthreads();
-    UNROLL for (int k = 0; k < K; ++k) {
-      float r[W];
-      UNROLL for (int w = 0; w < W; ++w) r[w] = h[4 * w + k];
-      float t;
-      if constexpr (W == 2) {
-        t = (is_max >> k) & 1u ? fmaxf(r[0], r[1]) : r[0] + r[1];
-      } else {
-        t = (is_max >> k) & 1u ? fmaxf(fmaxf(r[0], r[1]), fmaxf(r[2], r[3])) : (r[0] + r[1]) + (r[2] + r[3]);
-      }
-      v[k] = uniform(t);
-    }
-    ph ^= 1;
-  }
-
-  __device__ __forceinline__ float sum(const float (&x)[N]) {
-    if constexpr (N == 4) {
-      return tree_sum(x[0], x[1], x[2], x[3]);
-    } else {
-      float v[1] = {part_sum(x)};
-      combine<1>(v, 0u);
-      return v[0];
-    }
-  }
-  // max of ex, sums of ey and ez: the three step-control reductions
-  __device__ __forceinline__ void reduce3(const float (&ex)[N], const float (&ey)[N], const float (&ez)[N],
-                                          float &emax, float &esum, float &fsum) {
-    if constexpr (N == 4) {
-      emax = fmaxf(fmaxf(ex[0], ex[1]), fmaxf(ex[2], ex[3]));
-      esum = (ey[0] + ey[1]) + (ey[2] + ey[3]);
-      fsum = (ez[0] + ez[1]) + (ez[2] + ez[3]);
-      tree_max_sum_sum(emax, esum, fsum);
-    } else {
-      float v[3] = {part_max(ex), part_sum(ey), part_sum(ez)};
-      combine<3>(v, 1u);
-      emax = v[0]; esum = v[1]; fsum = v[2];
-    }
-  }
-  // sums of the squares of two or three vectors
-  __device__ __forceinline__ void sum_sq2(const float (&x)[N], const float (&y)[N], float &sx, float &sy) {
-    float a[N], b[N];
-    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; }
-    if constexpr (N == 4) {
-      sx = (a[0] + a[1]) + (a[2] + a[3]);
-      sy = (b[0] + b[1]) + (b[2] + b[3]);
-      tree_sum2(sx, sy);
-    } else {
-      float v[2] = {part_sum(a), part_sum(b)};
-      combine<2>(v, 0u);
-      sx = v[0]; sy = v[1];
-    }
-  }
-  __device__ __forceinline__ void sum_sq3(const float (&x)[N], const float (&y)[N], const float (&z)[N], float &sx,
-                                          float &sy, float &sz) {
-    float a[N], b[N], c[N];
-    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; c[j] = z[j] * z[j]; }
-    if constexpr (N == 4) {
-      sx = (a[0] + a[1]) + (a[2] + a[3]);
-      sy = (b[0] + b[1]) + (b[2] + b[3]);
-      sz = (c[0] + c[1]) + (c[2] + c[3]);
-      tree_sum3(sx, sy, sz);
-    } else {
-      float v[3] = {part_sum(a), part_sum(b), part_sum(c)};
-      combine<3>(v, 0u);
-      sx = v[0]; sy = v[1]; sz = v[2];
-    }
-  }
-  // section 0's value (slot 0 of the lane that holds it) in every lane
-  __device__ __forceinline__ float sec0_value(float x0) {
-    if constexpr (W == 1) {
-      return readlane(x0, 0);
-    } else {
-      float *h = xa + ph * 4 * W;
-      if (wave == 0 && lane == 0) h[0] = x0;
-      __syncthreads();
-      const float v = uniform(h[0]);
-      ph ^= 1;
-      return v;
-    }
-  }
-};
 
 template <int N>
 __device__ __forceinline__ void ld_slots(const float *p, float (&o)[N]) {
@@ -369,6 +219,204 @@ __device__ __forceinline__ void st_slots(float *p, const float (&v)[N]) {
   else
     *p = v[0];
 }
+
+// ------------------------------------------------ section layouts -------
+// A block's 256 sections over the W waves of a workgroup, N consecutive ones
+// per lane.
+//
+// N = 4 is one wave per block (W = 1): neighbour pressures move by DPP wave
+// shifts, reductions run as DPP butterflies, nothing goes through LDS and there
+// is no barrier.
+//
+// N = 2 and N = 1 spread a block over W = 4 and 8 waves, for launches that
+// leave SIMDs without a wave.  A wave owns 32 N sections (two rows of lanes)
+// and carries 16 N more on either side of them (on one side, twice as many, in
+// the first and last wave, so that a wave's ends are the block's ends).  All
+// its lanes do the same work, so a Jacobi sweep needs no exchange: each one
+// spoils the outermost valid section only, and after up to kReach sweeps the
+// owned sections are still those of the one-wave layout.  Then the owners'
+// pressures pass to the others through LDS behind a workgroup barrier (share),
+// and everything else follows from them in every lane that holds the section.
+// Totals of the owned sections pass the same way.  The area has two halves used
+// in turn, so one barrier per exchange suffices: a wave writes a half again
+// only after the next exchange's barrier, which every wave reaches after its
+// reads of that half.  Totals leave an exchange through readlane, so every
+// branch that depends on them is a scalar branch, and every wave of a block
+// forms the same totals bit for bit (the tree below) and takes the same
+// branches: the barriers always match.
+template <int N>
+struct Lay {
+  static_assert(N == 1 || N == 2 || N == 4, "1, 2 or 4 sections per lane");
+  static constexpr int W = N == 4 ? 1 : 8 / N;
+  static constexpr int kReach = N == 4 ? 1 << 30 : 16 * N - 1;   // sweeps between exchanges; one valid neighbour remains
+  // bytes of a half: two vectors, 2 W part totals of up to 4 floats, and a place
+  // for what lanes write that own nothing (a power of two: halves alternate by xor)
+  static constexpr unsigned kVec = 4 * CM_SECTIONS, kParts = 2 * kVec, kIdle = kParts + 16 * 2 * W, kHalf = 4096;
+  static_assert(kIdle + 4 * 64 * 4 <= kHalf, "a half holds its idle place");
+  int lane;
+  int wave;    // wave of the block (0 when W == 1)
+  char *xa;    // exchange area: 2 halves (W > 1)
+  float p0;    // section 0's pressure of the last share (W > 1)
+  unsigned put_at, part_at, get_at, total_at;   // this lane's places in the half of the next exchange (W > 1)
+
+  __device__ __forceinline__ Lay(int lane_, int wave_, char *xa_) : lane(lane_), wave(wave_), xa(xa_), p0(0.f) {
+    if constexpr (W > 1) {
+      const int rel = lane - own_lane();
+      unsigned mine = 4 * base(), part = kParts + 16 * (2 * wave + (rel >> 4));
+      asm volatile("" : "+v"(mine), "+v"(part));   // selected below, not branched around
+      put_at = (unsigned)rel < 32u ? mine : kIdle + 4 * N * lane;
+      part_at = (rel & ~16) == 0 ? part : kIdle + 16 * lane;
+      get_at = mine;
+      total_at = kParts + 16 * (lane & (2 * W - 1));
+    }
+  }
+
+  // The lane, compared anew at each use (W > 1): masks of lanes kept over the
+  // steps would take more scalar registers than there are.
+  __device__ __forceinline__ int here() const {
+    int l = lane;
+    if constexpr (W > 1) asm volatile("" : "+v"(l));
+    return l;
+  }
+  __device__ bool sec0() const { return (W == 1 || wave == 0) && here() == 0; }
+  __device__ bool last() const { return (W == 1 || wave == W - 1) && here() == 63; }
+  __device__ int base() const {
+    if constexpr (W == 1) return N * lane;
+    const int first = wave == 0 ? 0 : (wave == W - 1 ? CM_SECTIONS - 64 * N : 32 * N * wave - 16 * N);
+    return first + N * lane;
+  }
+  // first of the 32 lanes whose sections this wave owns
+  __device__ int own_lane() const { return wave == 0 ? 0 : (wave == W - 1 ? 32 : 16); }
+  __device__ bool own() const { return W == 1 || (unsigned)(here() - own_lane()) < 32u; }
+  // Slots that can hold section 254 or 255, whose lower coupling l_i is 0
+  // (l_i = 1 elsewhere): slots 2 and 3 when N = 4, every slot otherwise.
+  static constexpr bool has_low(int j) { return N == 4 ? j >= 2 : true; }
+  __device__ float low() const {
+    if (N == 4) return lane == 63 ? 0.0f : 1.0f;
+    return base() + N - 1 >= 254 ? 0.0f : 1.0f;
+  }
+
+  // Pressures of the sections just before and after this lane's slots (0 past
+  // either end of the wave), from every lane's last and first slot.
+  __device__ __forceinline__ void nbrs(float last_v, float first_v, float &left, float &right) const {
+    left = wave_shr1(last_v);
+    right = wave_shl1(first_v);
+  }
+
+  // ---- exchanges (W > 1) ----
+  // Writes of an exchange: the owned sections of vector `which`.
+  __device__ __forceinline__ void put(const float (&x)[N], int which) const {
+    st_slots<N>(reinterpret_cast<float *>(xa + put_at) + which * CM_SECTIONS, x);
+  }
+  // The one-wave tree is (s0 + s1) + (s2 + s3) over each lane's four sections,
+  // then xor 1, 2, 4, 8 up to the 64-section sums R_k and (R0 + R1) + (R2 + R3).
+  // Here a group of 4 sections spans 2 lanes (N = 2) or a quad (N = 1), a row of
+  // lanes holds 16 N sections, and lane i continues with the total of row i of
+  // the block: each step adds the same two partial sums as the matching one-wave
+  // step (IEEE addition is commutative).
+  template <int K, bool MAX0>
+  __device__ __forceinline__ void put_parts(float (&v)[K]) const {
+    tree_row<K, MAX0, true>(v);
+    float *h = reinterpret_cast<float *>(xa + part_at);
+    UNROLL for (int k = 0; k < K; ++k) h[k] = v[k];
+  }
+  // Ends the writes; returns the half to read from.  LDS only is waited for:
+  // rows on their way to memory are not.
+  struct Half {
+    unsigned get_at, total_at;
+  };
+  __device__ __forceinline__ Half meet() {
+    const Half h{get_at, total_at};
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    put_at ^= kHalf; part_at ^= kHalf; get_at ^= kHalf; total_at ^= kHalf;
+    return h;
+  }
+  template <int K, bool MAX0>
+  __device__ __forceinline__ void get_totals(const Half &h, float (&v)[K]) const {
+    const float *t = reinterpret_cast<const float *>(xa + h.total_at);
+    UNROLL for (int k = 0; k < K; ++k) v[k] = t[k];
+    tree_row<K, MAX0, N == 1>(v);
+    UNROLL for (int k = 0; k < K; ++k) v[k] = readlane(v[k], 0);
+  }
+  __device__ __forceinline__ void get(const Half &h, int which, float (&x)[N]) {
+    ld_slots<N>(reinterpret_cast<const float *>(xa + h.get_at) + which * CM_SECTIONS, x);
+    p0 = reinterpret_cast<const float *>(xa + (h.get_at & kHalf))[which * CM_SECTIONS];
+  }
+  // Every lane's pressures from their owners.
+  __device__ __forceinline__ void share(float (&p)[N]) {
+    if constexpr (W > 1) {
+      put(p, 0);
+      get(meet(), 0, p);
+    }
+  }
+  template <int K, bool MAX0>
+  __device__ __forceinline__ void totals(float (&v)[K]) {
+    put_parts<K, MAX0>(v);
+    get_totals<K, MAX0>(meet(), v);
+  }
+  static __device__ __forceinline__ float lane_sum(const float (&x)[N]) {
+    if constexpr (N == 4) return (x[0] + x[1]) + (x[2] + x[3]);
+    else if constexpr (N == 2) return x[0] + x[1];
+    else return x[0];
+  }
+  static __device__ __forceinline__ float lane_max(const float (&x)[N]) {
+    if constexpr (N == 4) return fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+    else if constexpr (N == 2) return fmaxf(x[0], x[1]);
+    else return x[0];
+  }
+
+  __device__ __forceinline__ float sum(const float (&x)[N]) {
+    if constexpr (N == 4) {
+      return tree_sum(x[0], x[1], x[2], x[3]);
+    } else {
+      float v[1] = {lane_sum(x)};
+      totals<1, false>(v);
+      return v[0];
+    }
+  }
+  // reduce3 and share in one exchange (W > 1)
+  __device__ __forceinline__ void reduce3_share(const float (&ex)[N], const float (&ey)[N], const float (&ez)[N],
+                                                float (&p)[N], float &emax, float &esum, float &fsum) {
+    float v[3] = {lane_max(ex), lane_sum(ey), lane_sum(ez)};
+    put(p, 0);
+    put_parts<3, true>(v);
+    const Half h = meet();
+    get(h, 0, p);
+    get_totals<3, true>(h, v);
+    emax = v[0]; esum = v[1]; fsum = v[2];
+  }
+  // max of ex, sums of ey and ez: the three step-control reductions
+  __device__ __forceinline__ void reduce3(const float (&ex)[N], const float (&ey)[N], const float (&ez)[N],
+                                          float &emax, float &esum, float &fsum) {
+    float v[3] = {lane_max(ex), lane_sum(ey), lane_sum(ez)};
+    if constexpr (N == 4) tree_max_sum_sum(v[0], v[1], v[2]);
+    else totals<3, true>(v);
+    emax = v[0]; esum = v[1]; fsum = v[2];
+  }
+  // sums of the squares of two or three vectors
+  __device__ __forceinline__ void sum_sq2(const float (&x)[N], const float (&y)[N], float &sx, float &sy) {
+    float a[N], b[N];
+    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; }
+    float v[2] = {lane_sum(a), lane_sum(b)};
+    if constexpr (N == 4) tree_sum2(v[0], v[1]);
+    else totals<2, false>(v);
+    sx = v[0]; sy = v[1];
+  }
+  __device__ __forceinline__ void sum_sq3(const float (&x)[N], const float (&y)[N], const float (&z)[N], float &sx,
+                                          float &sy, float &sz) {
+    float a[N], b[N], c[N];
+    UNROLL for (int j = 0; j < N; ++j) { a[j] = x[j] * x[j]; b[j] = y[j] * y[j]; c[j] = z[j] * z[j]; }
+    float v[3] = {lane_sum(a), lane_sum(b), lane_sum(c)};
+    if constexpr (N == 4) tree_sum3(v[0], v[1], v[2]);
+    else totals<3, false>(v);
+    sx = v[0]; sy = v[1]; sz = v[2];
+  }
+  // section 0's pressure in every lane (W > 1: of the last share)
+  __device__ __forceinline__ float sec0_value(float x0) const {
+    if constexpr (W == 1) return readlane(x0, 0);
+    else return p0;
+  }
+};
 
 // ------------------------------------------------- one time block -------
 // Per-lane constants of an item: section parameters of this lane's N sections.
@@ -507,6 +555,67 @@ __device__ __forceinline__ void sweeps_asm(const float (&Y)[4], const float (&r)
   }
 }
 
+// The spread layouts' sweeps.  Section 254 sits in a slot whose left neighbour
+// comes through DPP, which cannot fold l_i: a move of the right neighbour and a
+// multiply-add of l_i and the left one take its place (7 instructions for two
+// sections, 4 and a wait for one).  Operands read through DPP are two
+// instructions old, here and after the last sweep.
+#define CM_SWEEP2(p0, p1, t0, t1)                                                                    \
+  "v_mov_b32 %[" t0 "], %[" p1 "]\n\t"                                                               \
+  "v_add_f32_dpp %[a1], %[" p0 "], %[" p0 "] wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"              \
+  "v_fmac_f32_dpp %[" t0 "], %[" p1 "], %[low] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  "v_sub_f32 %[" t1 "], %[Y1], %[a1]\n\t"                                                            \
+  "v_sub_f32 %[" t0 "], %[Y0], %[" t0 "]\n\t"                                                        \
+  "v_mul_f32 %[" t0 "], %[r0], %[" t0 "]\n\t"                                                        \
+  "v_mul_f32 %[" t1 "], %[r1], %[" t1 "]\n\t"
+#define CM_SWEEP1(p0, t0)                                                                            \
+  "s_nop 1\n\t"                                                                                      \
+  "v_mov_b32_dpp %[" t0 "], %[" p0 "] wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"        \
+  "v_fmac_f32_dpp %[" t0 "], %[" p0 "], %[low] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+  "v_sub_f32 %[" t0 "], %[Y0], %[" t0 "]\n\t"                                                        \
+  "v_mul_f32 %[" t0 "], %[r0], %[" t0 "]\n\t"
+#define CM_PAIR2 CM_SWEEP2("p0", "p1", "t0", "t1") CM_SWEEP2("t0", "t1", "p0", "p1")
+#define CM_PAIR1 CM_SWEEP1("p0", "t0") CM_SWEEP1("t0", "p0")
+#define CM_LOOP(body) \
+  "s_nop 1\n" "1:\n\t" body "s_sub_i32 %[n], %[n], 1\n\ts_cmp_lg_u32 %[n], 0\n\ts_cbranch_scc1 1b\n\t"
+template <int PAIRS, int N>
+__device__ __forceinline__ void sweeps_spread(const float (&Y)[N], const float (&r)[N], float low, float (&p)[N],
+                                              int J) {
+  int n = J / (2 * PAIRS);
+  if constexpr (N == 2) {
+    // of the wave's last lane, which has no right neighbour (as a3 above)
+    float a1 = low * p[0] + 0.0f, t0, t1;
+#define CM_IO2 [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [a1] "+&v"(a1), [t0] "=&v"(t0), [t1] "=&v"(t1)
+#define CM_IN2 [Y0] "v"(Y[0]), [Y1] "v"(Y[1]), [r0] "v"(r[0]), [r1] "v"(r[1]), [low] "v"(low)
+    if (n > 0) {
+      if constexpr (PAIRS == 1) asm(CM_LOOP(CM_PAIR2) : CM_IO2, [n] "+&s"(n) : CM_IN2 : "scc");
+      else asm(CM_LOOP(CM_PAIR2 CM_PAIR2) : CM_IO2, [n] "+&s"(n) : CM_IN2 : "scc");
+    }
+    if (PAIRS == 2 && (J & 2)) asm("s_nop 1\n\t" CM_PAIR2 "s_nop 1" : CM_IO2 : CM_IN2);
+    if (J & 1) {
+      asm("s_nop 1\n\t" CM_SWEEP2("p0", "p1", "t0", "t1") "s_nop 1" : CM_IO2 : CM_IN2);
+      p[0] = t0; p[1] = t1;
+    }
+#undef CM_IO2
+#undef CM_IN2
+  } else {
+    float t0;
+#define CM_IO1 [p0] "+&v"(p[0]), [t0] "=&v"(t0)
+#define CM_IN1 [Y0] "v"(Y[0]), [r0] "v"(r[0]), [low] "v"(low)
+    if (n > 0) {
+      if constexpr (PAIRS == 1) asm(CM_LOOP(CM_PAIR1) : CM_IO1, [n] "+&s"(n) : CM_IN1 : "scc");
+      else asm(CM_LOOP(CM_PAIR1 CM_PAIR1) : CM_IO1, [n] "+&s"(n) : CM_IN1 : "scc");
+    }
+    if (PAIRS == 2 && (J & 2)) asm(CM_PAIR1 "s_nop 1" : CM_IO1 : CM_IN1);
+    if (J & 1) {
+      asm(CM_SWEEP1("p0", "t0") "s_nop 1" : CM_IO1 : CM_IN1);
+      p[0] = t0;
+    }
+#undef CM_IO1
+#undef CM_IN1
+  }
+}
+
 // J is wave-uniform: the count goes to a scalar register.  U (1, 2 or 4) is
 // the unroll of the sweep loop, a launch knob of the autotuner: sweeps come in
 // pairs (U = 2) or two pairs (U = 4) per trip, so the two iterates alternate
@@ -517,21 +626,27 @@ __device__ __forceinline__ void jacobi_sweeps(Lay<N> &L, const float (&Y)[N], co
                                               int J) {
   static_assert(U == 1 || U == 2 || U == 4, "unroll 1, 2 or 4");
   J = __builtin_amdgcn_readfirstlane(J);
+  float r[N];
+  if constexpr (U != 1) {
+    UNROLL for (int j = 0; j < N; ++j) r[j] = k.rsm[j];
+  }
   if constexpr (N == 4 && U != 1) {
-    const float r[4] = {k.rsm[0], k.rsm[1], k.rsm[2], k.rsm[3]};
     sweeps_asm<U / 2>(Y, r, k.low, p, J);
   } else {
-    float q[N];
-    int i = 0;
-    if (U != 1) {
-      for (; i + 2 <= J; i += 2) {
-        jacobi_sweep(L, Y, k, p, q);
-        jacobi_sweep(L, Y, k, q, p);
+    for (;;) {
+      const int c = J < Lay<N>::kReach ? J : Lay<N>::kReach;
+      if constexpr (U != 1) {
+        sweeps_spread<U / 2>(Y, r, k.low, p, c);
+      } else {
+        float q[N];
+        for (int i = 0; i < c; ++i) {
+          jacobi_sweep(L, Y, k, p, q);
+          UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
+        }
       }
-    }
-    for (; i < J; ++i) {
-      jacobi_sweep(L, Y, k, p, q);
-      UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
+      J -= c;
+      if (J <= 0) break;
+      L.share(p);
     }
   }
 }
@@ -556,10 +671,11 @@ __device__ __forceinline__ float resid2(Lay<N> &L, const float (&Y)[N], const K 
   UNROLL for (int j = 0; j < N; ++j) r[j] = r[j] * r[j];
   return L.sum(r);
 }
-// Squared residual of p and, from the same couplings, the next sweep's iterate q.
+// Squared residual of p and, from the same couplings, the next sweep's iterate q
+// (spread layouts: both owned sections only; take() picks one for all lanes).
 template <int N, class K>
 __device__ __forceinline__ float resid2_sweep(Lay<N> &L, const float (&Y)[N], const K &k, const float (&p)[N],
-                                              float (&q)[N]) {
+                                              float (&q)[N], typename Lay<N>::Half &h) {
   float left, right, r[N];
   L.nbrs(p[N - 1], p[0], left, right);
   UNROLL for (int j = 0; j < N; ++j) {
@@ -570,7 +686,25 @@ __device__ __forceinline__ float resid2_sweep(Lay<N> &L, const float (&Y)[N], co
     r[j] = r[j] * r[j];
     q[j] = (Y[j] - c) * k.rsm[j];
   }
-  return L.sum(r);
+  if constexpr (N == 4) {
+    return L.sum(r);
+  } else {
+    float v[1] = {L.lane_sum(r)};
+    L.put(p, 0);
+    L.put(q, 1);
+    L.template put_parts<1, false>(v);
+    h = L.meet();
+    L.template get_totals<1, false>(h, v);
+    return v[0];
+  }
+}
+template <int N>
+__device__ __forceinline__ void take(Lay<N> &L, const typename Lay<N>::Half &h, int which, float (&p)[N], const float (&x)[N]) {
+  if constexpr (N == 4) {
+    UNROLL for (int j = 0; j < N; ++j) p[j] = x[j];
+  } else {
+    L.get(h, which, p);
+  }
 }
 
 template <bool TOL, int N>
@@ -726,16 +860,23 @@ __device__ __forceinline__ int jacobi_tol(Lay<N> &L, const cm_bm_scalars &sc, co
   const float tau2 = sc.tol_rel * sc.tol_rel;
   const float lim = tau2 * yy;
   int J = 0;
-  if (rr <= lim || J >= sc.max_sweeps) return J;
+  if (rr <= lim || J >= sc.max_sweeps) {
+    L.share(p);
+    return J;
+  }
   int kk = sc.check_every < sc.max_sweeps ? sc.check_every : sc.max_sweeps;
   jacobi_sweeps<U>(L, Y, k, p, kk);
   for (;;) {
     J += kk;
     float q[N];
-    rr = resid2_sweep(L, Y, k, p, q);
-    if (rr <= lim || J >= sc.max_sweeps) return J;
+    typename Lay<N>::Half h{};
+    rr = resid2_sweep(L, Y, k, p, q, h);
+    if (rr <= lim || J >= sc.max_sweeps) {
+      take(L, h, 0, p, p);
+      return J;
+    }
     kk = sc.check_every < sc.max_sweeps - J ? sc.check_every : sc.max_sweeps - J;
-    UNROLL for (int j = 0; j < N; ++j) p[j] = q[j];
+    take(L, h, 1, p, q);
     jacobi_sweeps<U>(L, Y, k, p, kk - 1);
   }
 }
@@ -765,17 +906,8 @@ __device__ __forceinline__ void pass_finish(Lay<N> &L, const K &k, const ItemSca
 // divided out: the float quotient is above 6 where the exact one is above the
 // midpoint 6 + 2^-22 (a tie rounds to 6), and below 0.5 where the exact one is
 // below 0.5 - 2^-26; esum times either bound is exact in FP64.
-template <int N>
-__device__ __forceinline__ bool pass_control(Lay<N> &L, const cm_bm_scalars &sc, const ItemScal &c, float &dt,
-                                             const HalfN<N> &n, const float (&vref)[N], const float (&aref)[N]) {
-  float ex[N], ey[N], ez[N];
-  UNROLL for (int j = 0; j < N; ++j) {
-    ex[j] = __builtin_fabsf(aref[j] - n.a[j]);
-    ey[j] = __builtin_fabsf(n.v[j] - vref[j]);
-    ez[j] = ey[j] - fmaxf(c.mtt, n.v[j] * dt);
-  }
-  float emax, esum, fsum;
-  L.reduce3(ex, ey, ez, emax, esum, fsum);
+__device__ __forceinline__ bool step_control(const cm_bm_scalars &sc, const ItemScal &c, float &dt, float emax,
+                                             float esum, float fsum) {
   if (sc.decision_mode == 1) { emax = 0.f; esum = 0.f; fsum = 0.f; }
   bool above = false, below = true;   // L > 6, L < 0.5
   if (esum > c.mmspt) {
@@ -792,6 +924,25 @@ __device__ __forceinline__ bool pass_control(Lay<N> &L, const cm_bm_scalars &sc,
   dt = dt * 2.0f;
   if (dt > c.dt_max) dt = c.dt_max;
   return false;
+}
+// Its terms: the changes of acceleration and velocity since the last pass.
+template <int N>
+__device__ __forceinline__ void control_terms(const ItemScal &c, float dt, const float (&v)[N], const float (&a)[N],
+                                              const float (&vref)[N], const float (&aref)[N], float (&ex)[N],
+                                              float (&ey)[N], float (&ez)[N]) {
+  UNROLL for (int j = 0; j < N; ++j) {
+    ex[j] = __builtin_fabsf(aref[j] - a[j]);
+    ey[j] = __builtin_fabsf(v[j] - vref[j]);
+    ez[j] = ey[j] - fmaxf(c.mtt, v[j] * dt);
+  }
+}
+template <int N>
+__device__ __forceinline__ bool pass_control(Lay<N> &L, const cm_bm_scalars &sc, const ItemScal &c, float &dt,
+                                             const HalfN<N> &n, const float (&vref)[N], const float (&aref)[N]) {
+  float ex[N], ey[N], ez[N], emax, esum, fsum;
+  control_terms(c, dt, n.v, n.a, vref, aref, ex, ey, ez);
+  L.reduce3(ex, ey, ez, emax, esum, fsum);
+  return step_control(sc, c, dt, emax, esum, fsum);
 }
 
 // Commit of a step whose passes left side n: counters, sample advance with
@@ -819,7 +970,7 @@ __device__ __forceinline__ void step_commit(const BmLaunch &a, const cm_bm_item 
           if constexpr (N == 4)
             *reinterpret_cast<float4 *>(a.speeds + (int64_t)s.in_s * CM_SECTIONS + 4 * L.lane) =
                 make_float4(n.v[0], n.v[1], n.v[2], n.v[3]);
-          else
+          else if (L.own())
             st_slots<N>(a.speeds + (int64_t)s.in_s * CM_SECTIONS + L.base(), n.v);
         }
         if (L.sec0()) {
@@ -894,7 +1045,31 @@ __device__ __forceinline__ int solve_pass(Lay<N> &L, const cm_bm_scalars &sc, co
     return jacobi_tol<U>(L, sc, k, Y, yy, p, rr);
   } else {
     jacobi_sweeps<U>(L, Y, k, p, J_fixed);
+    L.share(p);
     return J_fixed;
+  }
+}
+
+// The solve, end and control of a corrector pass.  The fixed sweeps of a spread
+// block leave the owned pressures; these and the control's totals pass in one
+// exchange.
+template <bool TOL, int U, int N>
+__device__ __forceinline__ bool correct_end(const BmLaunch &a, Lay<N> &L, const ItemConstN<N> &k, const ItemScal &c,
+                                            ItemStateN<N> &s, HalfN<N> &n, const PassTerms<N> &T, const float (&Y)[N],
+                                            float sf, const float (&vref)[N], const float (&aref)[N], int J_fixed) {
+  if constexpr (N == 4 || TOL) {
+    s.n_sweeps += solve_pass<TOL, U>(L, a.sc, k, Y, s.p, J_fixed);
+    pass_finish(L, k, c, n, s.p, T, sf);
+    return pass_control(L, a.sc, c, s.dt, n, vref, aref);
+  } else {
+    jacobi_sweeps<U>(L, Y, k, s.p, J_fixed);
+    s.n_sweeps += J_fixed;
+    float acc[N], ex[N], ey[N], ez[N], emax, esum, fsum;
+    UNROLL for (int j = 0; j < N; ++j) acc[j] = (s.p[j] + T.G[j]) * k.rmass[j];
+    control_terms(c, s.dt, n.v, acc, vref, aref, ex, ey, ez);
+    L.reduce3_share(ex, ey, ez, s.p, emax, esum, fsum);
+    pass_finish(L, k, c, n, s.p, T, sf);
+    return step_control(a.sc, c, s.dt, emax, esum, fsum);
   }
 }
 
@@ -935,20 +1110,14 @@ __device__ __forceinline__ void step(const BmLaunch &a, const cm_bm_item &it, La
     UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
     correct(o, n, s.dt);
     pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
-    J = solve_pass<TOL, U>(L, a.sc, k, Y, s.p, a.sc.j_slow);
-    s.n_sweeps += J;
-    pass_finish(L, k, c, n, s.p, T, sf);
-    another = pass_control(L, a.sc, c, s.dt, n, vref, aref);
+    another = correct_end<TOL, U>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_slow);
     passes = 2;
     if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
     while (another) {
       UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
       correct(o, n, s.dt);
       pass_rhs<false>(k, c, n, s.Ptm, sf, L, T, Y);
-      J = solve_pass<TOL, U>(L, a.sc, k, Y, s.p, a.sc.j_fast);
-      s.n_sweeps += J;
-      pass_finish(L, k, c, n, s.p, T, sf);
-      another = pass_control(L, a.sc, c, s.dt, n, vref, aref);
+      another = correct_end<TOL, U>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_fast);
       ++passes;
       if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
     }

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(3)))
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int idx = blockIdx.x * WAVES + wave;
   __shared__ float4 pold_lds[WS ? WAVES * 65 : 1];
-  Lay<4> L{lane, 0, nullptr, 0};
+  Lay<4> L(lane, 0, nullptr);
   if (idx < a.n_items)
     run_item<4, TOL, WS, U>(a, __builtin_amdgcn_readfirstlane(a.order ? a.order[idx] : idx), L,
                             pold_lds + (WS ? wave * 65 : 0));
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
   const int idx = __builtin_amdgcn_readfirstlane(valid ? (a.order ? a.order[slot] : slot) : slot);   // item of this wave
   float4 *pold = pold_lds + wave * 65;
   float4 *keep = keep_lds + wave * 3 * 64;   // G, nxis, Ptm of the predictor pass
-  Lay<4> L{lane, 0, nullptr, 0};             // one wave per block
+  Lay<4> L(lane, 0, nullptr);             // one wave per block
 
   // zero the feature tile once (rows >= G stay zero)
   for (int e = threadIdx.x; e < 16 * WS_XS; e += 64 * G) Xs[e] = 0;
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(64 * G) void bm_ws_kernel(BmLaunch a, WsArgs w) {
 
 // Launcher used by the C-ABI layer.  sections_per_lane 4: one wave per block,
 // waves_per_block (1, 2 or 4) blocks per workgroup of grid_blocks; 2 or 1: one
-// block per workgroup of 2 or 4 waves, one workgroup per block (grid_blocks is
+// block per workgroup of 4 or 8 waves, one workgroup per block (grid_blocks is
 // not used).  Jacobi unroll 1, 2 or 4.
 extern "C" int cm_launch_bm(const cm::BmLaunch *a, int waves_per_block, int unroll, int sections_per_lane,
                             int grid_blocks, hipStream_t stream) {

@@ -72,7 +72,7 @@ struct BMHolder {
   int waves_per_block = 1;
   int persistent = 0;
   int jacobi_unroll = 2;   // Jacobi sweep loop unroll of bm_kernel launches (cm_set_bm_jacobi_unroll)
-  int sections_per_lane = 4;   // block layout of fused-kernel launches (cm_set_bm_sections_per_lane)
+  int sections_per_lane = 0;   // block layout of fused-kernel launches (cm_set_bm_sections_per_lane); 0: by size
   // solver options for BMOHCNewKernel launches (cm_set_bm_solver); defaults = reference method
   int jacobi_mode = 0, check_every = 4, max_sweeps = 1000, warm_start = 0;
   float tol_rel = 1e-4f;
@@ -202,8 +202,18 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
     rc = cm_launch_bm_ws(&a, &w, device_cus(), stream());
     rc = rc > 0 ? 0 : rc;
   } else {
-    rc = cm_launch_bm(&a, waves_per_block, unroll > 0 ? unroll : g_bm.jacobi_unroll,
-                      sections_per_lane > 0 ? sections_per_lane : g_bm.sections_per_lane, grid, stream());
+    if (sections_per_lane <= 0) sections_per_lane = g_bm.sections_per_lane;
+    if (sections_per_lane <= 0) {
+      // Spread a block over four waves where each CU has at most one: its SIMDs
+      // would run one wave or none.  Only the fixed sweeps gain (one exchange
+      // between waves per pass; solving to a tolerance has one per check).
+      // Blocks of 0.2 s of tones, ms for 4 and 2 sections per lane: 10 blocks 91.5
+      // and 85.8, 250 blocks 101.7 and 89.8, 500 blocks 104.7 and 111.2; to a
+      // tolerance 12 blocks 171 and 264.
+      sections_per_lane = sc.jacobi_mode == 0 && n_items <= device_cus() ? 2 : 4;
+    }
+    rc = cm_launch_bm(&a, waves_per_block, unroll > 0 ? unroll : g_bm.jacobi_unroll, sections_per_lane, grid,
+                      stream());
   }
   if (rc) {
     set_error("BM kernel launch failed (%d): %s", rc, hipGetErrorString(hipGetLastError()));
@@ -422,6 +432,11 @@ int cm_set_bm_sections_per_lane(int sections_per_lane) {
     return -3;
   }
   g_bm.sections_per_lane = sections_per_lane;
+  return 0;
+}
+
+int cm_reset_bm_sections_per_lane(void) {
+  g_bm.sections_per_lane = 0;
   return 0;
 }
 

@@ -65,14 +65,16 @@ int cm_set_bm_launch(int waves_per_block, int persistent);
  * include/cochlea.cuh:13962-13982).  Results are identical for every value;
  * cm_bm_autotune sets the fastest. */
 int cm_set_bm_jacobi_unroll(int unroll);
-/* Sections per lane (1, 2 or 4; default 4) of the following fused BM launches
- * (the learned lockstep kernel keeps 4).  4: one wave64 per time block, 4
- * sections per lane; 2 or 1: a block over a workgroup of 2 or 4 waves, the
- * wave-boundary pressures and partial reductions exchanged through LDS (the
- * reference runs one section per thread in 256-thread blocks,
+/* Sections per lane (1, 2 or 4) of the following fused BM launches (the learned
+ * lockstep kernel keeps 4).  4: one wave64 per time block, 4 sections per lane;
+ * 2 or 1: a block over a workgroup of 4 or 8 waves that carry their neighbours'
+ * sections and exchange pressures and totals through LDS (the reference runs
+ * one section per thread in 256-thread blocks,
  * include/cochlea.cuh:13708-13736).  Results are identical for every value;
- * cm_bm_autotune sets the fastest. */
+ * cm_bm_autotune sets the fastest.  Unset, or after cm_reset_: 4, or 2 for a
+ * fixed-sweep launch of no more blocks than the GPU has CUs. */
 int cm_set_bm_sections_per_lane(int sections_per_lane);
+int cm_reset_bm_sections_per_lane(void);
 /* Solver of the BMOHCNewKernel launches (no reference counterpart): jacobi_mode
  * 0 = the reference's fixed sweeps (default), 1 = Jacobi to relative residual
  * tol_rel checked every check_every sweeps, capped at max_sweeps; warm_start 0
