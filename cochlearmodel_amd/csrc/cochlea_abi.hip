@@ -179,6 +179,25 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
   if (order_override) a.order = order_override;
   a.use_queue = persistent ? 1 : 0;
   a.queue = nullptr;
+  const bool trial = sections_per_lane > 0;   // the autotuner's: launched as asked
+  if (!trial) sections_per_lane = g_bm.sections_per_lane;
+  if (sections_per_lane <= 0) {
+    // Spread a block over four waves where each CU has at most one: its SIMDs
+    // would run one wave or none.  Only the fixed sweeps gain (one exchange
+    // between waves per pass; solving to a tolerance has one per check).
+    // Blocks of 0.2 s of tones, ms for 4 and 2 sections per lane: 10 blocks 91.5
+    // and 85.8, 250 blocks 101.7 and 89.8, 500 blocks 104.7 and 111.2; to a
+    // tolerance 12 blocks 171 and 264.
+    sections_per_lane = sc.jacobi_mode == 0 && n_items <= device_cus() ? 2 : 4;
+  }
+  // One block per workgroup unless more are asked for, but four where that many
+  // blocks fill the chip's SIMDs once or twice: a workgroup's waves go to
+  // different SIMDs, single waves often to a SIMD that has one already.  ms for
+  // one and four, fixed sweeps: 250 blocks 107 and 110, 500 111 and 107, 1000 141
+  // and 108, 2000 198 and 152, 3000 211 and 206, 9000 529 and 526; to a tolerance
+  // with the extrapolated guess: 1000 172 and 162, 2000 229 and 198, 3000 254 and
+  // 265 (a workgroup's place is free again when its longest block ends).
+  if (!trial && waves_per_block == 1 && n_items > device_cus() && n_items <= 8 * device_cus()) waves_per_block = 4;
   int grid;
   if (persistent) {
     if (g_bm.queue.ensure(1)) return -1;
@@ -202,16 +221,6 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
     rc = cm_launch_bm_ws(&a, &w, device_cus(), stream());
     rc = rc > 0 ? 0 : rc;
   } else {
-    if (sections_per_lane <= 0) sections_per_lane = g_bm.sections_per_lane;
-    if (sections_per_lane <= 0) {
-      // Spread a block over four waves where each CU has at most one: its SIMDs
-      // would run one wave or none.  Only the fixed sweeps gain (one exchange
-      // between waves per pass; solving to a tolerance has one per check).
-      // Blocks of 0.2 s of tones, ms for 4 and 2 sections per lane: 10 blocks 91.5
-      // and 85.8, 250 blocks 101.7 and 89.8, 500 blocks 104.7 and 111.2; to a
-      // tolerance 12 blocks 171 and 264.
-      sections_per_lane = sc.jacobi_mode == 0 && n_items <= device_cus() ? 2 : 4;
-    }
     rc = cm_launch_bm(&a, waves_per_block, unroll > 0 ? unroll : g_bm.jacobi_unroll, sections_per_lane, grid,
                       stream());
   }

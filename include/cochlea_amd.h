@@ -58,7 +58,8 @@ float cudaEventsStopQueryTimer(void *start, void *stop, int condition, const cha
 int cudaEventsDestroy(void *start, void *stop);
 /* Duration of the last timed BM launch (Show_Run_Time & 1, or timed=1). */
 float cm_last_kernel_ms(void);
-/* BM launch shape: waves (time blocks) per workgroup, persistent queue. */
+/* BM launch shape: waves (time blocks) per workgroup (1, the default, leaves the
+ * choice of 1 or 4 to the number of blocks), persistent queue. */
 int cm_set_bm_launch(int waves_per_block, int persistent);
 /* Jacobi sweep loop unroll (1, 2 or 4; default 2) of the following bm_kernel
  * launches (no reference counterpart: the reference's sweep loop is
