@@ -66,6 +66,7 @@ _SIGS = {
     "cm_set_bm_jacobi_unroll": (C.c_int, [C.c_int]),
     "cm_set_bm_sections_per_lane": (C.c_int, [C.c_int]),
     "cm_reset_bm_sections_per_lane": (C.c_int, []),
+    "cm_reset_bm_jacobi_unroll": (C.c_int, []),
     "cm_set_bm_order": (C.c_int, [vp, C.c_int]),
     "cm_set_bm_solver": (C.c_int, [C.c_int, f32, C.c_int, C.c_int, C.c_int]),
     "cm_bm_autotune": (C.c_int, [vp, vp, i64, vp, vp, vp, C.c_int, vp, i64, C.c_int, vp]),

@@ -518,11 +518,24 @@ __device__ __forceinline__ void jacobi_sweep(Lay<N> &L, const float (&Y)[N], con
 #define CM_SWEEP_IN                                                                                     \
   [Y0] "v"(Y[0]), [Y1] "v"(Y[1]), [Y2] "v"(Y[2]), [Y3] "v"(Y[3]), [r0] "v"(r[0]), [r1] "v"(r[1]),       \
       [r2] "v"(r[2]), [r3] "v"(r[3]), [low] "v"(low)
-// J >= 0 sweeps; PAIRS (1 or 2) pairs per trip of the loop.
-template <int PAIRS>
+// J >= 0 sweeps; with TENS ten per trip as long as that many are left, the rest
+// PAIRS (1 or 2) pairs per trip.
+template <int PAIRS, bool TENS>
 __device__ __forceinline__ void sweeps_asm(const float (&Y)[4], const float (&r)[4], float low, float (&p)[4], int J) {
   float a3 = low * p[2] + 0.0f;
   float t0, t1, t2, t3;
+  if (TENS && __builtin_expect(J >= 10, 1)) {
+    int n = J / 10;
+    J -= 10 * n;
+    asm("s_nop 1\n"
+        "1:\n\t" CM_SWEEP_PT CM_SWEEP_TP CM_SWEEP_PT CM_SWEEP_TP CM_SWEEP_PT CM_SWEEP_TP CM_SWEEP_PT CM_SWEEP_TP
+        CM_SWEEP_PT CM_SWEEP_TP "s_sub_i32 %[n], %[n], 1\n\ts_cmp_lg_u32 %[n], 0\n\ts_cbranch_scc1 1b\n\t"
+        : [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [p2] "+&v"(p[2]), [p3] "+&v"(p[3]), [a3] "+&v"(a3), [n] "+&s"(n),
+          [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
+        : CM_SWEEP_IN
+        : "scc");
+    if (__builtin_expect(J == 0, 1)) return;
+  }
   int n = J / (2 * PAIRS);
   if (n > 0) {
     if constexpr (PAIRS == 1)
@@ -547,7 +560,7 @@ __device__ __forceinline__ void sweeps_asm(const float (&Y)[4], const float (&r)
         : [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [p2] "+&v"(p[2]), [p3] "+&v"(p[3]), [a3] "+&v"(a3), [t0] "=&v"(t0),
           [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
         : CM_SWEEP_IN);
-  if (J & 1) {
+  if (TENS ? __builtin_expect(J & 1, 0) : J & 1) {
     asm("s_nop 1\n\t" CM_SWEEP_PT
         : [a3] "+&v"(a3), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
         : [p0] "v"(p[0]), [p1] "v"(p[1]), [p2] "v"(p[2]), [p3] "v"(p[3]), CM_SWEEP_IN);
@@ -578,21 +591,27 @@ __device__ __forceinline__ void sweeps_asm(const float (&Y)[4], const float (&r)
 #define CM_PAIR1 CM_SWEEP1("p0", "t0") CM_SWEEP1("t0", "p0")
 #define CM_LOOP(body) \
   "s_nop 1\n" "1:\n\t" body "s_sub_i32 %[n], %[n], 1\n\ts_cmp_lg_u32 %[n], 0\n\ts_cbranch_scc1 1b\n\t"
-template <int PAIRS, int N>
+template <int PAIRS, bool TENS, int N>
 __device__ __forceinline__ void sweeps_spread(const float (&Y)[N], const float (&r)[N], float low, float (&p)[N],
                                               int J) {
-  int n = J / (2 * PAIRS);
   if constexpr (N == 2) {
     // of the wave's last lane, which has no right neighbour (as a3 above)
     float a1 = low * p[0] + 0.0f, t0, t1;
 #define CM_IO2 [p0] "+&v"(p[0]), [p1] "+&v"(p[1]), [a1] "+&v"(a1), [t0] "=&v"(t0), [t1] "=&v"(t1)
 #define CM_IN2 [Y0] "v"(Y[0]), [Y1] "v"(Y[1]), [r0] "v"(r[0]), [r1] "v"(r[1]), [low] "v"(low)
+    if (TENS && __builtin_expect(J >= 10, 1)) {
+      int n = J / 10;
+      J -= 10 * n;
+      asm(CM_LOOP(CM_PAIR2 CM_PAIR2 CM_PAIR2 CM_PAIR2 CM_PAIR2) : CM_IO2, [n] "+&s"(n) : CM_IN2 : "scc");
+      if (__builtin_expect(J == 0, 1)) return;
+    }
+    int n = J / (2 * PAIRS);
     if (n > 0) {
       if constexpr (PAIRS == 1) asm(CM_LOOP(CM_PAIR2) : CM_IO2, [n] "+&s"(n) : CM_IN2 : "scc");
       else asm(CM_LOOP(CM_PAIR2 CM_PAIR2) : CM_IO2, [n] "+&s"(n) : CM_IN2 : "scc");
     }
     if (PAIRS == 2 && (J & 2)) asm("s_nop 1\n\t" CM_PAIR2 "s_nop 1" : CM_IO2 : CM_IN2);
-    if (J & 1) {
+    if (TENS ? __builtin_expect(J & 1, 0) : J & 1) {
       asm("s_nop 1\n\t" CM_SWEEP2("p0", "p1", "t0", "t1") "s_nop 1" : CM_IO2 : CM_IN2);
       p[0] = t0; p[1] = t1;
     }
@@ -602,12 +621,19 @@ __device__ __forceinline__ void sweeps_spread(const float (&Y)[N], const float (
     float t0;
 #define CM_IO1 [p0] "+&v"(p[0]), [t0] "=&v"(t0)
 #define CM_IN1 [Y0] "v"(Y[0]), [r0] "v"(r[0]), [low] "v"(low)
+    if (TENS && __builtin_expect(J >= 10, 1)) {
+      int n = J / 10;
+      J -= 10 * n;
+      asm(CM_LOOP(CM_PAIR1 CM_PAIR1 CM_PAIR1 CM_PAIR1 CM_PAIR1) : CM_IO1, [n] "+&s"(n) : CM_IN1 : "scc");
+      if (__builtin_expect(J == 0, 1)) return;
+    }
+    int n = J / (2 * PAIRS);
     if (n > 0) {
       if constexpr (PAIRS == 1) asm(CM_LOOP(CM_PAIR1) : CM_IO1, [n] "+&s"(n) : CM_IN1 : "scc");
       else asm(CM_LOOP(CM_PAIR1 CM_PAIR1) : CM_IO1, [n] "+&s"(n) : CM_IN1 : "scc");
     }
     if (PAIRS == 2 && (J & 2)) asm(CM_PAIR1 "s_nop 1" : CM_IO1 : CM_IN1);
-    if (J & 1) {
+    if (TENS ? __builtin_expect(J & 1, 0) : J & 1) {
       asm(CM_SWEEP1("p0", "t0") "s_nop 1" : CM_IO1 : CM_IN1);
       p[0] = t0;
     }
@@ -619,9 +645,12 @@ __device__ __forceinline__ void sweeps_spread(const float (&Y)[N], const float (
 // J is wave-uniform: the count goes to a scalar register.  U (1, 2 or 4) is
 // the unroll of the sweep loop, a launch knob of the autotuner: sweeps come in
 // pairs (U = 2) or two pairs (U = 4) per trip, so the two iterates alternate
-// between register sets; U = 1 copies the iterate back each sweep.  Every U
-// performs the same sweeps in the same order, so results are identical.
-template <int U = 2, int N, class K>
+// between register sets; U = 1 copies the iterate back each sweep.  TENS (U = 4,
+// the fixed sweeps of a slow pass, 20 in the reference method) first takes ten
+// per trip: a taken branch keeps a lone wave waiting for about 26 cycles, as long
+// as five instructions.  Every U performs the same sweeps in the same order, so
+// results are identical.
+template <int U = 2, bool TENS = false, int N, class K>
 __device__ __forceinline__ void jacobi_sweeps(Lay<N> &L, const float (&Y)[N], const K &k, float (&p)[N],
                                               int J) {
   static_assert(U == 1 || U == 2 || U == 4, "unroll 1, 2 or 4");
@@ -631,12 +660,12 @@ __device__ __forceinline__ void jacobi_sweeps(Lay<N> &L, const float (&Y)[N], co
     UNROLL for (int j = 0; j < N; ++j) r[j] = k.rsm[j];
   }
   if constexpr (N == 4 && U != 1) {
-    sweeps_asm<U / 2>(Y, r, k.low, p, J);
+    sweeps_asm<U / 2, TENS>(Y, r, k.low, p, J);
   } else {
     for (;;) {
       const int c = J < Lay<N>::kReach ? J : Lay<N>::kReach;
       if constexpr (U != 1) {
-        sweeps_spread<U / 2>(Y, r, k.low, p, c);
+        sweeps_spread<U / 2, TENS>(Y, r, k.low, p, c);
       } else {
         float q[N];
         for (int i = 0; i < c; ++i) {
@@ -645,7 +674,7 @@ __device__ __forceinline__ void jacobi_sweeps(Lay<N> &L, const float (&Y)[N], co
         }
       }
       J -= c;
-      if (J <= 0) break;
+      if (__builtin_expect(J <= 0, 1)) break;
       L.share(p);
     }
   }
@@ -906,9 +935,25 @@ __device__ __forceinline__ void pass_finish(Lay<N> &L, const K &k, const ItemSca
 // divided out: the float quotient is above 6 where the exact one is above the
 // midpoint 6 + 2^-22 (a tie rounds to 6), and below 0.5 where the exact one is
 // below 0.5 - 2^-26; esum times either bound is exact in FP64.
+// LONE: without branches, which cost a wave that has a SIMD to itself more than
+// the operations they avoid.
+template <bool LONE>
 __device__ __forceinline__ bool step_control(const cm_bm_scalars &sc, const ItemScal &c, float &dt, float emax,
                                              float esum, float fsum) {
   if (sc.decision_mode == 1) { emax = 0.f; esum = 0.f; fsum = 0.f; }
+  if constexpr (LONE) {
+    const double e = esum, q = emax * dt;
+    const bool moved = esum > c.mmspt;
+    const bool above = moved & (q > e * (6.0 + 0x1p-22));       // L > 6
+    const bool below = !moved | (q < e * (0.5 - 0x1p-26));      // L < 0.5
+    const bool again = !above & ((fsum > 0.0f) | !below);
+    const float half = dt * 0.5f, twice = dt * 2.0f;
+    const float less = half < c.dt_min ? c.dt_min : half;
+    const float more = twice > c.dt_max ? c.dt_max : twice;
+    const float other = above ? less : more;
+    dt = again ? dt : other;
+    return again;
+  }
   bool above = false, below = true;   // L > 6, L < 0.5
   if (esum > c.mmspt) {
     const double e = esum, q = emax * dt;
@@ -936,13 +981,13 @@ __device__ __forceinline__ void control_terms(const ItemScal &c, float dt, const
     ez[j] = ey[j] - fmaxf(c.mtt, v[j] * dt);
   }
 }
-template <int N>
+template <bool LONE = false, int N>
 __device__ __forceinline__ bool pass_control(Lay<N> &L, const cm_bm_scalars &sc, const ItemScal &c, float &dt,
                                              const HalfN<N> &n, const float (&vref)[N], const float (&aref)[N]) {
   float ex[N], ey[N], ez[N], emax, esum, fsum;
   control_terms(c, dt, n.v, n.a, vref, aref, ex, ey, ez);
   L.reduce3(ex, ey, ez, emax, esum, fsum);
-  return step_control(sc, c, dt, emax, esum, fsum);
+  return step_control<LONE>(sc, c, dt, emax, esum, fsum);
 }
 
 // Commit of a step whose passes left side n: counters, sample advance with
@@ -1035,7 +1080,7 @@ __device__ __forceinline__ float extrapolate_guess(Lay<N> &L, const K &k, const 
 
 // The pressure solve of a corrector pass: fixed sweeps, or to the tolerance
 // from the resident pressure.
-template <bool TOL, int U, int N, class K>
+template <bool TOL, int U, bool SLOW = true, int N, class K>
 __device__ __forceinline__ int solve_pass(Lay<N> &L, const cm_bm_scalars &sc, const K &k, const float (&Y)[N],
                                           float (&p)[N], int J_fixed) {
   if constexpr (TOL) {
@@ -1044,7 +1089,7 @@ __device__ __forceinline__ int solve_pass(Lay<N> &L, const cm_bm_scalars &sc, co
     L.sum_sq2(r, Y, rr, yy);
     return jacobi_tol<U>(L, sc, k, Y, yy, p, rr);
   } else {
-    jacobi_sweeps<U>(L, Y, k, p, J_fixed);
+    jacobi_sweeps<U, SLOW && U == 4>(L, Y, k, p, J_fixed);
     L.share(p);
     return J_fixed;
   }
@@ -1053,23 +1098,23 @@ __device__ __forceinline__ int solve_pass(Lay<N> &L, const cm_bm_scalars &sc, co
 // The solve, end and control of a corrector pass.  The fixed sweeps of a spread
 // block leave the owned pressures; these and the control's totals pass in one
 // exchange.
-template <bool TOL, int U, int N>
+template <bool TOL, int U, bool SLOW, int N>
 __device__ __forceinline__ bool correct_end(const BmLaunch &a, Lay<N> &L, const ItemConstN<N> &k, const ItemScal &c,
                                             ItemStateN<N> &s, HalfN<N> &n, const PassTerms<N> &T, const float (&Y)[N],
                                             float sf, const float (&vref)[N], const float (&aref)[N], int J_fixed) {
   if constexpr (N == 4 || TOL) {
-    s.n_sweeps += solve_pass<TOL, U>(L, a.sc, k, Y, s.p, J_fixed);
+    s.n_sweeps += solve_pass<TOL, U, SLOW>(L, a.sc, k, Y, s.p, J_fixed);
     pass_finish(L, k, c, n, s.p, T, sf);
-    return pass_control(L, a.sc, c, s.dt, n, vref, aref);
+    return pass_control<!TOL && U == 4>(L, a.sc, c, s.dt, n, vref, aref);
   } else {
-    jacobi_sweeps<U>(L, Y, k, s.p, J_fixed);
+    jacobi_sweeps<U, SLOW && U == 4>(L, Y, k, s.p, J_fixed);
     s.n_sweeps += J_fixed;
     float acc[N], ex[N], ey[N], ez[N], emax, esum, fsum;
     UNROLL for (int j = 0; j < N; ++j) acc[j] = (s.p[j] + T.G[j]) * k.rmass[j];
     control_terms(c, s.dt, n.v, acc, vref, aref, ex, ey, ez);
     L.reduce3_share(ex, ey, ez, s.p, emax, esum, fsum);
     pass_finish(L, k, c, n, s.p, T, sf);
-    return step_control(a.sc, c, s.dt, emax, esum, fsum);
+    return step_control<U == 4>(a.sc, c, s.dt, emax, esum, fsum);
   }
 }
 
@@ -1110,14 +1155,14 @@ __device__ __forceinline__ void step(const BmLaunch &a, const cm_bm_item &it, La
     UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
     correct(o, n, s.dt);
     pass_rhs<true>(k, c, n, s.Ptm, sf, L, T, Y);
-    another = correct_end<TOL, U>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_slow);
+    another = correct_end<TOL, U, true>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_slow);
     passes = 2;
     if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
     while (another) {
       UNROLL for (int j = 0; j < N; ++j) { vref[j] = n.v[j]; aref[j] = n.a[j]; }
       correct(o, n, s.dt);
       pass_rhs<false>(k, c, n, s.Ptm, sf, L, T, Y);
-      another = correct_end<TOL, U>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_fast);
+      another = correct_end<TOL, U, false>(a, L, k, c, s, n, T, Y, sf, vref, aref, a.sc.j_fast);
       ++passes;
       if (passes >= a.sc.max_passes) { another = false; s.c_fail = 1.f; }
     }

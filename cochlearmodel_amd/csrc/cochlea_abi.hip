@@ -71,7 +71,7 @@ struct BMHolder {
   float last_kernel_ms = 0.f;
   int waves_per_block = 1;
   int persistent = 0;
-  int jacobi_unroll = 2;   // Jacobi sweep loop unroll of bm_kernel launches (cm_set_bm_jacobi_unroll)
+  int jacobi_unroll = 0;   // Jacobi sweep loop unroll of bm_kernel launches (cm_set_bm_jacobi_unroll); 0: by size
   int sections_per_lane = 0;   // block layout of fused-kernel launches (cm_set_bm_sections_per_lane); 0: by size
   // solver options for BMOHCNewKernel launches (cm_set_bm_solver); defaults = reference method
   int jacobi_mode = 0, check_every = 4, max_sweeps = 1000, warm_start = 0;
@@ -198,6 +198,13 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
   // with the extrapolated guess: 1000 172 and 162, 2000 229 and 198, 3000 254 and
   // 265 (a workgroup's place is free again when its longest block ends).
   if (!trial && waves_per_block == 1 && n_items > device_cus() && n_items <= 8 * device_cus()) waves_per_block = 4;
+  // Unroll 4 (ten sweeps a trip, step control without branches) where no SIMD has
+  // more than one wave, so that the waits of taken branches are not filled; its
+  // code is larger and does more, and with tolerance checks every few sweeps it
+  // has no long trips.  Fixed sweeps, ms with 2 and 4: 300 blocks 107 and 97, 500
+  // 107 and 99, 1000 108 and 100, 2000 152 and 153, 6000 380 and 390.
+  if (unroll <= 0) unroll = g_bm.jacobi_unroll;
+  if (unroll <= 0) unroll = sc.jacobi_mode == 0 && n_items <= 4 * device_cus() ? 4 : 2;
   int grid;
   if (persistent) {
     if (g_bm.queue.ensure(1)) return -1;
@@ -221,8 +228,7 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
     rc = cm_launch_bm_ws(&a, &w, device_cus(), stream());
     rc = rc > 0 ? 0 : rc;
   } else {
-    rc = cm_launch_bm(&a, waves_per_block, unroll > 0 ? unroll : g_bm.jacobi_unroll, sections_per_lane, grid,
-                      stream());
+    rc = cm_launch_bm(&a, waves_per_block, unroll, sections_per_lane, grid, stream());
   }
   if (rc) {
     set_error("BM kernel launch failed (%d): %s", rc, hipGetErrorString(hipGetLastError()));
@@ -441,6 +447,11 @@ int cm_set_bm_sections_per_lane(int sections_per_lane) {
     return -3;
   }
   g_bm.sections_per_lane = sections_per_lane;
+  return 0;
+}
+
+int cm_reset_bm_jacobi_unroll(void) {
+  g_bm.jacobi_unroll = 0;
   return 0;
 }
 

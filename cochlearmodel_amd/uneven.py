@@ -96,7 +96,7 @@ class UnevenBatch:
     def clear_order(self):
         """Back to the untuned launch order, Jacobi unroll and section layout."""
         check(lib().cm_set_bm_order(None, 0), "cm_set_bm_order")
-        check(lib().cm_set_bm_jacobi_unroll(2), "cm_set_bm_jacobi_unroll")
+        check(lib().cm_reset_bm_jacobi_unroll(), "cm_reset_bm_jacobi_unroll")
         check(lib().cm_reset_bm_sections_per_lane(), "cm_reset_bm_sections_per_lane")
 
     def run_bm(self, sc, timed: bool = True, waves_per_block: int | None = None):

@@ -61,11 +61,13 @@ float cm_last_kernel_ms(void);
 /* BM launch shape: waves (time blocks) per workgroup (1, the default, leaves the
  * choice of 1 or 4 to the number of blocks), persistent queue. */
 int cm_set_bm_launch(int waves_per_block, int persistent);
-/* Jacobi sweep loop unroll (1, 2 or 4; default 2) of the following bm_kernel
- * launches (no reference counterpart: the reference's sweep loop is
+/* Jacobi sweep loop unroll (1, 2 or 4) of the following bm_kernel launches (no
+ * reference counterpart: the reference's sweep loop is
  * include/cochlea.cuh:13962-13982).  Results are identical for every value;
- * cm_bm_autotune sets the fastest. */
+ * cm_bm_autotune sets the fastest.  Unset, or after cm_reset_: 2, or 4 for a
+ * fixed-sweep launch of at most four blocks per CU. */
 int cm_set_bm_jacobi_unroll(int unroll);
+int cm_reset_bm_jacobi_unroll(void);
 /* Sections per lane (1, 2 or 4) of the following fused BM launches (the learned
  * lockstep kernel keeps 4).  4: one wave64 per time block, 4 sections per lane;
  * 2 or 1: a block over a workgroup of 4 or 8 waves that carry their neighbours'
