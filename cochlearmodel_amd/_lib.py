@@ -151,12 +151,16 @@ _SIGS = {
     "cm_pack_section_params": (C.c_int, [vp]),
     "cm_default_bm_scalars": (C.c_int, [f32, vp]),
     "cm_gemm_bf16": (C.c_int, [C.c_int] * 5 + [vp, C.c_int, vp, C.c_int, vp, C.c_int, vp, f32]),
+    "cm_gemm_bf16_gelu": (C.c_int, [C.c_int] * 3 + [vp, C.c_int, vp, C.c_int, vp, vp, vp, C.c_int]),
+    "cm_gemm_bf16_gelu_back": (C.c_int, [C.c_int] * 3 + [vp, C.c_int, vp, C.c_int, vp, vp, vp, C.c_int]),
     "cm_gelu_fwd": (C.c_int, [vp, vp, vp, i64]),
     "cm_gelu_bwd": (C.c_int, [vp, vp, vp, vp, i64]),
     "cm_to_bf16": (C.c_int, [vp, vp, i64]),
     "cm_colsum": (C.c_int, [vp, vp, C.c_int, C.c_int]),
+    "cm_colsums": (C.c_int, [C.c_int, vp, vp, C.c_int, vp]),
     "cm_mse_grad": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, C.c_int]),
     "cm_adam": (C.c_int, [vp, vp, vp, vp, vp, i64, f32, f32, f32, f32, C.c_int, f32]),
+    "cm_adams": (C.c_int, [C.c_int, vp, vp, vp, vp, vp, vp, vp, f32, f32, f32, f32, C.c_int]),
     "cm_ws_load": (C.c_int, [vp, vp, vp, vp, vp, vp, f32]),
     "cm_ws_set_every": (C.c_int, [C.c_int]),
     "cm_ws_set_group": (C.c_int, [C.c_int]),

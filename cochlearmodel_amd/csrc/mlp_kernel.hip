@@ -24,6 +24,15 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float x) {
 }
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
+// GELU (tanh form) with the solver's tanh: g = 0.5 x (1 + tanh(c (x + 0.044715 x^3))).
+__device__ __forceinline__ float gelu_tanh_arg(float x) { return 0.7978845608f * (x + 0.044715f * x * x * x); }
+__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + tanhf(gelu_tanh_arg(x))); }
+__device__ __forceinline__ float gelu_slope(float x) {
+  const float t = tanhf(gelu_tanh_arg(x));
+  const float dt = (1.0f - t * t) * 0.7978845608f * (1.0f + 3.0f * 0.044715f * x * x);
+  return 0.5f * (1.0f + t) + 0.5f * x * dt;
+}
+
 // A workgroup owns a 64 x TN tile of C and walks K in steps of 128 G: each of its
 // G groups of 4 waves loads 128 of them, and every element of C is one chain of
 // products in the order of k, whatever G is (activations are rounded to BF16
@@ -153,12 +162,17 @@ struct Operand {
   }
 };
 
-template <int TN, int G, bool TA, bool TB>
+// What a product's element becomes: itself, or with the activation of its layer
+// (a pass over C and a launch less: 3.7 and 3.2 us each at 1024 x 512).
+enum class End { plain, gelu, gelu_back };
+
+template <int TN, int G, bool TA, bool TB, End END>
 __global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned N, unsigned K,
                                                             const uint16_t *__restrict__ A, int lda,
                                                             const uint16_t *__restrict__ B, int ldb,
                                                             float *__restrict__ C, int ldc,
-                                                            const float *__restrict__ bias, float beta) {
+                                                            const float *__restrict__ bias, float beta,
+                                                            const float *__restrict__ Z, uint16_t *__restrict__ Cbf) {
   constexpr int kTileWords = (TM + TN) * kRowWords;
   // 16 x 16 tiles of a multiplying wave, and those waves' place in the tile
   constexpr int NI = G == 1 ? 2 : 1, NJ = G == 1 ? TN / 32 : 1, kWavesN = TN / (16 * NJ);
@@ -239,32 +253,58 @@ __global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned
         const unsigned gm = m0 + wm + 16 * i + cm + q, gn = n0 + wn + 16 * j + cn;
         if (gm < M && gn < N) {
           float v = acc[i][j][q];
-          if (bias) v += bias[gn];
-          float *dst = C + (int64_t)gm * ldc + gn;
-          *dst = beta != 0.f ? beta * *dst + v : v;
+          const int64_t at = (int64_t)gm * ldc + gn;
+          if constexpr (END == End::plain) {
+            if (bias) v += bias[gn];
+            C[at] = beta != 0.f ? beta * C[at] + v : v;
+          } else if constexpr (END == End::gelu) {
+            if (bias) v += bias[gn];
+            C[at] = v;
+            Cbf[at] = f32_to_bf16(gelu(v));
+          } else {
+            v *= gelu_slope(Z[at]);
+            C[at] = v;
+            Cbf[at] = f32_to_bf16(v);
+          }
         }
       }
 }
 
-template <int TN, int G>
-void launch_gemm(int transA, int transB, int M, int N, int K, const uint16_t *A, int lda, const uint16_t *B, int ldb,
-                 float *C, int ldc, const float *bias, float beta) {
-  auto kernel = transA ? (transB ? gemm_bf16_kernel<TN, G, true, true> : gemm_bf16_kernel<TN, G, true, false>)
-                       : (transB ? gemm_bf16_kernel<TN, G, false, true> : gemm_bf16_kernel<TN, G, false, false>);
-  const unsigned cols = ((unsigned)N + TN - 1) / TN, rows = ((unsigned)M + TM - 1) / TM;
-  hipLaunchKernelGGL(kernel, dim3(cols, rows), dim3(256 * G), 0, stream(), M, N, K, A, lda, B, ldb, C, ldc, bias, beta);
+struct GemmCall {
+  int M, N, K;
+  const void *A;
+  int lda;
+  const void *B;
+  int ldb;
+  float *C;
+  int ldc;
+  const float *bias;
+  float beta;
+  const float *Z;
+  void *Cbf;
+};
+template <int TN, int G, bool TA, bool TB, End END>
+void launch_tiles(const GemmCall &a) {
+  const unsigned cols = ((unsigned)a.N + TN - 1) / TN, rows = ((unsigned)a.M + TM - 1) / TM;
+  hipLaunchKernelGGL((gemm_bf16_kernel<TN, G, TA, TB, END>), dim3(cols, rows), dim3(256 * G), 0, stream(), a.M, a.N,
+                     a.K, (const uint16_t *)a.A, a.lda, (const uint16_t *)a.B, a.ldb, a.C, a.ldc, a.bias, a.beta, a.Z,
+                     (uint16_t *)a.Cbf);
 }
-
-// GELU (tanh form) with the solver's tanh: g = 0.5 x (1 + tanh(c (x + 0.044715 x^3))).
-__device__ __forceinline__ float gelu_tanh_arg(float x) { return 0.7978845608f * (x + 0.044715f * x * x * x); }
-
+template <bool TA, bool TB, End END = End::plain>
+int launch_gemm(const GemmCall &a) {
+  const int64_t tiles = (((int64_t)a.M + TM - 1) / TM) * (((int64_t)a.N + 31) / 32);
+  if (tiles <= device_cus())
+    launch_tiles<32, 4, TA, TB, END>(a);
+  else
+    launch_tiles<64, 1, TA, TB, END>(a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
 
 __global__ void gelu_fwd_kernel(const float *__restrict__ Z, uint16_t *__restrict__ Gbf, float *__restrict__ Gf,
                                 int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float x = Z[i];
-  const float g = 0.5f * x * (1.0f + tanhf(gelu_tanh_arg(x)));
+  const float g = gelu(Z[i]);
   if (Gbf) Gbf[i] = f32_to_bf16(g);
   if (Gf) Gf[i] = g;
 }
@@ -274,10 +314,7 @@ __global__ void gelu_bwd_kernel(const float *__restrict__ dG, const float *__res
                                 float *__restrict__ dZf, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const float x = Z[i];
-  const float t = tanhf(gelu_tanh_arg(x));
-  const float dt = (1.0f - t * t) * 0.7978845608f * (1.0f + 3.0f * 0.044715f * x * x);
-  const float d = dG[i] * (0.5f * (1.0f + t) + 0.5f * x * dt);
+  const float d = dG[i] * gelu_slope(Z[i]);
   if (dZbf) dZbf[i] = f32_to_bf16(d);
   if (dZf) dZf[i] = d;
 }
@@ -287,26 +324,36 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
   if (i < n) y[i] = f32_to_bf16(x[i]);
 }
 
-// column sums of dZ [M x N] -> db [N] (bias gradient).  A workgroup takes 32
-// columns with 32 threads each, which add every 32nd row; their sums are then
-// added in order.  1024 x 512: 235 us with one thread per column -> 3.9 us.
-constexpr int kSumCols = 32, kSumRows = 32;
-__global__ __launch_bounds__(kSumCols * kSumRows) void colsum_kernel(const float *__restrict__ dZ,
-                                                                     float *__restrict__ db, int M, int N) {
+// column sums of dZ [M x N] -> db [N] (bias gradients), up to kMany matrices of
+// M rows in one launch.  A workgroup takes 32 columns with 32 threads each, which
+// add every 32nd row; their sums are then added in order.  1024 x 512: 235 us
+// with one thread per column -> 3.9 us, 1024 x (512, 512, 256) 4.5 us.
+constexpr int kMany = 8, kSumCols = 32, kSumRows = 32;
+struct ColSums {
+  const float *dZ[kMany];
+  float *db[kMany];
+  int N[kMany], first[kMany];   // columns; first group of 32
+};
+__global__ __launch_bounds__(kSumCols * kSumRows) void colsum_kernel(ColSums a, int n, int M, int groups) {
   __shared__ float part[kSumRows][kSumCols + 1];
   const int c = threadIdx.x % kSumCols, r = threadIdx.x / kSumCols;
-  for (int64_t n0 = (int64_t)blockIdx.x * kSumCols; n0 < N; n0 += (int64_t)gridDim.x * kSumCols) {
-    const int64_t n = n0 + c;
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    int k = 0;
+    for (int i = 1; i < n; ++i)
+      if (g >= a.first[i]) k = i;
+    const float *__restrict__ dZ = a.dZ[k];
+    const int N = a.N[k];
+    const int64_t col = (int64_t)(g - a.first[k]) * kSumCols + c;
     float s = 0.f;
-    if (n < N) {
+    if (col < N) {
 #pragma unroll 8
-      for (int m = r; m < M; m += kSumRows) s += dZ[(int64_t)m * N + n];
+      for (int m = r; m < M; m += kSumRows) s += dZ[(int64_t)m * N + col];
     }
     part[r][c] = s;
     __syncthreads();
-    if (r == 0 && n < N) {
-      for (int k = 1; k < kSumRows; ++k) s += part[k][c];
-      db[n] = s;
+    if (r == 0 && col < N) {
+      for (int i = 1; i < kSumRows; ++i) s += part[i][c];
+      a.db[k][col] = s;
     }
     __syncthreads();
   }
@@ -335,21 +382,34 @@ __global__ void mse_grad_kernel(const float *__restrict__ Y, const float *__rest
   if (threadIdx.x == 0) row_loss[m] = sh[0];
 }
 
-// Adam on FP32 master weights; refreshes the BF16 copy.
-__global__ void adam_kernel(float *__restrict__ w, uint16_t *__restrict__ wbf, const float *__restrict__ g,
-                            float *__restrict__ m1, float *__restrict__ m2, int64_t n, float lr, float b1, float b2,
-                            float eps, float bc1, float bc2, float wd) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i] + wd * w[i];
-  const float a = b1 * m1[i] + (1.f - b1) * gi;
-  const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
-  m1[i] = a;
-  m2[i] = b;
-  const float upd = lr * (a / bc1) / (sqrtf(b / bc2) + eps);
+// Adam on FP32 master weights; refreshes the BF16 copy.  Up to kMany arrays in one
+// launch, each from its own block on: memory bound, and six arrays of a network
+// one after another ran into each launch's latency (16 -> 7.7 us).
+struct AdamSet {
+  float *w[kMany], *m1[kMany], *m2[kMany];
+  uint16_t *wbf[kMany];
+  const float *g[kMany];
+  int64_t n[kMany];
+  float wd[kMany];
+  unsigned first[kMany];
+};
+__global__ __launch_bounds__(256) void adam_kernel(AdamSet a, int count, float lr, float b1, float b2, float eps,
+                                                   float bc1, float bc2) {
+  int k = 0;
+  for (int i = 1; i < count; ++i)
+    if (blockIdx.x >= a.first[i]) k = i;
+  const int64_t i = (int64_t)(blockIdx.x - a.first[k]) * 256 + threadIdx.x;
+  if (i >= a.n[k]) return;
+  float *__restrict__ w = a.w[k], *__restrict__ m1 = a.m1[k], *__restrict__ m2 = a.m2[k];
+  const float gi = a.g[k][i] + a.wd[k] * w[i];
+  const float m = b1 * m1[i] + (1.f - b1) * gi;
+  const float v = b2 * m2[i] + (1.f - b2) * gi * gi;
+  m1[i] = m;
+  m2[i] = v;
+  const float upd = lr * (m / bc1) / (sqrtf(v / bc2) + eps);
   const float nw = w[i] - upd;
   w[i] = nw;
-  if (wbf) wbf[i] = f32_to_bf16(nw);
+  if (a.wbf[k]) a.wbf[k][i] = f32_to_bf16(nw);
 }
 
 }  // namespace cm
@@ -364,10 +424,27 @@ int cm_gemm_bf16(int transA, int transB, int M, int N, int K, const void *A, int
     set_error("cm_gemm_bf16: bad arguments");
     return -3;
   }
-  const int64_t tiles = (((int64_t)M + TM - 1) / TM) * (((int64_t)N + 31) / 32);
-  (tiles <= device_cus() ? launch_gemm<32, 4> : launch_gemm<64, 1>)(
-      transA, transB, M, N, K, (const uint16_t *)A, lda, (const uint16_t *)B, ldb, C, ldc, bias, beta);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  const GemmCall a{M, N, K, A, lda, B, ldb, C, ldc, bias, beta, nullptr, nullptr};
+  if (transA) return transB ? launch_gemm<true, true>(a) : launch_gemm<true, false>(a);
+  return transB ? launch_gemm<false, true>(a) : launch_gemm<false, false>(a);
+}
+
+int cm_gemm_bf16_gelu(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias, float *Z,
+                      void *G, int ld) {
+  if (M <= 0 || N <= 0 || K <= 0 || !A || !B || !Z || !G) {
+    set_error("cm_gemm_bf16_gelu: bad arguments");
+    return -3;
+  }
+  return launch_gemm<false, false, End::gelu>(GemmCall{M, N, K, A, lda, B, ldb, Z, ld, bias, 0.f, nullptr, G});
+}
+
+int cm_gemm_bf16_gelu_back(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *Z,
+                           float *dZ, void *dZbf, int ld) {
+  if (M <= 0 || N <= 0 || K <= 0 || !A || !B || !Z || !dZ || !dZbf) {
+    set_error("cm_gemm_bf16_gelu_back: bad arguments");
+    return -3;
+  }
+  return launch_gemm<false, true, End::gelu_back>(GemmCall{M, N, K, A, lda, B, ldb, dZ, ld, nullptr, 0.f, Z, dZbf});
 }
 
 int cm_gelu_fwd(const float *Z, void *Gbf, float *Gf, int64_t n) {
@@ -390,24 +467,75 @@ int cm_to_bf16(const float *x, void *y, int64_t n) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int cm_colsum(const float *dZ, float *db, int M, int N) {
-  const int64_t groups = ((int64_t)N + kSumCols - 1) / kSumCols;
+int cm_colsums(int n, const float *const *dZ, float *const *db, int M, const int *N) {
+  if (n < 1 || n > kMany || !dZ || !db || !N) {
+    set_error("cm_colsums: 1 to %d matrices", kMany);
+    return -3;
+  }
+  ColSums a{};
+  int64_t groups = 0;
+  for (int i = 0; i < n; ++i) {
+    if (N[i] < 0) {
+      set_error("cm_colsums: %d columns", N[i]);
+      return -3;
+    }
+    a.dZ[i] = dZ[i];
+    a.db[i] = db[i];
+    a.N[i] = N[i];
+    a.first[i] = (int)groups;
+    groups += ((int64_t)N[i] + kSumCols - 1) / kSumCols;
+  }
+  if (groups > INT32_MAX) {
+    set_error("cm_colsums: too many columns");
+    return -3;
+  }
   hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)(groups < 65536 ? groups : 65536)), dim3(kSumCols * kSumRows), 0,
-                     stream(), dZ, db, M, N);
+                     stream(), a, n, M, (int)groups);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+
+int cm_colsum(const float *dZ, float *db, int M, int N) { return cm_colsums(1, &dZ, &db, M, &N); }
 
 int cm_mse_grad(const float *Y, const float *T, float *dY, void *dYbf, float *row_loss, int M, int N) {
   hipLaunchKernelGGL(mse_grad_kernel, dim3(M), dim3(256), 0, stream(), Y, T, dY, (uint16_t *)dYbf, row_loss, M, N);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+int cm_adams(int count, float *const *w, void *const *wbf, const float *const *g, float *const *m1, float *const *m2,
+             const int64_t *n, const float *wd, float lr, float b1, float b2, float eps, int step) {
+  if (count < 1 || count > kMany || !w || !wbf || !g || !m1 || !m2 || !n || !wd) {
+    set_error("cm_adams: 1 to %d arrays", kMany);
+    return -3;
+  }
+  AdamSet a{};
+  int64_t blocks = 0;
+  for (int k = 0; k < count; ++k) {
+    if (n[k] < 0) {
+      set_error("cm_adams: negative size");
+      return -3;
+    }
+    a.w[k] = w[k];
+    a.wbf[k] = (uint16_t *)wbf[k];
+    a.g[k] = g[k];
+    a.m1[k] = m1[k];
+    a.m2[k] = m2[k];
+    a.n[k] = n[k];
+    a.wd[k] = wd[k];
+    a.first[k] = (unsigned)blocks;
+    blocks += (n[k] + 255) / 256;
+  }
+  if (blocks > UINT32_MAX) {
+    set_error("cm_adams: too many values");
+    return -3;
+  }
+  const float bc1 = 1.f - powf(b1, (float)step), bc2 = 1.f - powf(b2, (float)step);
+  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)blocks), dim3(256), 0, stream(), a, count, lr, b1, b2, eps, bc1, bc2);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int cm_adam(float *w, void *wbf, const float *g, float *m1, float *m2, int64_t n, float lr, float b1, float b2,
             float eps, int step, float wd) {
-  const float bc1 = 1.f - powf(b1, (float)step), bc2 = 1.f - powf(b2, (float)step);
-  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream(), w, (uint16_t *)wbf, g,
-                     m1, m2, n, lr, b1, b2, eps, bc1, bc2, wd);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return cm_adams(1, &w, &wbf, &g, &m1, &m2, &n, &wd, lr, b1, b2, eps, step);
 }
 
 }  // extern "C"

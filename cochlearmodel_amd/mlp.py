@@ -25,6 +25,11 @@ SIZES = (769, 512, 512, 256)
 N_IN, N_OUT = SIZES[0], SIZES[-1]
 
 
+def _ptrs(tensors):
+    """The tensors' device addresses as a C array."""
+    return (C.c_void_p * len(tensors))(*(None if t is None else t.data_ptr() for t in tensors))
+
+
 class WarmStartMLP:
     def __init__(self, seed: int = 0, device: str = "cuda", params=None):
         import torch
@@ -70,7 +75,6 @@ class WarmStartMLP:
         self.Gbf = [t.empty((B, n), dtype=t.bfloat16, device=d) for n in SIZES[1:-1]]
         self.dY = t.empty((B, SIZES[-1]), dtype=t.float32, device=d)
         self.dYbf = t.empty((B, SIZES[-1]), dtype=t.bfloat16, device=d)
-        self.dG = [t.empty((B, n), dtype=t.float32, device=d) for n in SIZES[1:-1]]
         self.dZ = [t.empty((B, n), dtype=t.float32, device=d) for n in SIZES[1:-1]]
         self.dZbf = [t.empty((B, n), dtype=t.bfloat16, device=d) for n in SIZES[1:-1]]
         self.rowloss = t.empty(B, dtype=t.float32, device=d)
@@ -94,42 +98,42 @@ class WarmStartMLP:
         inp = self.Xbf
         for i in range(3):
             kin, kout = SIZES[i], SIZES[i + 1]
-            check(L.cm_gemm_bf16(0, 0, B, kout, kin, ptr(inp), kin, ptr(self.Wbf[i]), kout, ptr(self.Z[i]), kout,
-                                 ptr(self.b[i]), 0.0), "gemm")
             if i < 2:
-                check(L.cm_gelu_fwd(ptr(self.Z[i]), ptr(self.Gbf[i]), None, B * kout), "gelu")
+                check(L.cm_gemm_bf16_gelu(B, kout, kin, ptr(inp), kin, ptr(self.Wbf[i]), kout, ptr(self.b[i]),
+                                          ptr(self.Z[i]), ptr(self.Gbf[i]), kout), "gemm gelu")
                 inp = self.Gbf[i]
+            else:
+                check(L.cm_gemm_bf16(0, 0, B, kout, kin, ptr(inp), kin, ptr(self.Wbf[i]), kout, ptr(self.Z[i]), kout,
+                                     ptr(self.b[i]), 0.0), "gemm")
         return self.Z[2][:B]
 
     def backward(self, T, B):
         """MSE against T (B, 256); fills gradients, returns the loss."""
         L = self.L
         check(L.cm_mse_grad(ptr(self.Z[2]), ptr(T), ptr(self.dY), ptr(self.dYbf), ptr(self.rowloss), B, N_OUT), "mse")
-        dcur_bf, dcur_f = self.dYbf, self.dY
+        dcur_bf = self.dYbf
         for i in (2, 1, 0):
             kin, kout = SIZES[i], SIZES[i + 1]
             a_in = self.Xbf if i == 0 else self.Gbf[i - 1]
-            # dW = a_in^T dcur, db = colsum(dcur)
+            # dW = a_in^T dcur
             check(L.cm_gemm_bf16(1, 0, kin, kout, B, ptr(a_in), kin, ptr(dcur_bf), kout, ptr(self.gW[i]), kout, None,
                                  0.0), "gemm dW")
-            check(L.cm_colsum(ptr(dcur_f), ptr(self.gb[i]), B, kout), "colsum")
             if i > 0:
-                # dG = dcur W^T ; dZ = dG * gelu'(Z)
-                check(L.cm_gemm_bf16(0, 1, B, kin, kout, ptr(dcur_bf), kout, ptr(self.Wbf[i]), kout,
-                                     ptr(self.dG[i - 1]), kin, None, 0.0), "gemm dG")
-                check(L.cm_gelu_bwd(ptr(self.dG[i - 1]), ptr(self.Z[i - 1]), ptr(self.dZbf[i - 1]),
-                                    ptr(self.dZ[i - 1]), B * kin), "gelu bwd")
-                dcur_bf, dcur_f = self.dZbf[i - 1], self.dZ[i - 1]
+                # dZ = (dcur W^T) * gelu'(Z)
+                check(L.cm_gemm_bf16_gelu_back(B, kin, kout, ptr(dcur_bf), kout, ptr(self.Wbf[i]), kout,
+                                               ptr(self.Z[i - 1]), ptr(self.dZ[i - 1]), ptr(self.dZbf[i - 1]), kin),
+                      "gemm dZ")
+                dcur_bf = self.dZbf[i - 1]
+        # db = colsum(dcur) of every layer
+        check(L.cm_colsums(3, _ptrs(self.dZ + [self.dY]), _ptrs(self.gb), B, (C.c_int * 3)(*SIZES[1:])), "colsums")
         return float(self.rowloss[:B].sum().item()) / (B * N_OUT)
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.t += 1
-        L = self.L
-        for i in range(3):
-            check(L.cm_adam(ptr(self.W[i]), ptr(self.Wbf[i]), ptr(self.gW[i]), ptr(self.mW[i]), ptr(self.vW[i]),
-                            self.W[i].numel(), lr, b1, b2, eps, self.t, wd), "adam")
-            check(L.cm_adam(ptr(self.b[i]), None, ptr(self.gb[i]), ptr(self.mb[i]), ptr(self.vb[i]),
-                            self.b[i].numel(), lr, b1, b2, eps, self.t, 0.0), "adam")
+        sizes = (C.c_int64 * 6)(*(p.numel() for p in self.W + self.b))
+        check(self.L.cm_adams(6, _ptrs(self.W + self.b), _ptrs(self.Wbf + [None] * 3), _ptrs(self.gW + self.gb),
+                              _ptrs(self.mW + self.mb), _ptrs(self.vW + self.vb), sizes,
+                              (C.c_float * 6)(wd, wd, wd, 0.0, 0.0, 0.0), lr, b1, b2, eps, self.t), "adams")
 
     def train(self, X, T, epochs=3, batch=1024, lr=1e-3, seed=0, log=None, decay=0.5):
         """Mini-batch Adam over device tensors X (N, 769), T (N, 256)."""

@@ -368,6 +368,13 @@ int cm_default_bm_scalars(float Fs, cm_bm_scalars *out);
  * the flag is set; BF16 MFMA with FP32 accumulation. */
 int cm_gemm_bf16(int transA, int transB, int M, int N, int K, const void *A, int lda, const void *B, int ldb,
                  float *C, int ldc, const float *bias, float beta);
+/* The same products with their layer's activation: Z = A B + bias and
+ * G = bf16(gelu(Z)); dZ = (A B^T) * gelu'(Z), fp32 and bf16.  All outputs and Z
+ * have leading dimension ld. */
+int cm_gemm_bf16_gelu(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *bias, float *Z,
+                      void *G, int ld);
+int cm_gemm_bf16_gelu_back(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *Z,
+                           float *dZ, void *dZbf, int ld);
 /* G = gelu(Z) (tanh form) to bf16 and/or fp32 (either output may be NULL) */
 int cm_gelu_fwd(const float *Z, void *Gbf, float *Gf, int64_t n);
 /* dZ = dG * gelu'(Z) to bf16 and/or fp32 */
@@ -376,6 +383,8 @@ int cm_gelu_bwd(const float *dG, const float *Z, void *dZbf, float *dZf, int64_t
 int cm_to_bf16(const float *x, void *y, int64_t n);
 /* db[n] = sum over rows of dZ[M x N] */
 int cm_colsum(const float *dZ, float *db, int M, int N);
+/* the same for n (1 to 8) matrices of M rows, N[i] columns each, in one launch */
+int cm_colsums(int n, const float *const *dZ, float *const *db, int M, const int *N);
 /* dY = 2 (Y - T) / (M N) (fp32 and bf16); row_loss[m] = sum_n (Y - T)^2 */
 int cm_mse_grad(const float *Y, const float *T, float *dY, void *dYbf, float *row_loss, int M, int N);
 /* In-solver use (cm_bm_scalars.warm_start = 2, jacobi_mode = 1): lockstep
@@ -411,6 +420,9 @@ int cm_ws_release(void);
  * gradient); refreshes the bf16 copy wbf when it is not NULL */
 int cm_adam(float *w, void *wbf, const float *g, float *m1, float *m2, int64_t n, float lr, float b1, float b2,
             float eps, int step, float wd);
+/* the same for count (1 to 8) arrays in one launch; wbf[k] may be NULL */
+int cm_adams(int count, float *const *w, void *const *wbf, const float *const *g, float *const *m1, float *const *m2,
+             const int64_t *n, const float *wd, float lr, float b1, float b2, float eps, int step);
 
 #ifdef __cplusplus
 }

@@ -66,3 +66,66 @@ def test_colsum_groups(M, N):
     torch.cuda.synchronize()
     tol = M * 2.0 ** -24 * np.abs(x).sum(0, dtype=np.float64) + 1e-30
     assert np.all(np.abs(db.cpu().numpy() - x.sum(0, dtype=np.float64)) <= tol)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 31, 40), (65, 97, 129), (1024, 512, 256), (2048, 1090, 9)])
+def test_products_with_activation_equal_the_separate_kernels(M, N, K):
+    torch = _cuda()
+    from cochlearmodel_amd._lib import check, lib
+    L = lib()
+    print(f"gemm with gelu M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    dev = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
+    new = lambda t: torch.full((M, N), 7.0, dtype=t, device="cuda")
+    p = lambda t: t.data_ptr()
+    A, W, Wt, bias = dev(M, K).bfloat16(), dev(K, N).bfloat16(), dev(N, K).bfloat16(), dev(N)
+    Z, G, Z2, G2 = new(torch.float32), new(torch.bfloat16), new(torch.float32), new(torch.bfloat16)
+    check(L.cm_gemm_bf16(0, 0, M, N, K, p(A), K, p(W), N, p(Z), N, p(bias), 0.0))
+    check(L.cm_gelu_fwd(p(Z), p(G), None, M * N))
+    check(L.cm_gemm_bf16_gelu(M, N, K, p(A), K, p(W), N, p(bias), p(Z2), p(G2), N))
+    d, dZ, dZb, dZ2, dZb2 = (new(t) for t in (torch.float32, torch.float32, torch.bfloat16, torch.float32,
+                                              torch.bfloat16))
+    check(L.cm_gemm_bf16(0, 1, M, N, K, p(A), K, p(Wt), K, p(d), N, None, 0.0))
+    check(L.cm_gelu_bwd(p(d), p(Z), p(dZb), p(dZ), M * N))
+    check(L.cm_gemm_bf16_gelu_back(M, N, K, p(A), K, p(Wt), K, p(Z), p(dZ2), p(dZb2), N))
+    torch.cuda.synchronize()
+    for a, b in ((Z, Z2), (G, G2), (dZ, dZ2), (dZb, dZb2)):
+        assert torch.equal(a, b)
+
+
+def test_many_sums_and_adam_steps_in_one_launch():
+    torch = _cuda()
+    from cochlearmodel_amd._lib import check, lib
+    from cochlearmodel_amd.mlp import _ptrs
+    import ctypes as C
+    L = lib()
+    rng = np.random.default_rng(9)
+    dev = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
+    M, cols = 77, [1, 32, 33, 0, 512, 31, 64, 5]
+    print(f"colsums M={M} N={cols}", flush=True)
+    xs = [dev(M, n) for n in cols]
+    one, many = ([torch.full((n,), 7.0, device="cuda") for n in cols] for _ in range(2))
+    for x, o, n in zip(xs, one, cols):
+        if n:
+            check(L.cm_colsum(x.data_ptr(), o.data_ptr(), M, n))
+    check(L.cm_colsums(8, _ptrs(xs), _ptrs(many), M, (C.c_int * 8)(*cols)))
+    sizes = [1, 256, 257, 0, 70001]
+    print(f"adams n={sizes}", flush=True)
+    w, g, m, v = ([dev(n).abs() for n in sizes] for _ in range(4))
+    wb = [torch.zeros(n, dtype=torch.bfloat16, device="cuda") if k % 2 else None for k, n in enumerate(sizes)]
+    ref = [[t.clone() for t in s] for s in (w, m, v)]
+    rwb = [None if t is None else t.clone() for t in wb]
+    wd = [0.0, 0.1, 0.2, 0.0, 0.5]
+    for k, n in enumerate(sizes):
+        if n:
+            check(L.cm_adam(ref[0][k].data_ptr(), None if rwb[k] is None else rwb[k].data_ptr(), g[k].data_ptr(),
+                            ref[1][k].data_ptr(), ref[2][k].data_ptr(), n, 1e-2, 0.9, 0.999, 1e-8, 3, wd[k]))
+    check(L.cm_adams(5, _ptrs(w), _ptrs(wb), _ptrs(g), _ptrs(m), _ptrs(v), (C.c_int64 * 5)(*sizes),
+                     (C.c_float * 5)(*wd), 1e-2, 0.9, 0.999, 1e-8, 3))
+    torch.cuda.synchronize()
+    for a, b in [*zip(one, many), *zip(ref[0], w), *zip(ref[1], m), *zip(ref[2], v)]:
+        assert torch.equal(a, b)
+    for a, b in zip(rwb, wb):
+        assert a is None or torch.equal(a, b)
+    assert L.cm_colsums(9, _ptrs(xs), _ptrs(many), M, (C.c_int * 8)(*cols)) == -3
+    assert L.cm_adams(0, None, None, None, None, None, None, None, 0.0, 0.0, 0.0, 0.0, 1) == -3
