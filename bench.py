@@ -86,46 +86,46 @@ TONE_ORDER = {"learned_tol": "high", "learned_tol_every2": "high", "learned_tol_
 MLP_FLOP_PER_STEP = 2.0 * (769 * 512 + 512 * 512 + 512 * 256)   # forward, one block-step
 # HBM bytes per launch on the 256-tone batch from rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (KiB per dispatch), scaled by what the counters read for a 1 GiB
-# device copy (FETCH x 2.0, WRITE x 1.0); profiles/pmc_traffic_c2.md
+# device copy (FETCH x 2.0, WRITE x 1.0); profiles/counters.md
 MEASURED_HBM_BYTES = {
-    "learned_tol": (12239.25 * 2.0 + 2258200.0) * 1024,
-    "reference_20_2": (6085.375 * 2.0 + 2258260.0) * 1024,
-    "ihc_lambda": (1150991.3125 * 2.0 + 4515840.0 + 2288920.5 * 2.0 + 6773760.0) * 1024,
+    "learned_tol": (12248.6875 * 2.0 + 2258200.0) * 1024,
+    "reference_20_2": (6199.8125 * 2.0 + 2258260.0) * 1024,
+    "ihc_lambda": (1300195.562 * 2.0 + 6776912.625) * 1024,
 }
 PEAK_BF16_TFLOPS = 2500.0    # MI355X dense BF16 MFMA
 # VALU instructions per launch on the 256-tone batch (rocprofv3 --pmc SQ_INSTS_VALU;
-# profiles/pmc_valu_c2_reference.md, profiles/pmc_mix_c2_learned.md) and the issue
+# profiles/counters.md) and the issue
 # capacity they are measured against: a wave64 FP32 VALU instruction holds a SIMD
 # for 4 cycles, 1024 SIMDs at 2.4 GHz
-MEASURED_VALU_INSTS = {"reference_20_2": 1.0995e11, "learned_tol": 1.64154213976e11,
-                       "ihc_lambda": 1.40262e9 + 2.68728e9}   # ac_ds_kernel + dc_lambda_kernel
+MEASURED_VALU_INSTS = {"reference_20_2": 9.746969734e10, "learned_tol": 1.566305881e11,
+                       "ihc_lambda": 1.531922475e9}
 # VALU issue capacity: the rate bm_kernel's own instruction mix reaches at full
-# occupancy (SQ_INSTS_VALU / kernel time on the JND sweep's 48300 blocks,
-# profiles/pmc_valu_c4_reference.md).  The 4-cycle model (1024 SIMDs x 2.4 GHz
+# occupancy (SQ_INSTS_VALU / kernel time of plain tolerance mode on 20480 blocks,
+# profiles/counters.md).  The 4-cycle model (1024 SIMDs x 2.4 GHz
 # / 4 cycles per wave64 FP32 instruction = 6.14e11/s) sits below it, so it is
 # not a ceiling for this mix.
-VALU_ISSUE_PER_S = 7.38e11
-VALU_ISSUE_MODEL = ("measured: bm_kernel at full occupancy issues 7.38e11 VALU instructions/s "
-                    "(profiles/pmc_valu_c4_reference.md); the 4-cycle wave64 model gives 6.14e11/s")
+VALU_ISSUE_PER_S = 7.33e11
+VALU_ISSUE_MODEL = ("measured: bm_kernel at full occupancy issues 7.33e11 VALU instructions/s "
+                    "(profiles/counters.md); the 4-cycle wave64 model gives 6.14e11/s")
 # L2 -> L1 fill of all CUs: 64 B per clock per CU, 256 CUs at 2.4 GHz
 L1_FILL_BYTES_PER_S = 64 * 256 * 2.4e9
 # FP32 without packed-FP32 instructions (the build disables them): one FMA per
 # lane per cycle, half the published vector peak
 PEAK_FP32_UNPACKED_TFLOPS = PEAK_FP32_TFLOPS / 2
 # The same counters on one launch of the held-out set (2048 tones, 20480 blocks,
-# longest block first; profiles/pmc_traffic_c5_learned.md, profiles/pmc_mix_c5_learned.md)
+# longest block first; profiles/counters.md)
 C5_MEASURED = {
     "tones_per_launch": 2048,
-    "hbm_bytes": {"learned_tol": (2918599.625 * 2.0 + 732940369.34375) * 1024,
-                  "ihc_lambda": (9206258.75 * 2.0 + 36126720.0 + 18361109.0625 * 2.0 + 54190080.0) * 1024},
-    "valu_insts": {"learned_tol": 1.230589350574e12, "plain_tol": 1.269936053668e12,
-                   "ihc_lambda": 1.1221170816e10 + 2.1498514912e10},
-    "l2_read_bytes": {"learned_tol": 3.90384312554e11 * 128},
+    "hbm_bytes": {"learned_tol": (40958464.75 * 2.0 + 873560629.3) * 1024,
+                  "ihc_lambda": (10403518.25 * 2.0 + 54215846.38) * 1024},
+    "valu_insts": {"learned_tol": 1.165197976e12, "plain_tol": 1.178144026e12,
+                   "ihc_lambda": 1.225412694e10},
+    "l2_read_bytes": {"learned_tol": 3.970973155e11 * 128},
     "mfma_insts": {"learned_tol": 4.769789056e10},
 }
 # L1<-L2 reads of the learned kernel: TCP_TCC_READ_REQ_sum x 128 B (a 1 GiB copy
-# reads 8.389e6 requests); profiles/pmc_mix_c2_learned.md
-MEASURED_L2_READ_BYTES = {"learned_tol": 6.5295415974e10 * 128}
+# reads 8.389e6 requests); profiles/counters.md
+MEASURED_L2_READ_BYTES = {"learned_tol": 6.529537941e10 * 128}
 
 
 def load_warm_start_model():
@@ -716,8 +716,8 @@ def c5_main(args):
                                            "on a 1 GiB copy); algorithmic: input 72 MB + velocity 18.5 GB")
         if args.variant == "learned_tol":
             out["roofline"]["traffic_note"] += (
-                "; the learned kernel's groups of 16 (4 waves per SIMD, 128 VGPRs) spill 64 B per lane: the "
-                "reloads hit the 4 MB L2 of each XCD (2 MiB of spill slots per XCD), and the spill stores make "
+                "; the learned kernel's groups of 16 (4 waves per SIMD, 128 VGPRs) spill 96 B per lane: the "
+                "reloads hit the 4 MB L2 of each XCD (3 MiB of spill slots per XCD), and the spill stores make "
                 "almost all of the write traffic")
     if args.variant in M["valu_insts"]:
         out["roofline"]["valu_issue"] = {
@@ -864,7 +864,7 @@ def c2_main(args):
                                "256 sections, Decouple_Filter=10, 2560 time blocks, input synthesis + BM + "
                                "IHC/lambda per step; BM solver: " + desc[args.variant],
                    "variant": args.variant, "signals": work.n, "time_blocks": work.TB, "rows": work.rows,
-                   "sections_per_lane": 4 if args.variant == "learned_tol" else args.sections_per_lane},
+                   "sections_per_lane": 4 if args.variant == "learned_tol" else args.sections_per_lane or 4},
         "jacobi_iters_per_step": sweeps / steps, "passes_per_step": passes / steps,
         "committed_steps": steps, "signals_per_s": work.n / (ms_per_step * 1e-3),
         "bm_ms": bm_avg, "ihc_lambda_ms": float(np.mean(ihc_ms)), "input_ms": float(np.mean(in_ms)),
@@ -971,8 +971,9 @@ def main():
     ap.add_argument("--c3-signals", type=int, default=1024)
     ap.add_argument("--c4-intervals", type=int, default=8, help="calculated intervals checked on the CPU")
     ap.add_argument("--no-graph", action="store_true", help="c4: launch the post-BM stages eagerly")
-    ap.add_argument("--sections-per-lane", type=int, default=4, choices=(4, 2, 1),
-                    help="block layout of the fused BM kernels (the learned kernel keeps 4)")
+    ap.add_argument("--sections-per-lane", type=int, default=None, choices=(4, 2, 1),
+                    help="block layout of the fused BM kernels (default: by the launch's size; the learned kernel "
+                         "keeps 4)")
     ap.add_argument("--copy-probe-mb", type=int, default=0,
                     help="first run one device-to-device copy of this many MiB (calibrates HBM byte counters)")
     args = ap.parse_args()
@@ -991,7 +992,8 @@ def main():
         torch.cuda.synchronize()
         del src, dst
     from cochlearmodel_amd import _lib
-    _lib.check(_lib.lib().cm_set_bm_sections_per_lane(args.sections_per_lane), "cm_set_bm_sections_per_lane")
+    if args.sections_per_lane is not None:
+        _lib.check(_lib.lib().cm_set_bm_sections_per_lane(args.sections_per_lane), "cm_set_bm_sections_per_lane")
     if args.workload == "c1":
         return c1_main(args)
     if args.workload == "c3":
