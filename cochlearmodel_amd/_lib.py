@@ -153,6 +153,7 @@ _SIGS = {
     "cm_gemm_bf16": (C.c_int, [C.c_int] * 5 + [vp, C.c_int, vp, C.c_int, vp, C.c_int, vp, f32]),
     "cm_gemm_bf16_gelu": (C.c_int, [C.c_int] * 3 + [vp, C.c_int, vp, C.c_int, vp, vp, vp, C.c_int]),
     "cm_gemm_bf16_gelu_back": (C.c_int, [C.c_int] * 3 + [vp, C.c_int, vp, C.c_int, vp, vp, vp, C.c_int]),
+    "cm_weight_grads": (C.c_int, [C.c_int, C.c_int, vp, vp, vp, vp, vp]),
     "cm_gelu_fwd": (C.c_int, [vp, vp, vp, i64]),
     "cm_gelu_bwd": (C.c_int, [vp, vp, vp, vp, i64]),
     "cm_to_bf16": (C.c_int, [vp, vp, i64]),

@@ -166,13 +166,34 @@ struct Operand {
 // (a pass over C and a launch less: 3.7 and 3.2 us each at 1024 x 512).
 enum class End { plain, gelu, gelu_back };
 
+struct GemmArgs {
+  unsigned M, N, K;
+  const uint16_t *A;
+  int lda;
+  const uint16_t *B;
+  int ldb;
+  float *C;
+  int ldc;
+  const float *bias;
+  float beta;
+  const float *Z;
+  uint16_t *Cbf;
+};
+// Place of workgroup blk in the order of tiles that gives each XCD neighbours.
+__device__ __forceinline__ unsigned xcd_order(unsigned blk, unsigned tiles) {
+  const unsigned xcd = blk & 7, rem = tiles & 7;
+  return xcd * (tiles >> 3) + (xcd < rem ? xcd : rem) + (blk >> 3);
+}
+
 template <int TN, int G, bool TA, bool TB, End END>
-__global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned N, unsigned K,
-                                                            const uint16_t *__restrict__ A, int lda,
-                                                            const uint16_t *__restrict__ B, int ldb,
-                                                            float *__restrict__ C, int ldc,
-                                                            const float *__restrict__ bias, float beta,
-                                                            const float *__restrict__ Z, uint16_t *__restrict__ Cbf) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsigned n0) {
+  const unsigned M = g_.M, N = g_.N, K = g_.K;
+  const uint16_t *__restrict__ A = g_.A, *__restrict__ B = g_.B;
+  const int lda = g_.lda, ldb = g_.ldb, ldc = g_.ldc;
+  float *__restrict__ C = g_.C;
+  const float *__restrict__ bias = g_.bias, *__restrict__ Z = g_.Z;
+  const float beta = g_.beta;
+  uint16_t *__restrict__ Cbf = g_.Cbf;
   constexpr int kTileWords = (TM + TN) * kRowWords;
   // 16 x 16 tiles of a multiplying wave, and those waves' place in the tile
   constexpr int NI = G == 1 ? 2 : 1, NJ = G == 1 ? TN / 32 : 1, kWavesN = TN / (16 * NJ);
@@ -181,10 +202,6 @@ __global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned
   __shared__ __align__(16) uint32_t lds[G * kTileWords];
   const int tid = threadIdx.x & 255, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = wave >> 2;
-  const unsigned blk = blockIdx.y * gridDim.x + blockIdx.x, tiles = gridDim.x * gridDim.y;
-  const unsigned xcd = blk & 7, rem = tiles & 7;
-  const unsigned tile = xcd * (tiles >> 3) + (xcd < rem ? xcd : rem) + (blk >> 3);
-  const unsigned m0 = tile / gridDim.x * TM, n0 = tile % gridDim.x * TN;
   const int wm = wave / kWavesN * 16 * NI, wn = wave % kWavesN * 16 * NJ;
   Operand<TM, !TA> a{A, lda, M, K, m0, {}, {}};
   Operand<TN, TB> b{B, ldb, N, K, n0, {}, {}};
@@ -270,28 +287,37 @@ __global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(unsigned M, unsigned
       }
 }
 
-struct GemmCall {
-  int M, N, K;
-  const void *A;
-  int lda;
-  const void *B;
-  int ldb;
-  float *C;
-  int ldc;
-  const float *bias;
-  float beta;
-  const float *Z;
-  void *Cbf;
-};
 template <int TN, int G, bool TA, bool TB, End END>
-void launch_tiles(const GemmCall &a) {
-  const unsigned cols = ((unsigned)a.N + TN - 1) / TN, rows = ((unsigned)a.M + TM - 1) / TM;
-  hipLaunchKernelGGL((gemm_bf16_kernel<TN, G, TA, TB, END>), dim3(cols, rows), dim3(256 * G), 0, stream(), a.M, a.N,
-                     a.K, (const uint16_t *)a.A, a.lda, (const uint16_t *)a.B, a.ldb, a.C, a.ldc, a.bias, a.beta, a.Z,
-                     (uint16_t *)a.Cbf);
+__global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(GemmArgs a) {
+  const unsigned tile = xcd_order(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  gemm_tile<TN, G, TA, TB, END>(a, tile / gridDim.x * TM, tile % gridDim.x * TN);
+}
+
+// Up to kMany products A^T B (weight gradients) in one launch: none of a network's
+// fills the chip, together they do.  At batch 1024 three launches took 20 us,
+// this 11.
+constexpr int kMany = 8;
+struct GemmSet {
+  GemmArgs a[kMany];
+  unsigned first[kMany], cols[kMany];   // a product's first tile, and its tiles per row
+};
+template <int G>
+__global__ __launch_bounds__(256 * G) void gemm_many_kernel(GemmSet s, int n) {
+  const unsigned tile = xcd_order(blockIdx.x, gridDim.x);
+  int k = 0;
+  for (int i = 1; i < n; ++i)
+    if (tile >= s.first[i]) k = i;
+  const unsigned t = tile - s.first[k], cols = s.cols[k];
+  gemm_tile<64, G, true, false, End::plain>(s.a[k], t / cols * TM, t % cols * 64);
+}
+
+template <int TN, int G, bool TA, bool TB, End END>
+void launch_tiles(const GemmArgs &a) {
+  const unsigned cols = (a.N + TN - 1) / TN, rows = (a.M + TM - 1) / TM;
+  hipLaunchKernelGGL((gemm_bf16_kernel<TN, G, TA, TB, END>), dim3(cols, rows), dim3(256 * G), 0, stream(), a);
 }
 template <bool TA, bool TB, End END = End::plain>
-int launch_gemm(const GemmCall &a) {
+int launch_gemm(const GemmArgs &a) {
   const int64_t tiles = (((int64_t)a.M + TM - 1) / TM) * (((int64_t)a.N + 31) / 32);
   if (tiles <= device_cus())
     launch_tiles<32, 4, TA, TB, END>(a);
@@ -327,8 +353,8 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
 // column sums of dZ [M x N] -> db [N] (bias gradients), up to kMany matrices of
 // M rows in one launch.  A workgroup takes 32 columns with 32 threads each, which
 // add every 32nd row; their sums are then added in order.  1024 x 512: 235 us
-// with one thread per column -> 3.9 us, 1024 x (512, 512, 256) 4.5 us.
-constexpr int kMany = 8, kSumCols = 32, kSumRows = 32;
+// with one thread per column -> 3.9 us, 1024 x (512, 512, 256, 1) 4.5 us.
+constexpr int kSumCols = 32, kSumRows = 32;
 struct ColSums {
   const float *dZ[kMany];
   float *db[kMany];
@@ -424,7 +450,8 @@ int cm_gemm_bf16(int transA, int transB, int M, int N, int K, const void *A, int
     set_error("cm_gemm_bf16: bad arguments");
     return -3;
   }
-  const GemmCall a{M, N, K, A, lda, B, ldb, C, ldc, bias, beta, nullptr, nullptr};
+  const GemmArgs a{(unsigned)M, (unsigned)N, (unsigned)K, (const uint16_t *)A, lda, (const uint16_t *)B, ldb,
+                   C, ldc, bias, beta, nullptr, nullptr};
   if (transA) return transB ? launch_gemm<true, true>(a) : launch_gemm<true, false>(a);
   return transB ? launch_gemm<false, true>(a) : launch_gemm<false, false>(a);
 }
@@ -435,7 +462,9 @@ int cm_gemm_bf16_gelu(int M, int N, int K, const void *A, int lda, const void *B
     set_error("cm_gemm_bf16_gelu: bad arguments");
     return -3;
   }
-  return launch_gemm<false, false, End::gelu>(GemmCall{M, N, K, A, lda, B, ldb, Z, ld, bias, 0.f, nullptr, G});
+  return launch_gemm<false, false, End::gelu>(
+      GemmArgs{(unsigned)M, (unsigned)N, (unsigned)K, (const uint16_t *)A, lda, (const uint16_t *)B, ldb, Z, ld, bias,
+               0.f, nullptr, (uint16_t *)G});
 }
 
 int cm_gemm_bf16_gelu_back(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *Z,
@@ -444,7 +473,41 @@ int cm_gemm_bf16_gelu_back(int M, int N, int K, const void *A, int lda, const vo
     set_error("cm_gemm_bf16_gelu_back: bad arguments");
     return -3;
   }
-  return launch_gemm<false, true, End::gelu_back>(GemmCall{M, N, K, A, lda, B, ldb, dZ, ld, nullptr, 0.f, Z, dZbf});
+  return launch_gemm<false, true, End::gelu_back>(
+      GemmArgs{(unsigned)M, (unsigned)N, (unsigned)K, (const uint16_t *)A, lda, (const uint16_t *)B, ldb, dZ, ld,
+               nullptr, 0.f, Z, (uint16_t *)dZbf});
+}
+
+int cm_weight_grads(int n, int K, const int *M, const int *N, const void *const *A, const void *const *B,
+                    float *const *C) {
+  if (n < 1 || n > kMany || K <= 0 || !M || !N || !A || !B || !C) {
+    set_error("cm_weight_grads: 1 to %d products", kMany);
+    return -3;
+  }
+  GemmSet s{};
+  int64_t tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    if (M[i] <= 0 || N[i] <= 0 || !A[i] || !B[i] || !C[i]) {
+      set_error("cm_weight_grads: bad product %d", i);
+      return -3;
+    }
+    s.a[i] = GemmArgs{(unsigned)M[i], (unsigned)N[i], (unsigned)K, (const uint16_t *)A[i], M[i],
+                      (const uint16_t *)B[i], N[i], C[i], N[i], nullptr, 0.f, nullptr, nullptr};
+    s.first[i] = (unsigned)tiles;
+    s.cols[i] = ((unsigned)N[i] + 63) / 64;
+    tiles += (((int64_t)M[i] + TM - 1) / TM) * s.cols[i];
+  }
+  if (tiles > INT32_MAX) {
+    set_error("cm_weight_grads: too many tiles");
+    return -3;
+  }
+  // sixteen waves per tile while every tile has a CU of its own, as for one product:
+  // 200 tiles of K = 1024 11.0 us (four waves 15.8), 296 tiles 18.7 (18.5), 384 16.3 (13.4)
+  if (tiles <= device_cus())
+    hipLaunchKernelGGL((gemm_many_kernel<4>), dim3((unsigned)tiles), dim3(1024), 0, stream(), s, n);
+  else
+    hipLaunchKernelGGL((gemm_many_kernel<1>), dim3((unsigned)tiles), dim3(256), 0, stream(), s, n);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int cm_gelu_fwd(const float *Z, void *Gbf, float *Gf, int64_t n) {

@@ -78,6 +78,7 @@ class WarmStartMLP:
         self.dZ = [t.empty((B, n), dtype=t.float32, device=d) for n in SIZES[1:-1]]
         self.dZbf = [t.empty((B, n), dtype=t.bfloat16, device=d) for n in SIZES[1:-1]]
         self.rowloss = t.empty(B, dtype=t.float32, device=d)
+        self.loss = t.empty(1, dtype=t.float32, device=d)
         self.gW = [t.empty_like(w) for w in self.W]
         self.gb = [t.empty_like(b) for b in self.b]
 
@@ -111,22 +112,18 @@ class WarmStartMLP:
         """MSE against T (B, 256); fills gradients, returns the loss."""
         L = self.L
         check(L.cm_mse_grad(ptr(self.Z[2]), ptr(T), ptr(self.dY), ptr(self.dYbf), ptr(self.rowloss), B, N_OUT), "mse")
-        dcur_bf = self.dYbf
-        for i in (2, 1, 0):
+        dbf = self.dZbf + [self.dYbf]
+        for i in (2, 1):
+            # dZ = (d W^T) * gelu'(Z) of the layer below
             kin, kout = SIZES[i], SIZES[i + 1]
-            a_in = self.Xbf if i == 0 else self.Gbf[i - 1]
-            # dW = a_in^T dcur
-            check(L.cm_gemm_bf16(1, 0, kin, kout, B, ptr(a_in), kin, ptr(dcur_bf), kout, ptr(self.gW[i]), kout, None,
-                                 0.0), "gemm dW")
-            if i > 0:
-                # dZ = (dcur W^T) * gelu'(Z)
-                check(L.cm_gemm_bf16_gelu_back(B, kin, kout, ptr(dcur_bf), kout, ptr(self.Wbf[i]), kout,
-                                               ptr(self.Z[i - 1]), ptr(self.dZ[i - 1]), ptr(self.dZbf[i - 1]), kin),
-                      "gemm dZ")
-                dcur_bf = self.dZbf[i - 1]
-        # db = colsum(dcur) of every layer
-        check(L.cm_colsums(3, _ptrs(self.dZ + [self.dY]), _ptrs(self.gb), B, (C.c_int * 3)(*SIZES[1:])), "colsums")
-        return float(self.rowloss[:B].sum().item()) / (B * N_OUT)
+            check(L.cm_gemm_bf16_gelu_back(B, kin, kout, ptr(dbf[i]), kout, ptr(self.Wbf[i]), kout,
+                                           ptr(self.Z[i - 1]), ptr(self.dZ[i - 1]), ptr(dbf[i - 1]), kin), "gemm dZ")
+        # dW = input^T d, db = colsum(d) of every layer, and the sum of the row losses
+        check(L.cm_weight_grads(3, B, (C.c_int * 3)(*SIZES[:-1]), (C.c_int * 3)(*SIZES[1:]),
+                                _ptrs([self.Xbf] + self.Gbf), _ptrs(dbf), _ptrs(self.gW)), "weight grads")
+        check(L.cm_colsums(4, _ptrs(self.dZ + [self.dY, self.rowloss]), _ptrs(self.gb + [self.loss]), B,
+                           (C.c_int * 4)(*SIZES[1:], 1)), "colsums")
+        return self.loss.item() / (B * N_OUT)
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.t += 1

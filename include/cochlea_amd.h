@@ -375,6 +375,10 @@ int cm_gemm_bf16_gelu(int M, int N, int K, const void *A, int lda, const void *B
                       void *G, int ld);
 int cm_gemm_bf16_gelu_back(int M, int N, int K, const void *A, int lda, const void *B, int ldb, const float *Z,
                            float *dZ, void *dZbf, int ld);
+/* n (1 to 8) weight gradients in one launch: C[i] (M[i] x N[i]) = A[i]^T B[i], A[i]
+ * K x M[i] and B[i] K x N[i] bf16, all dense */
+int cm_weight_grads(int n, int K, const int *M, const int *N, const void *const *A, const void *const *B,
+                    float *const *C);
 /* G = gelu(Z) (tanh form) to bf16 and/or fp32 (either output may be NULL) */
 int cm_gelu_fwd(const float *Z, void *Gbf, float *Gf, int64_t n);
 /* dZ = dG * gelu'(Z) to bf16 and/or fp32 */

@@ -129,3 +129,28 @@ def test_many_sums_and_adam_steps_in_one_launch():
         assert a is None or torch.equal(a, b)
     assert L.cm_colsums(9, _ptrs(xs), _ptrs(many), M, (C.c_int * 8)(*cols)) == -3
     assert L.cm_adams(0, None, None, None, None, None, None, None, 0.0, 0.0, 0.0, 0.0, 1) == -3
+
+
+@pytest.mark.parametrize("K,dims", [(1, [(1, 1)]), (129, [(65, 33), (1, 70), (64, 64), (130, 5)]),
+                                    (1024, [(769, 512), (512, 512), (512, 256)]),
+                                    (40, [(1100, 1030), (3, 2), (64, 1025)])])
+def test_weight_gradients_in_one_launch_equal_single_products(K, dims):
+    torch = _cuda()
+    from cochlearmodel_amd._lib import check, lib
+    from cochlearmodel_amd.mlp import _ptrs
+    import ctypes as C
+    L = lib()
+    print(f"weight grads K={K} {dims}", flush=True)
+    rng = np.random.default_rng(K)
+    dev = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda().bfloat16()
+    A, B = [dev(K, m) for m, _ in dims], [dev(K, n) for _, n in dims]
+    one, many = ([torch.full((m, n), 7.0, device="cuda") for m, n in dims] for _ in range(2))
+    for a, b, c, (m, n) in zip(A, B, one, dims):
+        check(L.cm_gemm_bf16(1, 0, m, n, K, a.data_ptr(), m, b.data_ptr(), n, c.data_ptr(), n, None, 0.0))
+    num = C.c_int * len(dims)
+    check(L.cm_weight_grads(len(dims), K, num(*(m for m, _ in dims)), num(*(n for _, n in dims)), _ptrs(A), _ptrs(B),
+                            _ptrs(many)))
+    torch.cuda.synchronize()
+    for a, b in zip(one, many):
+        assert torch.equal(a, b)
+    assert L.cm_weight_grads(0, K, None, None, None, None, None) == -3
