@@ -70,3 +70,36 @@ def test_tolerance(every, most, guess):
     sc = solver.default_scalars(FS)
     sc.jacobi_mode, sc.tol_rel, sc.check_every, sc.max_sweeps, sc.warm_start = 1, 1e-5, every, most, guess
     _same(torch, sc, f"checks every {every}, at most {most}, warm start {guess}")
+
+
+@pytest.mark.parametrize("n", [250, 263, 1025, 2049])
+@pytest.mark.parametrize("tol", [False, True])
+def test_launch_shapes_chosen_by_size(n, tol):
+    """The shapes that the number of blocks selects (either side of one, four and
+    eight blocks per CU, of 256) against one that is asked for."""
+    torch = _cuda()
+    from cochlearmodel_amd import _lib, solver
+    from cochlearmodel_amd.uneven import UnevenBatch
+    L = _lib.lib()
+    rng = np.random.default_rng(n)
+    sigs = [(0.1 * rng.standard_normal(int(FS * 0.0004 * (1 + k % 3)))).astype(np.float32) for k in range(n)]
+    ub = UnevenBatch(sigs, np.ones((n, 256), np.float32), [8.0] * n, FS, block_s=0.002, overlap_s=0.0005)
+    print(f"case: {ub.TB} blocks, tolerance {tol}", flush=True)
+    sc = solver.default_scalars(FS)
+    if tol:
+        sc.jacobi_mode, sc.tol_rel, sc.check_every, sc.max_sweeps, sc.warm_start = 1, 1e-5, 4, 1000, 1
+    order = np.arange(ub.TB, dtype=np.int32)[::-1].copy()
+    got = []
+    try:
+        for asked in (False, True):
+            if asked:
+                _lib.check(L.cm_set_bm_sections_per_lane(4))
+                _lib.check(L.cm_set_bm_jacobi_unroll(2))
+            _lib.check(L.cm_set_bm_order(_lib.ptr(order), len(order)))
+            ub.d_speeds.fill_(7.0)
+            ub.run_bm(sc, timed=False, waves_per_block=2 if asked else 1)
+            torch.cuda.synchronize()
+            got.append((ub.d_speeds.cpu().numpy().tobytes(), ub.d_stats.cpu().numpy().tobytes()))
+    finally:
+        ub.clear_order()
+    assert got[0] == got[1]
