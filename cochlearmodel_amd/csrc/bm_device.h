@@ -1127,8 +1127,9 @@ __device__ __forceinline__ bool correct_end(const BmLaunch &a, Lay<N> &L, const 
 // (DPP, FP64).  So the step is written for few instructions: per block-step of
 // the reference method 1589 VALU and 122 SALU, where one pass loop for all
 // kinds of pass, a branch per tanh, divided-out step control and copied states
-// took 1793 and 246 (600 tones of 200 ms, 20-90 dB).  5 blocks: 141 -> 111 ms;
-// 610 blocks, extrapolated guess: 183 -> 143 ms; 6000 blocks: 408 -> 380 ms.
+// took 1793 and 246 (600 tones of 200 ms, 20-90 dB).  5 blocks: 141 -> 111 ms (85
+// over four waves each, with ten sweeps a trip); 610 blocks, extrapolated guess:
+// 183 -> 143 ms; 6000 blocks: 408 -> 380 ms.
 template <int N, bool TOL, int WS, int U>
 __device__ __forceinline__ void step(const BmLaunch &a, const cm_bm_item &it, Lay<N> &L, const ItemConstN<N> &k,
                                      const ItemScal &c, ItemStateN<N> &s, const HalfN<N> &o, HalfN<N> &n,

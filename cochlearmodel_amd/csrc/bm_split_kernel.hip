@@ -6,9 +6,9 @@
 // translation unit of its own, so that the one-wave kernels' code object is the
 // same with or without it.
 // Bound: instruction issue of lone waves, as bm_kernel, and the exchanges.  Per
-// step of a 5-block recording (five passes): 4 sections per lane 2177 VALU and
-// 11.6 kcycles, 2 per lane 1274 and 10.9 of which 3.0 wait for the five
-// exchanges, 1 per lane 838 and 10.1 (it wins nowhere else).  Exchanging each
+// step of a 5-block recording (five passes, unroll 4): 4 sections per lane 2195
+// VALU and 11.0 kcycles, 2 per lane 1288 and 10.1 of which 2.7 wait for the five
+// exchanges, 1 per lane 856 and 10.1 of which 3.8 wait.  Exchanging each
 // sweep's boundary pressures instead took 9 to 46 exchanges a step.
 #include <hip/hip_runtime.h>
 
