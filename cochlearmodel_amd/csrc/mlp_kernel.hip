@@ -351,18 +351,30 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
 }
 
 // column sums of dZ [M x N] -> db [N] (bias gradients), up to kMany matrices of
-// M rows in one launch.  A workgroup takes 32 columns with 32 threads each, which
-// add every 32nd row; their sums are then added in order.  1024 x 512: 235 us
-// with one thread per column -> 3.9 us, 1024 x (512, 512, 256, 1) 4.5 us.
-constexpr int kSumCols = 32, kSumRows = 32;
+// M rows in one launch.  Every sum adds its rows in order, one after another from
+// 0: the gradients of a training step, and what Adam makes of them, are then the
+// same whatever the launch looks like (a sum in another order moves the biases by
+// a rounding, and some steps later activations by whole BF16 steps).
+// A workgroup takes 16 columns.  Its 1024 threads load tiles of 512 rows into two
+// LDS buffers in turn, the next tile's loads in flight meanwhile, and 16 lanes of
+// its first wave add a tile's rows, 32 per trip with the next trip's LDS reads in
+// flight, four rows to a read (a column's rows lie next to each other; 4 words of
+// padding spread the columns over the banks).  Rows past the matrix are zeros: a
+// sum that starts at 0 is never -0, so adding them changes nothing.
+// Bound: the chain of one addition per row, about 11 cycles each.  M x (512, 512,
+// 256) in one launch: M = 33 4.3 us, 1024 7.4, 8192 39; one thread per column and
+// nothing in flight took 235 us for 1024 x 512 alone.
+constexpr int kSumCols = 16, kSumRows = 512, kSumThreads = 1024;
+constexpr int kSumLoads = kSumCols * kSumRows / kSumThreads, kSumStride = kSumRows + 4;
 struct ColSums {
   const float *dZ[kMany];
   float *db[kMany];
-  int N[kMany], first[kMany];   // columns; first group of 32
+  int N[kMany], first[kMany];   // columns; first group of kSumCols
 };
-__global__ __launch_bounds__(kSumCols * kSumRows) void colsum_kernel(ColSums a, int n, int M, int groups) {
-  __shared__ float part[kSumRows][kSumCols + 1];
+__global__ __launch_bounds__(kSumThreads) void colsum_kernel(ColSums a, int n, int M, int groups) {
+  __shared__ __align__(16) float tile[2][kSumCols * kSumStride];
   const int c = threadIdx.x % kSumCols, r = threadIdx.x / kSumCols;
+  constexpr int kStep = kSumThreads / kSumCols;   // rows between a thread's loads
   for (int g = blockIdx.x; g < groups; g += gridDim.x) {
     int k = 0;
     for (int i = 1; i < n; ++i)
@@ -370,18 +382,58 @@ __global__ __launch_bounds__(kSumCols * kSumRows) void colsum_kernel(ColSums a, 
     const float *__restrict__ dZ = a.dZ[k];
     const int N = a.N[k];
     const int64_t col = (int64_t)(g - a.first[k]) * kSumCols + c;
-    float s = 0.f;
-    if (col < N) {
-#pragma unroll 8
-      for (int m = r; m < M; m += kSumRows) s += dZ[(int64_t)m * N + col];
+    const int64_t step = (int64_t)kStep * N;
+    // of this thread's first row in the next tile; a column past the matrix reads
+    // the group's first one and is not stored
+    const float *at = dZ + (int64_t)r * N + (col < N ? col : col - c);
+    float x[kSumLoads];
+    auto load = [&](int64_t row0) {
+      if (row0 + kSumRows <= M) {
+#pragma unroll
+        for (int i = 0; i < kSumLoads; ++i) x[i] = at[i * step];
+      } else {
+#pragma unroll
+        for (int i = 0; i < kSumLoads; ++i) x[i] = row0 + r + i * kStep < M ? at[i * step] : 0.0f;
+      }
+      at += kSumLoads * step;
+    };
+    load(0);
+    float s = 0.0f;
+    int half = 0;
+    for (int64_t row0 = 0; row0 < M; row0 += kSumRows, half ^= 1) {
+      float *t = tile[half];
+#pragma unroll
+      for (int i = 0; i < kSumLoads; ++i) t[c * kSumStride + r + i * kStep] = x[i];
+      // one barrier per tile: a buffer is written again only after the next
+      // tile's barrier, which the adding wave reaches when it is done with it
+      __syncthreads();
+      load(row0 + kSumRows);
+      if (threadIdx.x < kSumCols) {
+        const float4 *q = reinterpret_cast<const float4 *>(t + c * kSumStride);
+        const int64_t left = M - row0;
+        const int trips = (int)((left < kSumRows ? left : kSumRows) + 31) / 32;
+        float4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = q[i];
+        for (int j = 1; j <= trips; ++j) {
+          float4 u[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            u[i] = v[i];
+            v[i] = q[8 * (j < trips ? j : 0) + i];   // in flight during the additions
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            s += u[i].x;
+            s += u[i].y;
+            s += u[i].z;
+            s += u[i].w;
+          }
+        }
+      }
     }
-    part[r][c] = s;
-    __syncthreads();
-    if (r == 0 && col < N) {
-      for (int i = 1; i < kSumRows; ++i) s += part[i][c];
-      a.db[k][col] = s;
-    }
-    __syncthreads();
+    if (threadIdx.x < kSumCols && col < N) a.db[k][col] = s;
+    __syncthreads();   // the next group's first tile may take the buffer added last
   }
 }
 
@@ -552,7 +604,7 @@ int cm_colsums(int n, const float *const *dZ, float *const *db, int M, const int
     set_error("cm_colsums: too many columns");
     return -3;
   }
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)(groups < 65536 ? groups : 65536)), dim3(kSumCols * kSumRows), 0,
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)(groups < 65536 ? groups : 65536)), dim3(kSumThreads), 0,
                      stream(), a, n, M, (int)groups);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

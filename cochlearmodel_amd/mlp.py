@@ -78,7 +78,6 @@ class WarmStartMLP:
         self.dZ = [t.empty((B, n), dtype=t.float32, device=d) for n in SIZES[1:-1]]
         self.dZbf = [t.empty((B, n), dtype=t.bfloat16, device=d) for n in SIZES[1:-1]]
         self.rowloss = t.empty(B, dtype=t.float32, device=d)
-        self.loss = t.empty(1, dtype=t.float32, device=d)
         self.gW = [t.empty_like(w) for w in self.W]
         self.gb = [t.empty_like(b) for b in self.b]
 
@@ -118,12 +117,11 @@ class WarmStartMLP:
             kin, kout = SIZES[i], SIZES[i + 1]
             check(L.cm_gemm_bf16_gelu_back(B, kin, kout, ptr(dbf[i]), kout, ptr(self.Wbf[i]), kout,
                                            ptr(self.Z[i - 1]), ptr(self.dZ[i - 1]), ptr(dbf[i - 1]), kin), "gemm dZ")
-        # dW = input^T d, db = colsum(d) of every layer, and the sum of the row losses
+        # dW = input^T d and db = colsum(d) of every layer
         check(L.cm_weight_grads(3, B, (C.c_int * 3)(*SIZES[:-1]), (C.c_int * 3)(*SIZES[1:]),
                                 _ptrs([self.Xbf] + self.Gbf), _ptrs(dbf), _ptrs(self.gW)), "weight grads")
-        check(L.cm_colsums(4, _ptrs(self.dZ + [self.dY, self.rowloss]), _ptrs(self.gb + [self.loss]), B,
-                           (C.c_int * 4)(*SIZES[1:], 1)), "colsums")
-        return self.loss.item() / (B * N_OUT)
+        check(L.cm_colsums(3, _ptrs(self.dZ + [self.dY]), _ptrs(self.gb), B, (C.c_int * 3)(*SIZES[1:])), "colsums")
+        return float(self.rowloss[:B].sum().item()) / (B * N_OUT)
 
     def adam_step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.t += 1
