@@ -129,7 +129,12 @@ __device__ __forceinline__ float tree_sum(float x0, float x1, float x2, float x3
 // one tree alone waits in every step; three interleaved trees never do.  One
 // asm block, because the compiler keeps the trees apart and, for the maximum,
 // adds a canonicalising move and operation per step (values here come from
-// arithmetic, so no operand is a signalling NaN).
+// arithmetic, so no operand is a signalling NaN).  Nor does the compiler see what
+// a block wrote last, so each block ends with the wait states that a reader of it
+// needs: two after v_readlane, for a vector instruction that reads the SGPR, and
+// one after a VGPR, for v_readlane.
+#define CM_SGPR_READY "\n\ts_nop 1"
+#define CM_VGPR_READY "s_nop 0"
 #define CM_TREE3(op0, op1, op2, ctrl)                                   \
   op0 " %0, %0, %0 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
   op1 " %1, %1, %1 " ctrl " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
@@ -144,7 +149,7 @@ __device__ __forceinline__ float tree_sum(float x0, float x1, float x2, float x3
 #define CM_TREE_MAX_SUM_SUM(ctrl) CM_TREE3("v_max_f32_dpp", "v_add_f32_dpp", "v_add_f32_dpp", ctrl)
 #define CM_TREE_SUM3(ctrl) CM_TREE3("v_add_f32_dpp", "v_add_f32_dpp", "v_add_f32_dpp", ctrl)
 #define CM_TREE_READ3 \
-  "v_readlane_b32 %3, %0, 63\n\tv_readlane_b32 %4, %1, 63\n\tv_readlane_b32 %5, %2, 63"
+  "v_readlane_b32 %3, %0, 63\n\tv_readlane_b32 %4, %1, 63\n\tv_readlane_b32 %5, %2, 63" CM_SGPR_READY
 __device__ __forceinline__ void tree_max_sum_sum(float &x, float &y, float &z) {
   float a, b, c;
   asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE_MAX_SUM_SUM) CM_TREE_READ3
@@ -159,7 +164,7 @@ __device__ __forceinline__ void tree_sum3(float &x, float &y, float &z) {
 }
 __device__ __forceinline__ void tree_sum2(float &x, float &y) {
   float a, b;
-  asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE2) "v_readlane_b32 %2, %0, 63\n\tv_readlane_b32 %3, %1, 63"
+  asm("s_nop 1\n\t" CM_TREE_STEPS(CM_TREE2) "v_readlane_b32 %2, %0, 63\n\tv_readlane_b32 %3, %1, 63" CM_SGPR_READY
       : "+&v"(x), "+&v"(y), "=s"(a), "=s"(b));
   x = a; y = b;
 }
@@ -176,17 +181,19 @@ template <int K, bool MAX0, bool ROW>
 __device__ __forceinline__ void tree_row(float (&v)[K]) {
   static_assert(K >= 1 && K <= 3 && !(MAX0 && K != 3), "one to three sums, or a maximum and two sums");
   if constexpr (K == 1) {
-    if constexpr (ROW) asm(CM_ROW_STEPS(CM_TREE1) : "+v"(v[0]));
-    else asm(CM_OCT_STEPS(CM_TREE1) : "+v"(v[0]));
-  } else if constexpr (K == 2) {
+    if constexpr (ROW) asm(CM_ROW_STEPS(CM_TREE1) CM_VGPR_READY : "+v"(v[0]));
+    else asm(CM_OCT_STEPS(CM_TREE1) CM_VGPR_READY : "+v"(v[0]));
+  } else if constexpr (K == 2) {   // CM_TREE2 ends with a wait state
     if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE2) : "+v"(v[0]), "+v"(v[1]));
     else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE2) : "+v"(v[0]), "+v"(v[1]));
   } else if constexpr (MAX0) {
-    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_MAX_SUM_SUM) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
-    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_MAX_SUM_SUM) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    if constexpr (ROW)
+      asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_MAX_SUM_SUM) CM_VGPR_READY : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    else
+      asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_MAX_SUM_SUM) CM_VGPR_READY : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
   } else {
-    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_SUM3) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
-    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_SUM3) : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    if constexpr (ROW) asm("s_nop 1\n\t" CM_ROW_STEPS(CM_TREE_SUM3) CM_VGPR_READY : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
+    else asm("s_nop 1\n\t" CM_OCT_STEPS(CM_TREE_SUM3) CM_VGPR_READY : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]));
   }
 }
 
