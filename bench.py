@@ -325,10 +325,9 @@ def c3_main(args):
     steps, passes, sweeps = ub.stats()
     ms_per_step = 1e3 * wall / args.steps
     bm_avg = float(np.mean(bm_ms))
-    # the same launch without the tuning: one wave per workgroup, natural order,
-    # sweeps in pairs
+    # the same launch without the tuning: natural order, the shape chosen by size
     ub.clear_order()
-    ms_untuned = ub.run_bm(sc, waves_per_block=1)
+    ms_untuned = ub.run_bm(sc)
     flops = flops_per_launch(steps, passes, sweeps)
     lam_bytes = ub.rows * SECTIONS * 16.0
     out = {

@@ -63,6 +63,8 @@ _SIGS = {
     "cudaEventsDestroy": (C.c_int, [vp, vp]),
     "cm_last_kernel_ms": (C.c_float, []),
     "cm_set_bm_launch": (C.c_int, [C.c_int, C.c_int]),
+    "cm_reset_bm_launch": (C.c_int, []),
+    "cm_bm_launch_shape": (C.c_int, [C.c_int, C.c_int, C.c_int, vp, vp, vp]),
     "cm_set_bm_jacobi_unroll": (C.c_int, [C.c_int]),
     "cm_set_bm_sections_per_lane": (C.c_int, [C.c_int]),
     "cm_reset_bm_sections_per_lane": (C.c_int, []),

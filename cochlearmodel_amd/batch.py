@@ -91,7 +91,7 @@ class ToneBatch:
             lib.check(L.cm_set_bm_order(lib.ptr(self.order), len(self.order)), "order")
         lib.check(L.cm_bm_run(C.byref(sc), lib.ptr(self.d_input), self.d_input.numel(), lib.ptr(self.bm.sec),
                               lib.ptr(self.bm.gamma), lib.ptr(self.d_items), self.TB, lib.ptr(self.d_speeds),
-                              self.bufP1, None, None, None, None, None, None, None, None, lib.ptr(self.d_stats), 1, 0,
+                              self.bufP1, None, None, None, None, None, None, None, None, lib.ptr(self.d_stats), 0, 0,
                               1 if timed else 0), "bm")
         return L.cm_last_kernel_ms() if timed else None
 

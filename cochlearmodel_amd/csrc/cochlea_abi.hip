@@ -69,7 +69,7 @@ struct BMHolder {
   int last_blocks = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   float last_kernel_ms = 0.f;
-  int waves_per_block = 1;
+  int waves_per_block = 0;   // blocks per workgroup of BMOHCNewKernel launches (cm_set_bm_launch); 0: by size
   int persistent = 0;
   int jacobi_unroll = 0;   // Jacobi sweep loop unroll of bm_kernel launches (cm_set_bm_jacobi_unroll); 0: by size
   int sections_per_lane = 0;   // block layout of fused-kernel launches (cm_set_bm_sections_per_lane); 0: by size
@@ -143,6 +143,37 @@ void block_decomposition(int TB, int bufP1, int overlap, int DF, std::vector<cm_
   }
 }
 
+// The shape of a launch of n_items blocks: what is asked for (waves per workgroup,
+// unroll and sections per lane above 0), the rest chosen by size.
+struct BmShape {
+  int waves, unroll, sections;
+};
+static BmShape bm_shape(int64_t n_items, int64_t cus, int jacobi_mode, BmShape s) {
+  // Spread a block over four waves where each CU has at most one: its SIMDs
+  // would run one wave or none.  Only the fixed sweeps gain (one exchange
+  // between waves per pass; solving to a tolerance has one per check).
+  // Blocks of 0.2 s of tones, ms for 4 and 2 sections per lane: 10 blocks 91.5
+  // and 85.8, 250 blocks 101.7 and 89.8, 500 blocks 104.7 and 111.2; to a
+  // tolerance 12 blocks 171 and 264.
+  if (s.sections <= 0) s.sections = jacobi_mode == 0 && n_items <= cus ? 2 : 4;
+  // One block per workgroup, but four where that many blocks fill the chip's
+  // SIMDs once or twice: a workgroup's waves go to different SIMDs, single waves
+  // at times to a SIMD that has one already.  ms for one and four, fixed sweeps:
+  // 300 blocks 97.6 and 95.8, 1000 100.0 and 99.9, 2000 152.6 and 150.1; to a
+  // tolerance: 300 227 and 216, 500 186 and 177, 1000 306 and 303, 1500 237 and
+  // 233, 2000 251 and 251; with the extrapolated guess: 300 139 and 134, 500 144
+  // and 137, 1000 164 and 160, 1500 198 and 196, 2000 200 and 200, 3000 257 and
+  // 263 (a workgroup's place is free again when its longest block ends).
+  if (s.waves == 0) s.waves = s.sections == 4 && n_items > cus && n_items <= 8 * cus ? 4 : 1;
+  // Unroll 4 (ten sweeps a trip, step control without branches) where no SIMD has
+  // more than one wave, so that the waits of taken branches are not filled; its
+  // code is larger and does more, and with tolerance checks every few sweeps it
+  // has no long trips.  Fixed sweeps, ms with 2 and 4: 300 blocks 107 and 97, 500
+  // 107 and 99, 1000 108 and 100, 2000 152 and 153, 6000 380 and 390.
+  if (s.unroll <= 0) s.unroll = jacobi_mode == 0 && n_items <= 4 * cus ? 4 : 2;
+  return s;
+}
+
 int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input_len, const float *d_sec,
                     const float *d_gamma, const cm_bm_item *d_items, int n_items, float *d_speeds, int64_t rows,
                     int32_t *failed_nodes, float *ct, float *cl, float *cj, int32_t *fb, float *ctb, float *clb,
@@ -179,32 +210,10 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
   if (order_override) a.order = order_override;
   a.use_queue = persistent ? 1 : 0;
   a.queue = nullptr;
-  const bool trial = sections_per_lane > 0;   // the autotuner's: launched as asked
-  if (!trial) sections_per_lane = g_bm.sections_per_lane;
-  if (sections_per_lane <= 0) {
-    // Spread a block over four waves where each CU has at most one: its SIMDs
-    // would run one wave or none.  Only the fixed sweeps gain (one exchange
-    // between waves per pass; solving to a tolerance has one per check).
-    // Blocks of 0.2 s of tones, ms for 4 and 2 sections per lane: 10 blocks 91.5
-    // and 85.8, 250 blocks 101.7 and 89.8, 500 blocks 104.7 and 111.2; to a
-    // tolerance 12 blocks 171 and 264.
-    sections_per_lane = sc.jacobi_mode == 0 && n_items <= device_cus() ? 2 : 4;
-  }
-  // One block per workgroup unless more are asked for, but four where that many
-  // blocks fill the chip's SIMDs once or twice: a workgroup's waves go to
-  // different SIMDs, single waves often to a SIMD that has one already.  ms for
-  // one and four, fixed sweeps: 250 blocks 107 and 110, 500 111 and 107, 1000 141
-  // and 108, 2000 198 and 152, 3000 211 and 206, 9000 529 and 526; to a tolerance
-  // with the extrapolated guess: 1000 172 and 162, 2000 229 and 198, 3000 254 and
-  // 265 (a workgroup's place is free again when its longest block ends).
-  if (!trial && waves_per_block == 1 && n_items > device_cus() && n_items <= 8 * device_cus()) waves_per_block = 4;
-  // Unroll 4 (ten sweeps a trip, step control without branches) where no SIMD has
-  // more than one wave, so that the waits of taken branches are not filled; its
-  // code is larger and does more, and with tolerance checks every few sweeps it
-  // has no long trips.  Fixed sweeps, ms with 2 and 4: 300 blocks 107 and 97, 500
-  // 107 and 99, 1000 108 and 100, 2000 152 and 153, 6000 380 and 390.
-  if (unroll <= 0) unroll = g_bm.jacobi_unroll;
-  if (unroll <= 0) unroll = sc.jacobi_mode == 0 && n_items <= 4 * device_cus() ? 4 : 2;
+  const BmShape shape = bm_shape(n_items, device_cus(), sc.jacobi_mode,
+                                 {waves_per_block, unroll > 0 ? unroll : g_bm.jacobi_unroll,
+                                  sections_per_lane > 0 ? sections_per_lane : g_bm.sections_per_lane});
+  waves_per_block = shape.waves;
   int grid;
   if (persistent) {
     if (g_bm.queue.ensure(1)) return -1;
@@ -228,7 +237,7 @@ int launch_bm_items(const cm_bm_scalars &sc, const float *d_input, int64_t input
     rc = cm_launch_bm_ws(&a, &w, device_cus(), stream());
     rc = rc > 0 ? 0 : rc;
   } else {
-    rc = cm_launch_bm(&a, waves_per_block, unroll, sections_per_lane, grid, stream());
+    rc = cm_launch_bm(&a, waves_per_block, shape.unroll, shape.sections, grid, stream());
   }
   if (rc) {
     set_error("BM kernel launch failed (%d): %s", rc, hipGetErrorString(hipGetLastError()));
@@ -457,6 +466,24 @@ int cm_reset_bm_jacobi_unroll(void) {
 
 int cm_reset_bm_sections_per_lane(void) {
   g_bm.sections_per_lane = 0;
+  return 0;
+}
+
+int cm_reset_bm_launch(void) {
+  g_bm.waves_per_block = 0;
+  return 0;
+}
+
+int cm_bm_launch_shape(int n_items, int n_cus, int jacobi_mode, int *waves_per_block, int *unroll,
+                       int *sections_per_lane) {
+  if (n_items < 0 || n_cus < 1 || !waves_per_block || !unroll || !sections_per_lane) {
+    set_error("cm_bm_launch_shape: bad arguments");
+    return -3;
+  }
+  const BmShape s = bm_shape(n_items, n_cus, jacobi_mode, {*waves_per_block, *unroll, *sections_per_lane});
+  *waves_per_block = s.waves;
+  *unroll = s.unroll;
+  *sections_per_lane = s.sections;
   return 0;
 }
 

@@ -118,7 +118,7 @@ class BatchedBM:
         self.gamma = torch.from_numpy(np.ascontiguousarray(np.atleast_2d(sets_gamma), np.float32).reshape(-1)).to(
             device)
 
-    def run(self, sc: BMScalars, d_input, items: np.ndarray, rows: int, waves_per_block: int = 1,
+    def run(self, sc: BMScalars, d_input, items: np.ndarray, rows: int, waves_per_block: int = 0,
             persistent: int = 0, timed: bool = False, diagnostics: bool = False, d_speeds=None):
         torch = self.torch
         dev = self.device

@@ -75,7 +75,7 @@ class UnevenBatch:
         self.d_speeds = torch.zeros((self.rows, SECTIONS), dtype=torch.float32, device=dev)
         self.d_stats = torch.zeros(self.TB * 3, dtype=torch.int64, device=dev)
         self.ihc = stages.BatchedIHC(fs, ihc_vectors=list(ihc), device=dev)
-        self.waves_per_block = 1
+        self.waves_per_block = 0   # by size; 1, 2 or 4 after autotune
         self.tuning = None
         self.stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
@@ -94,7 +94,9 @@ class UnevenBatch:
         return out[0]
 
     def clear_order(self):
-        """Back to the untuned launch order, Jacobi unroll and section layout."""
+        """Back to the untuned launch shape: order, Jacobi unroll, section layout
+        and waves per workgroup."""
+        self.waves_per_block = 0
         check(lib().cm_set_bm_order(None, 0), "cm_set_bm_order")
         check(lib().cm_reset_bm_jacobi_unroll(), "cm_reset_bm_jacobi_unroll")
         check(lib().cm_reset_bm_sections_per_lane(), "cm_reset_bm_sections_per_lane")

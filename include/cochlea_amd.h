@@ -58,9 +58,11 @@ float cudaEventsStopQueryTimer(void *start, void *stop, int condition, const cha
 int cudaEventsDestroy(void *start, void *stop);
 /* Duration of the last timed BM launch (Show_Run_Time & 1, or timed=1). */
 float cm_last_kernel_ms(void);
-/* BM launch shape: waves (time blocks) per workgroup (1, the default, leaves the
- * choice of 1 or 4 to the number of blocks), persistent queue. */
+/* BM launch shape of BMOHCNewKernel: waves (time blocks) per workgroup (1, 2 or
+ * 4), persistent queue.  Unset, or after cm_reset_: 4 between one and eight
+ * blocks per CU, 1 elsewhere. */
 int cm_set_bm_launch(int waves_per_block, int persistent);
+int cm_reset_bm_launch(void);
 /* Jacobi sweep loop unroll (1, 2 or 4) of the following bm_kernel launches (no
  * reference counterpart: the reference's sweep loop is
  * include/cochlea.cuh:13962-13982).  Results are identical for every value;
@@ -78,6 +80,11 @@ int cm_reset_bm_jacobi_unroll(void);
  * fixed-sweep launch of no more blocks than the GPU has CUs. */
 int cm_set_bm_sections_per_lane(int sections_per_lane);
 int cm_reset_bm_sections_per_lane(void);
+/* The shape in which a BM launch of n_items blocks runs on a GPU of n_cus CUs: in
+ * *waves_per_block, *unroll and *sections_per_lane what is asked for, 0 for the
+ * choice by size; on return what is launched.  A host calculation. */
+int cm_bm_launch_shape(int n_items, int n_cus, int jacobi_mode, int *waves_per_block, int *unroll,
+                       int *sections_per_lane);
 /* Solver of the BMOHCNewKernel launches (no reference counterpart): jacobi_mode
  * 0 = the reference's fixed sweeps (default), 1 = Jacobi to relative residual
  * tol_rel checked every check_every sweeps, capped at max_sweeps; warm_start 0
@@ -126,7 +133,8 @@ int BMOHCNewKernel(const float *input_samples, int override_input_samples, float
  * launch (src/solver.cpp:312).  The kernel reads input only inside
  * [0, input_len) (zero elsewhere) and writes rows only inside [0, rows); each
  * item's set must index a row of d_gamma (the table is device memory, which
- * the host does not read). */
+ * the host does not read).  waves_per_block: 1, 2 or 4 blocks per workgroup, or
+ * 0 for the choice by size (cm_reset_bm_launch). */
 int cm_bm_run(const cm_bm_scalars *sc, const float *d_input, int64_t input_len, const float *d_sec,
               const float *d_gamma, const cm_bm_item *d_items, int n_items, float *d_speeds, int64_t rows,
               int32_t *d_failed_nodes, float *d_conv_time, float *d_conv_loops, float *d_conv_jacobi,
