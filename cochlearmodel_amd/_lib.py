@@ -71,6 +71,7 @@ _SIGS = {
     "cm_reset_bm_jacobi_unroll": (C.c_int, []),
     "cm_set_bm_order": (C.c_int, [vp, C.c_int]),
     "cm_set_bm_solver": (C.c_int, [C.c_int, f32, C.c_int, C.c_int, C.c_int]),
+    "cm_bm_trial_stride": (C.c_int, [C.c_int, C.c_int, C.c_int]),
     "cm_bm_autotune": (C.c_int, [vp, vp, i64, vp, vp, vp, C.c_int, vp, i64, C.c_int, vp]),
     "BMOHCKernel_Init": (C.c_int, [vp] * 11 + [f32, f32, sz, sz, sz, C.c_int, C.c_int, C.c_int]),
     "BMOHCNewKernel": (C.c_int, [vp, C.c_int, f32, f32, f32, f32, f32, C.c_int, C.c_int, C.c_int, f32, f32, f32,

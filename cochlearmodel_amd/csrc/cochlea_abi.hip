@@ -344,11 +344,28 @@ int cm_set_bm_order(const int32_t *h_order, int n) {
   return 0;
 }
 
+// The stride at which the autotuner samples a table: the caller's, but no more
+// than leaves the sample more than eight blocks per CU, and 1 for tables of fewer.
+// Below that the number of blocks per CU decides which layout, unroll and
+// workgroup is fastest (bm_shape), and a sample of fewer blocks would find another
+// one: 915 uneven blocks, tuned on 229, ran with 2 sections per lane in 188 ms,
+// tuned on all in 113, as untuned (2806: 242 on 702, 237).  A trial of such a table
+// takes about as long for a quarter of its blocks.
+int cm_bm_trial_stride(int n_items, int n_cus, int trial_stride) {
+  if (n_items < 1 || n_cus < 1 || trial_stride < 1) {
+    set_error("cm_bm_trial_stride: bad arguments");
+    return -3;
+  }
+  const int64_t most = ((int64_t)n_items - 1) / (8 * (int64_t)n_cus);
+  return (int)std::max<int64_t>(1, std::min<int64_t>(trial_stride, most));
+}
+
 // Times every launch configuration on a sample of the block table (every
 // trial_stride-th block in longest-first order, so the sample keeps the length
-// mix) and returns the fastest; with order_lpt the full longest-first order is
-// installed for the following launches of this table.  Trial runs write their
-// rows of d_speeds, which the real launch overwrites.
+// mix; fewer are left out where cm_bm_trial_stride says so) and returns the
+// fastest; with order_lpt the full longest-first order is installed for the
+// following launches of this table.  Trial runs write their rows of d_speeds,
+// which the real launch overwrites.
 int cm_bm_autotune(const cm_bm_scalars *sc, const float *d_input, int64_t input_len, const float *d_sec,
                    const float *d_gamma, const cm_bm_item *h_items, int n_items, float *d_speeds, int64_t rows,
                    int trial_stride, cm_bm_tuning *out) {
@@ -356,6 +373,7 @@ int cm_bm_autotune(const cm_bm_scalars *sc, const float *d_input, int64_t input_
     set_error("cm_bm_autotune: bad arguments");
     return -3;
   }
+  trial_stride = cm_bm_trial_stride(n_items, device_cus(), trial_stride);
   std::vector<int32_t> full;
   lpt_order(h_items, n_items, full);
   std::vector<cm_bm_item> sample;

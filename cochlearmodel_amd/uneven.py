@@ -81,8 +81,9 @@ class UnevenBatch:
 
     def autotune(self, sc, trial_stride: int = 4):
         """Pick the sections per lane, Jacobi unroll, waves per workgroup and
-        launch order on a sample of the blocks; the library keeps the section
-        layout, unroll and order for the following launches."""
+        launch order on a sample of the blocks (every trial_stride-th, or more
+        where the sample would have fewer than eight blocks per CU); the library
+        keeps the section layout, unroll and order for the following launches."""
         L = lib()
         L.cm_set_stream(self.stream)
         out = np.zeros(1, TUNING_DTYPE)

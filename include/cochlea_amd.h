@@ -99,11 +99,14 @@ int cm_set_bm_order(const int32_t *h_order, int n);
  * Jacobi unroll x order) on every trial_stride-th block of the table (taken in
  * longest-first order) and reports the fastest; installs its sections per
  * lane and unroll, and the longest-first order when it wins.  Results are
- * identical for every configuration.
+ * identical for every configuration.  A smaller stride is taken where the sample
+ * would not be more than eight blocks per CU (cm_bm_trial_stride, a host
+ * calculation): fewer blocks have another fastest shape.
  * h_items: the block table on the host; d_speeds receives the trial rows. */
 int cm_bm_autotune(const cm_bm_scalars *sc, const float *d_input, int64_t input_len, const float *d_sec,
                    const float *d_gamma, const cm_bm_item *h_items, int n_items, float *d_speeds, int64_t rows,
                    int trial_stride, cm_bm_tuning *out);
+int cm_bm_trial_stride(int n_items, int n_cus, int trial_stride);
 
 /* ---- BM velocity ------------------------------------------------------- */
 /* replaces BMOHCKernel_Init, include/cochlea_common.h:209-230 */
