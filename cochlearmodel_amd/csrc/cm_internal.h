@@ -113,10 +113,14 @@ size_t bm_result_nodes();
 float *bm_input_ptr();
 size_t bm_input_cap();
 int bm_ensure_input(size_t n);
-// IHC/lambda tables (ihc_kernel.hip): one pass possible; table inside the
-// kernel's arguments (then d_ivs may be NULL)
-bool ihc_one_pass(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc);
-bool ihc_table_inline(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc);
+// IHC/lambda calls (ihc_kernel.hip): run in one pass; table inside the kernel's
+// arguments (then d_ivs may be NULL)
+struct IhcBuffers {
+  const float *bm, *scratch, *lambda, *stages;
+  int64_t rows;
+};
+bool ihc_one_pass(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc, const IhcBuffers &b);
+bool ihc_table_inline(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc, const IhcBuffers &b);
 
 }  // namespace cm
 

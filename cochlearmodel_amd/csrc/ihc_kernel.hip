@@ -810,10 +810,11 @@ static int tile_trips(const cm_ihc_interval *h_ivs, int n_ivs, int cus) {
 }
 
 // Runs the whole IHC/lambda chain for one interval table.  One pass wherever
-// every window starts in its interval (kbase 0) and the DC window fits the
-// tiles' halo: 16 B of HBM traffic per node, and the workspace d_scratch (2 x
-// rows x 256 floats: AC, dS) is not touched unless an IIR AC filter writes its
-// AC there first.  Other tables take two passes through the workspace.
+// every window starts in its interval (kbase 0), the DC window fits the tiles'
+// halo and no output lies over the velocity: 16 B of HBM traffic per node, and the
+// workspace d_scratch (2 x rows x 256 floats: AC, dS) is not touched unless an IIR
+// AC filter writes its AC there first.  Other calls take two passes through the
+// workspace.
 // 847 k rows: one pass 1.52 ms, two passes (before the box-car sums and the
 // shorter log10) 3.43 ms.
 extern "C" int cm_launch_ihc_lambda(const float *d_bm, int64_t rows, const cm_ihc_interval *d_ivs,
@@ -843,7 +844,7 @@ extern "C" int cm_launch_ihc_lambda(const float *d_bm, int64_t rows, const cm_ih
   a.rows = rows;
   a.lambda = d_lambda;
   a.stages = d_stages;
-  const bool one_pass = ihc_one_pass(h_ivs, n_ivs, n_dc);
+  const bool one_pass = ihc_one_pass(h_ivs, n_ivs, n_dc, {d_bm, d_scratch, d_lambda, d_stages, rows});
   if (!d_scratch && (!one_pass || iir)) return -3;
   float *AC = d_scratch;
   float *dS = d_scratch ? d_scratch + rows * CM_SECTIONS : nullptr;
@@ -876,17 +877,25 @@ extern "C" int cm_launch_ihc_lambda(const float *d_bm, int64_t rows, const cm_ih
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Whether a table runs in one pass, and whether it then travels in the kernel's
-// arguments (d_ivs NULL) instead of through device memory.
+// Whether a call runs in one pass, and whether its table then travels in the
+// kernel's arguments (d_ivs NULL) instead of through device memory.  One pass
+// writes a tile's outputs while others still read the BM velocity around it, so
+// outputs that lie over the velocity take two passes where there is a workspace:
+// the second reads only that.
 namespace cm {
-bool ihc_one_pass(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc) {
+static bool overlap(const float *a, int64_t na, const float *b, int64_t nb) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return a && b && x < y + (uintptr_t)nb * sizeof(float) && y < x + (uintptr_t)na * sizeof(float);
+}
+bool ihc_one_pass(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc, const IhcBuffers &b) {
   if (n_dc > kHalo + 1) return false;
   for (int i = 0; i < n_ivs; ++i)
     if (h_ivs[i].kbase != 0) return false;
-  return true;
+  const int64_t plane = b.rows * CM_SECTIONS;
+  return !b.scratch || !(overlap(b.bm, plane, b.lambda, 3 * plane) || overlap(b.bm, plane, b.stages, 5 * plane));
 }
-bool ihc_table_inline(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc) {
-  return n_ivs <= kInlineIvs && ihc_one_pass(h_ivs, n_ivs, n_dc);
+bool ihc_table_inline(const cm_ihc_interval *h_ivs, int n_ivs, int n_dc, const IhcBuffers &b) {
+  return n_ivs <= kInlineIvs && ihc_one_pass(h_ivs, n_ivs, n_dc, b);
 }
 }  // namespace cm
 

@@ -201,12 +201,12 @@ static int pad_taps(Buf<double> &dst, const double *d_src, int n) {
 // the interval table in device memory unless it travels with the launch, and
 // zero-padded taps for the two-pass kernels.
 static int prepare_tables(const cm_ihc_interval *h_ivs, int n_ivs, const double *d_ac_b, int n_ac, const double *d_dc,
-                          int n_dc, const cm_ihc_interval **d_ivs) {
+                          int n_dc, const IhcBuffers &b, const cm_ihc_interval **d_ivs) {
   *d_ivs = nullptr;
-  if (ihc_table_inline(h_ivs, n_ivs, n_dc)) return 0;
+  if (ihc_table_inline(h_ivs, n_ivs, n_dc, b)) return 0;
   if (g_st.ivs.upload(h_ivs, n_ivs)) return -1;
   *d_ivs = g_st.ivs.ptr;
-  if (ihc_one_pass(h_ivs, n_ivs, n_dc)) return 0;
+  if (ihc_one_pass(h_ivs, n_ivs, n_dc, b)) return 0;
   return pad_taps(g_st.ac_bpad, d_ac_b, n_ac) || pad_taps(g_st.dcpad, d_dc, n_dc) ? -1 : 0;
 }
 
@@ -244,13 +244,16 @@ int RunIHCKernel(float *host_backup, int Show_Run_Time, int save_lambda, int bac
   }
   std::vector<cm_ihc_interval> fir, iir;
   build_intervals(rows, fir, iir);
-  const cm_ihc_interval *d_ivs = nullptr;
-  if (prepare_tables(fir.data(), (int)fir.size(), g_st.ac_b.ptr, g_st.n_ac, g_st.dc.ptr, g_st.n_dc, &d_ivs)) return -1;
-  if (g_st.is_iir && g_st.iir_ivs.upload(iir.data(), iir.size())) return -1;
   const size_t plane = (size_t)rows * CM_SECTIONS;
   const int want_stages = backup_stage >= 9 && backup_stage <= 14 && host_backup;
   if (want_stages && g_st.stages.ensure(5 * plane)) return -1;
   if (g_st.lambda.ensure(3 * plane) || g_st.scratch.ensure(2 * plane)) return -1;
+  const cm_ihc_interval *d_ivs = nullptr;
+  if (prepare_tables(fir.data(), (int)fir.size(), g_st.ac_b.ptr, g_st.n_ac, g_st.dc.ptr, g_st.n_dc,
+                     {bm_speeds_ptr(), g_st.scratch.ptr, g_st.lambda.ptr, want_stages ? g_st.stages.ptr : nullptr, rows},
+                     &d_ivs))
+    return -1;
+  if (g_st.is_iir && g_st.iir_ivs.upload(iir.data(), iir.size())) return -1;
   int rc = cm_launch_ihc_lambda(bm_speeds_ptr(), rows, d_ivs, fir.data(), (int)fir.size(), g_st.iir_ivs.ptr,
                                 iir.data(), (int)iir.size(), g_st.ac_b.ptr, g_st.ac_bpad.ptr, g_st.is_iir ? g_st.ac_a.ptr : nullptr,
                                 g_st.n_ac, g_st.dc.ptr, g_st.dcpad.ptr, g_st.n_dc, g_st.damage.ptr, g_st.A.ptr, g_st.spont, g_st.sat,
@@ -419,7 +422,8 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
     }
   if (d_ac_a && g_st.iir_ivs.upload(h_iir_ivs, n_iir_ivs)) return -1;
   const cm_ihc_interval *d_ivs = nullptr;
-  if (prepare_tables(h_ivs, n_ivs, d_ac_b, n_ac, d_dc, n_dc, &d_ivs)) return -1;
+  if (prepare_tables(h_ivs, n_ivs, d_ac_b, n_ac, d_dc, n_dc, {d_bm, d_scratch, d_lambda, d_stages, rows}, &d_ivs))
+    return -1;
   const int rc = cm_launch_ihc_lambda(d_bm, rows, d_ivs, h_ivs, n_ivs, g_st.iir_ivs.ptr, h_iir_ivs, n_iir_ivs, d_ac_b,
                                       g_st.ac_bpad.ptr, d_ac_a, n_ac, d_dc, g_st.dcpad.ptr, n_dc, d_damage, d_A, spont3, lambda_sat, eta_ac, eta_dc,
                                       scale_bm, d_scratch, d_lambda, d_stages, stream());
@@ -461,7 +465,7 @@ int cm_ihc_lambda_run_noalloc(const float *d_bm, int64_t rows, const cm_ihc_inte
     }
   }
   cm_ihc_interval *d_ivs = nullptr;
-  if (!ihc_table_inline(h_ivs, n_ivs, n_dc)) {
+  if (!ihc_table_inline(h_ivs, n_ivs, n_dc, {d_bm, nullptr, d_lambda, d_stages, rows})) {
     d_ivs = reinterpret_cast<cm_ihc_interval *>(noalloc_scratch());
     if (!d_ivs) return -1;
     if (check(hipMemcpyAsync(d_ivs, h_ivs, (size_t)n_ivs * sizeof(cm_ihc_interval), hipMemcpyHostToDevice, stream()),

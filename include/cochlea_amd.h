@@ -223,6 +223,7 @@ void *getCudaMeanRate(void);
  * kbase 0 and the DC filter at most 97 taps; d_scratch (2 x rows x 256 floats)
  * holds AC and dS for the two-pass kernels of the other tables, and the AC of
  * an IIR filter.  d_scratch = NULL is refused where one of these needs it.
+ * d_lambda and d_stages may lie over d_bm where d_scratch is given (two passes).
  * Tables of up to 4 intervals travel with the launch (no upload).  With an IIR
  * AC filter (d_ac_a) h_iir_ivs lists the runs the recursion restarts on:
  * rows [row0, row0 + len), period len (CudaIIRFilterDecoupled,
