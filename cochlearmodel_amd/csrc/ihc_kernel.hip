@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   // a box-car DC filter: every tap is the first one
   bool same = true;
-  const double dc0 = a.dc[0];
+  const double dc0 = a.ndc > 0 ? a.dc[0] : 0.0;
   for (int t = lane; t < a.ndc; t += 64) same = same && a.dc[t] == dc0;
   const bool boxcar = a.ndc >= kRows && __builtin_amdgcn_ballot_w64(!same) == 0;
   LambdaNode node;

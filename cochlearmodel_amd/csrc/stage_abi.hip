@@ -388,6 +388,10 @@ int cm_ihc_lambda_run(const float *d_bm, int64_t rows, const cm_ihc_interval *h_
     set_error("cm_ihc_lambda_run: null argument");
     return -3;
   }
+  if (n_ac < 0 || n_dc < 0) {
+    set_error("cm_ihc_lambda_run: negative count (%d AC taps, %d DC taps)", n_ac, n_dc);
+    return -3;
+  }
   if (!d_scratch) {   // the one-pass kernel: FIR AC, windows from each interval's first row, DC in the halo
     if (d_ac_a) {
       set_error("cm_ihc_lambda_run: an IIR AC filter needs the workspace");
