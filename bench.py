@@ -305,10 +305,9 @@ def c3_main(args):
     t_tune = time.perf_counter() - t0
     print(f"# autotune {t_tune:.1f} s: {tune}", file=sys.stderr, flush=True)
     d_lambda = torch.empty((3, ub.rows, SECTIONS), dtype=torch.float32, device="cuda")
-    d_scratch = torch.empty((2, ub.rows, SECTIONS), dtype=torch.float32, device="cuda")
     for _ in range(args.warmup):
         ub.run_bm(sc)
-        ub.run_lambda(d_lambda, d_scratch)
+        ub.run_lambda(d_lambda)
     torch.cuda.synchronize()
     bm_ms, lam_ms = [], []
     t0 = time.perf_counter()
@@ -316,7 +315,7 @@ def c3_main(args):
         bm_ms.append(ub.run_bm(sc))
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record()
-        ub.run_lambda(d_lambda, d_scratch)
+        ub.run_lambda(d_lambda)
         e1.record()
         e1.synchronize()
         lam_ms.append(e0.elapsed_time(e1))
@@ -615,17 +614,13 @@ def c5_main(args):
     """Learned warm start against the plain batched solver on the 4096 held-out
     tones (drawn like the 256-tone grid, seeds disjoint from training), 200 ms
     at 44.1 kHz, 256 sections.  The two launches of 2048 tones stay resident
-    (profiles, inputs, BM velocity, lambda high/medium/low: about 185 GB of
-    HBM with the shared IHC workspace); one step = input synthesis + BM +
+    (profiles, inputs, BM velocity, lambda high/medium/low: about 148 GB of
+    HBM); one step = input synthesis + BM +
     IHC/lambda of one launch, alternating between the two."""
     import torch
     from cochlearmodel_amd import batch
     sets = c5_tone_sets(C5_BATCHES, C5_PER_BATCH)
-    tbs, scratch = [], None
-    for f, db in sets:
-        tb = batch.ToneBatch(f, db, 0.2, d_scratch=scratch)
-        scratch = tb.d_scratch
-        tbs.append(tb)
+    tbs = [batch.ToneBatch(f, db, 0.2) for f, db in sets]
     rows0 = tbs[0].rows
     nb = len(tbs)
     # launch order per variant and batch (each launch installs its own):

@@ -62,10 +62,9 @@ class ToneBatch:
             self.ihc = stages.BatchedIHC(FS)
             self.fir_ivs, _ = stages.reference_intervals(self.rows, self.block, self.TB, self.DF)
             self.d_lambda = torch.empty((3, self.rows, SECTIONS), dtype=torch.float32, device=dev)
-            # the IHC/lambda AC/dS workspace; batches run one after another may share one
-            if d_scratch is None:
-                d_scratch = torch.empty((2, self.rows, SECTIONS), dtype=torch.float32, device=dev)
-            if d_scratch.numel() < 2 * self.rows * SECTIONS:
+            # an IHC/lambda AC/dS workspace of the caller's; the batch's own calls run
+            # in one pass and need none
+            if d_scratch is not None and d_scratch.numel() < 2 * self.rows * SECTIONS:
                 raise ValueError("d_scratch holds fewer than 2 x rows x 256 floats")
             self.d_scratch = d_scratch
         self.stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)

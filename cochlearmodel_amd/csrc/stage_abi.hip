@@ -101,6 +101,11 @@ using namespace cm;
 
 extern "C" {
 
+// Whether RunIHCKernel needs the AC/dS workspace: the intervals of its runs start
+// their windows (kbase 0), so a FIR AC filter and a DC filter that fits go in one
+// pass.
+static bool needs_workspace() { return g_st.is_iir || !ihc_one_pass(nullptr, 0, g_st.n_dc, {}); }
+
 // include/cochlea_common.h:238-274 -> src/cochlea.cu:2417-2598.
 // Nerves_Clusters = {spont[3], (unused)[3], W[3]}.
 int IHCNewKernel(const double *IHC_Damage_Factor, const float *Nerves_Clusters, const double *dc_filter,
@@ -159,7 +164,7 @@ int IHCNewKernel(const double *IHC_Damage_Factor, const float *Nerves_Clusters, 
     }
   }
   const size_t nodes = (size_t)allocateTime * CM_SECTIONS;
-  if (g_st.lambda.ensure(3 * nodes) || g_st.scratch.ensure(2 * nodes)) return -1;
+  if (g_st.lambda.ensure(3 * nodes) || (needs_workspace() && g_st.scratch.ensure(2 * nodes))) return -1;
   if (asMemoryHandlingOnly) return 0;
   return 0;
 }
@@ -247,17 +252,18 @@ int RunIHCKernel(float *host_backup, int Show_Run_Time, int save_lambda, int bac
   const size_t plane = (size_t)rows * CM_SECTIONS;
   const int want_stages = backup_stage >= 9 && backup_stage <= 14 && host_backup;
   if (want_stages && g_st.stages.ensure(5 * plane)) return -1;
-  if (g_st.lambda.ensure(3 * plane) || g_st.scratch.ensure(2 * plane)) return -1;
+  if (g_st.lambda.ensure(3 * plane) || (needs_workspace() && g_st.scratch.ensure(2 * plane))) return -1;
+  float *const scratch_ptr = needs_workspace() ? g_st.scratch.ptr : nullptr;
   const cm_ihc_interval *d_ivs = nullptr;
   if (prepare_tables(fir.data(), (int)fir.size(), g_st.ac_b.ptr, g_st.n_ac, g_st.dc.ptr, g_st.n_dc,
-                     {bm_speeds_ptr(), g_st.scratch.ptr, g_st.lambda.ptr, want_stages ? g_st.stages.ptr : nullptr, rows},
+                     {bm_speeds_ptr(), scratch_ptr, g_st.lambda.ptr, want_stages ? g_st.stages.ptr : nullptr, rows},
                      &d_ivs))
     return -1;
   if (g_st.is_iir && g_st.iir_ivs.upload(iir.data(), iir.size())) return -1;
   int rc = cm_launch_ihc_lambda(bm_speeds_ptr(), rows, d_ivs, fir.data(), (int)fir.size(), g_st.iir_ivs.ptr,
                                 iir.data(), (int)iir.size(), g_st.ac_b.ptr, g_st.ac_bpad.ptr, g_st.is_iir ? g_st.ac_a.ptr : nullptr,
                                 g_st.n_ac, g_st.dc.ptr, g_st.dcpad.ptr, g_st.n_dc, g_st.damage.ptr, g_st.A.ptr, g_st.spont, g_st.sat,
-                                g_st.eta_ac, g_st.eta_dc, g_st.scale, g_st.scratch.ptr, g_st.lambda.ptr,
+                                g_st.eta_ac, g_st.eta_dc, g_st.scale, scratch_ptr, g_st.lambda.ptr,
                                 want_stages ? g_st.stages.ptr : nullptr, stream());
   if (rc) {
     set_error("RunIHCKernel: launch failed (%d)", rc);

@@ -18,6 +18,7 @@ DATA = os.path.join(os.path.dirname(os.path.abspath(__file__)), "data")
 
 # include/const.h:268-297, src/params.cpp:51, 71-73, 111, 123-138
 AIHC_DEFAULT = (70.0, 50.0, 30.0)
+ONE_PASS_DC_TAPS = 97   # DC taps that the one-pass IHC/lambda kernel holds
 SPONT_DEFAULT = (60.0, 3.0, 0.1)
 W_DEFAULT = (0.61, 0.23, 0.16)
 LAMBDA_SAT = 500.0
@@ -135,6 +136,12 @@ def signal_intervals(starts, lengths, sets=None):
     return out
 
 
+def _overlap(a, b):
+    """Whether two contiguous tensors share memory."""
+    return (a.data_ptr() < b.data_ptr() + b.numel() * b.element_size() and
+            b.data_ptr() < a.data_ptr() + a.numel() * a.element_size())
+
+
 class BatchedIHC:
     """Device-resident IHC/lambda through cm_ihc_lambda_run."""
 
@@ -158,15 +165,20 @@ class BatchedIHC:
 
     def run(self, d_bm, rows: int, intervals: np.ndarray, iir_intervals=None, d_lambda=None, d_scratch=None,
             stages=False, workspace=True):
-        """workspace=False runs the one-pass kernel (no AC/dS workspace)."""
+        """The chain runs in one pass, which needs no AC/dS workspace, where every
+        interval has kbase 0, the DC filter at most 97 taps, the AC filter is FIR
+        and no output lies over d_bm.  Other calls take d_scratch, or a workspace
+        of their own unless workspace=False, with which they are refused (outputs
+        over d_bm are not checked then)."""
         torch = self.torch
         dev = self.device
         if d_lambda is None:
             d_lambda = torch.empty((LAMBDA_COUNT, rows, SECTIONS), dtype=torch.float32, device=dev)
-        if d_scratch is None and workspace:
+        ivs = np.ascontiguousarray(intervals, IHC_INTERVAL_DTYPE)
+        if d_scratch is None and workspace and (self.a is not None or self.n_dc > ONE_PASS_DC_TAPS or
+                                                ivs["kbase"].any() or _overlap(d_bm, d_lambda)):
             d_scratch = torch.empty((2, rows, SECTIONS), dtype=torch.float32, device=dev)
         d_st = torch.zeros((5, rows, SECTIONS), dtype=torch.float32, device=dev) if stages else None
-        ivs = np.ascontiguousarray(intervals, IHC_INTERVAL_DTYPE)
         iir = None if iir_intervals is None else np.ascontiguousarray(iir_intervals, IHC_INTERVAL_DTYPE)
         L = lib()
         L.cm_set_stream(C.c_void_p(torch.cuda.current_stream().cuda_stream))
