@@ -616,12 +616,19 @@ __device__ __forceinline__ void fir_rows(const MakeWindow &window, const cm_ihc_
 // first row and the taps - 16 rows before it, which are whole blocks and the
 // end (`part` rows) of one more.  Output i adds rows 1 .. i of the block and
 // the 15 - i rows just before the common ones.  All LDS reads are requested
-// together; the rows before the whole blocks ascend in the ring.  All terms
-// are squares, so each sum is within 40 rounding errors of exact, like the
-// tap-order sum within 98.
+// together; the rows before the whole blocks ascend in the ring.  All terms are
+// squares, so a sum's relative error is at most one unit of 2^-53 for each
+// addition that a term goes through: 15 in its block's sum, one for each whole
+// block and end row of the common ones (4 + 15 at 95 taps), 15 of the rows before
+// for output 0, 49 in all.  The tap-order sum has one per tap.
+constexpr int kWhole = (kHalo + 1 - kRows) / kRows;
+constexpr int kBoxcarRoundings = (kRows - 1) + (kWhole + kRows - 1) + (kRows - 1);
+// relative distance of the two sums, scaled by the tap: theirs and 3 for the
+// product and the two ends of its range
+constexpr double kBoxcarBound = 0x1p-45;
+static_assert(kBoxcarRoundings + (kHalo + 1) + 3 <= 256, "the bound holds 256 units of 2^-53");
 __device__ __forceinline__ void dc_boxcar(const float *col, const double *sums, int blk, int taps,
                                           const float (&ds)[kRows], double (&acc)[kRows]) {
-  constexpr int kWhole = (kHalo + 1 - kRows) / kRows;
   const int whole = (taps - kRows) / kRows, part = (taps - kRows) % kRows;
   double w[kWhole];
 #pragma unroll
@@ -752,14 +759,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (fast) {
         double acc[kRows];
         dc_boxcar(ring.col, sums, blk, a.ndc, ds, acc);
-        // the window sum is within 2^-45 (relative) of the tap-order sum: where
-        // that leaves two floats open, the taps decide
+        // where the sums' distance leaves two floats open, the taps decide
         bool open = false;
 #pragma unroll
         for (int i = 0; i < kRows; ++i) {
           const double y = acc[i] * dc0;
-          dc[i] = (float)(y * (1.0 - 0x1p-45));
-          open = open || dc[i] != (float)(y * (1.0 + 0x1p-45));
+          dc[i] = (float)(y * (1.0 - kBoxcarBound));
+          open = open || dc[i] != (float)(y * (1.0 + kBoxcarBound));
         }
         done = __builtin_amdgcn_ballot_w64(open) == 0;
       }
