@@ -921,7 +921,8 @@ __device__ __forceinline__ int jacobi_tol(Lay<N> &L, const cm_bm_scalars &sc, co
 // The oval window's division by the constant sigma_ow is a product with its
 // reciprocal in FP64: a quotient of two floats is at least 2^-49 (relative)
 // from the midpoint of two floats, the product within 2^-52 of the quotient,
-// so it rounds to the same float (in the normal range).
+// so it rounds to the same float (below the normal range unless sigma_ow is an
+// even integer: only then can a quotient lie on a midpoint there).
 template <int N, class K>
 __device__ __forceinline__ void pass_finish(Lay<N> &L, const K &k, const ItemScal &c, HalfN<N> &n,
                                             const float (&p)[N], const PassTerms<N> &T, float sf) {

@@ -83,7 +83,9 @@ struct JndWave {
 #pragma unroll
     for (int m = 0; m < N; ++m) {
       // (cal - ref) / dA: the FP64 product with the reciprocal rounds to the
-      // same float (a quotient of floats is 2^-49 from any midpoint of two)
+      // same float (a quotient of floats is 2^-49 from any midpoint of two; below
+      // the normal range too unless dA is an even integer, and a dl of that size
+      // squares to 0)
       dl[m] = dA > 0 ? (float)((double)(cal[m] - ref[m]) * inv_dA) : 0.0f;
       sq[m] = dl[m] * dl[m];
       in_range = in_range && (ref[m] > 0x1p-100f && ref[m] < 0x1p100f && sq[m] < __builtin_inff());
