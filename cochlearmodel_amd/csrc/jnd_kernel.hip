@@ -167,8 +167,37 @@ __device__ __forceinline__ double jnd_time(const JndWave &w, float *pre, bool ai
   return acc;
 }
 
-__global__ __launch_bounds__(1024) void jnd_kernel(JndArgs a) {
-  __shared__ float pre_lds[4][2 * kTileRows * 64];
+// A short body's sums by the thread of their section, in the same order: no tiles
+// to fill, and a quarter of the threads.  Returns the Fisher sum.
+__device__ __forceinline__ float jnd_short(const JndWave &w, bool ai, double &acc_c, double &acc_r) {
+  float accv = 0.0f;
+  acc_c = acc_r = 0.0;
+  const float *c = w.c + w.s, *r = w.r + w.s;
+  if (!ai) {
+#pragma unroll 8
+    for (int k = 0; k < w.L; ++k) {
+      acc_c = acc_c + (double)c[(int64_t)k * CM_SECTIONS];
+      acc_r = acc_r + (double)r[(int64_t)k * CM_SECTIONS];
+    }
+    return accv;
+  }
+#pragma unroll 4
+  for (int k = 0; k < w.L; ++k) {
+    const int64_t at = (int64_t)k * CM_SECTIONS;
+    const float cal = c[at], ref = r[at];
+    acc_c = acc_c + (double)cal;
+    acc_r = acc_r + (double)ref;
+    const float dl = w.dA > 0 ? (float)((double)(cal - ref) * w.inv_dA) : 0.0f;
+    const float p = (float)((double)(dl * dl) / (w.a.Fs * (double)ref));
+    accv += p;
+    if (w.node_stage) w.node_stage[at + w.s] = w.stage == 3 ? dl : p;
+  }
+  return accv;
+}
+
+template <bool SHORT>
+__global__ __launch_bounds__(SHORT ? CM_SECTIONS : 1024) void jnd_kernel(JndArgs a) {
+  __shared__ float pre_lds[SHORT ? 1 : 4][SHORT ? 1 : 2 * kTileRows * 64];
   __shared__ double mean_lds[2][CM_SECTIONS];
   __shared__ float fisher_lds[CM_SECTIONS];
   __shared__ float sh[CM_SECTIONS];
@@ -183,11 +212,13 @@ __global__ __launch_bounds__(1024) void jnd_kernel(JndArgs a) {
   float *node_stage = (stage == 3 || stage == 4) ? a.buffer + c : nullptr;
   float ai = 0.f, rms = 0.f;
   if (a.calc_ai || a.calc_rms) {
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = wave >> 2, role = wave & 3;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = SHORT ? wave : wave >> 2, role = wave & 3;
     const int lane = t & 63, s = group * 64 + lane;
     const JndWave w{a, a.lambda + c, a.lambda + r, node_stage, L, s, lane, stage, dAv, 1.0 / (double)dAv};
     float accv;
-    if (role == 0) {
+    if constexpr (SHORT) {
+      fisher_lds[s] = jnd_short(w, a.calc_ai, mean_lds[0][s], mean_lds[1][s]);
+    } else if (role == 0) {
       jnd_time<0>(w, pre_lds[group], a.calc_ai, accv);
       fisher_lds[s] = accv;
     } else if (role == 1) {
@@ -253,11 +284,28 @@ __global__ void calc_dA_kernel(const float *input, float *dA, int n, int interva
 
 }  // namespace cm
 
+// Which bodies are short.  With w workgroups per CU, a tile's barriers are hidden
+// by other workgroups the better the fewer threads each has, so the longest short
+// body grows with w.  us for tiles and for short, Fisher and rate terms: 2
+// intervals of 8 rows 7.8 and 5.9, of 32 rows 8.0 and 10.1; 90 (w = 1.05) of 32
+// 14.8 and 10.9, of 64 20.5 and 24.8; 300 (3.5) of 64 41 and 30, of 256 100 and
+// 103; 700 (8.2) of 128 136 and 122, of 256 240 and 272; 2000 (23) of 512 1158 and
+// 1012.  Rates alone: 90 of 512 38 and 33, of 1024 79 and 83; 300 of 1024 194 and
+// 193, of 2000 364 and 376; 2000 of 2000 2222 and 2151; at w < 1 tiles always.
+static bool short_bodies(const cm::JndArgs &a) {
+  const int64_t n = a.n_intervals, L = a.length_nodes, cus = cm::device_cus();
+  if (a.calc_ai) return L <= 16 || (3 * n > cus && (L - 24) * cus <= 20 * 3 * n);
+  return 3 * n > cus && L * cus <= 512 * 3 * n;
+}
+
 extern "C" int cm_launch_jnd(const cm::JndArgs *a, hipStream_t stream) {
   using namespace cm;
   if (a->n_intervals <= 0) return 0;
   if (a->n_intervals > 0x7fffffff) return -3;
-  hipLaunchKernelGGL(jnd_kernel, dim3(a->n_intervals, 3), dim3(1024), 0, stream, *a);
+  if (short_bodies(*a))
+    hipLaunchKernelGGL((jnd_kernel<true>), dim3(a->n_intervals, 3), dim3(CM_SECTIONS), 0, stream, *a);
+  else
+    hipLaunchKernelGGL((jnd_kernel<false>), dim3(a->n_intervals, 3), dim3(1024), 0, stream, *a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
