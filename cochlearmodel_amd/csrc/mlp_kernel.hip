@@ -362,8 +362,8 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
 // padding spread the columns over the banks).  Rows past the matrix are zeros: a
 // sum that starts at 0 is never -0, so adding them changes nothing.
 // Bound: the chain of one addition per row, about 11 cycles each.  M x (512, 512,
-// 256) in one launch: M = 33 4.3 us, 1024 7.4, 8192 39; one thread per column and
-// nothing in flight took 235 us for 1024 x 512 alone.
+// 256) in one launch: M = 1024 7.4 us, 8192 39; one thread per column took 94 us for
+// 1024 x 512 alone, or 21 with eight loads in flight.
 constexpr int kSumCols = 16, kSumRows = 512, kSumThreads = 1024;
 constexpr int kSumLoads = kSumCols * kSumRows / kSumThreads, kSumStride = kSumRows + 4;
 struct ColSums {
@@ -434,6 +434,25 @@ __global__ __launch_bounds__(kSumThreads) void colsum_kernel(ColSums a, int n, i
     }
     if (threadIdx.x < kSumCols && col < N) a.db[k][col] = s;
     __syncthreads();   // the next group's first tile may take the buffer added last
+  }
+}
+
+// The same sums by one thread per column, 256 columns to a workgroup (`first` counts
+// these): for few rows or very many columns (cm_colsums has the line).  Bound: one
+// thread's loads, eight in flight, or the memory (1e6 columns of 1024 rows 5.8 TB/s).
+constexpr int kWideCols = 256;
+__global__ __launch_bounds__(kWideCols) void colsum_wide_kernel(ColSums a, int n, int M, int groups) {
+  for (int g = blockIdx.x; g < groups; g += gridDim.x) {
+    int k = 0;
+    for (int i = 1; i < n; ++i)
+      if (g >= a.first[i]) k = i;
+    const int64_t N = a.N[k], col = (int64_t)(g - a.first[k]) * kWideCols + threadIdx.x;
+    if (col >= N) continue;
+    const float *__restrict__ at = a.dZ[k] + col;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int m = 0; m < M; ++m, at += N) s += *at;
+    a.db[k][col] = s;
   }
 }
 
@@ -588,7 +607,7 @@ int cm_colsums(int n, const float *const *dZ, float *const *db, int M, const int
     return -3;
   }
   ColSums a{};
-  int64_t groups = 0;
+  int64_t groups = 0;   // of kSumCols columns
   for (int i = 0; i < n; ++i) {
     if (N[i] < 0) {
       set_error("cm_colsums: %d columns", N[i]);
@@ -597,15 +616,31 @@ int cm_colsums(int n, const float *const *dZ, float *const *db, int M, const int
     a.dZ[i] = dZ[i];
     a.db[i] = db[i];
     a.N[i] = N[i];
-    a.first[i] = (int)groups;
     groups += ((int64_t)N[i] + kSumCols - 1) / kSumCols;
   }
   if (groups > INT32_MAX) {
     set_error("cm_colsums: too many columns");
     return -3;
   }
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)(groups < 65536 ? groups : 65536)), dim3(kSumThreads), 0,
-                     stream(), a, n, M, (int)groups);
+  // One thread per column for few rows, and for more of them where the columns
+  // fill the chip: a workgroup of the tiled form takes 6 us whatever it adds, and
+  // two fit on a CU.  us for tiles and threads: 512 columns of 128 rows 6.1 and
+  // 4.5, of 256 6.6 and 6.9, of 1024 7.6 and 21.5; 32768 (4 rounds of the chip) of
+  // 512 25 and 24, of 1024 44 and 46, of 4096 172 and 275; 131072 (16) of 4096 707
+  // and 367.
+  const int64_t rounds = (groups + 2 * device_cus() - 1) / (2 * device_cus());
+  const bool wide = M <= 240 * rounds || rounds > 8;
+  const int cols = wide ? kWideCols : kSumCols;
+  groups = 0;
+  for (int i = 0; i < n; ++i) {
+    a.first[i] = (int)groups;
+    groups += ((int64_t)N[i] + cols - 1) / cols;
+  }
+  const dim3 grid((unsigned)(groups < 65536 ? groups : 65536));
+  if (wide)
+    hipLaunchKernelGGL(colsum_wide_kernel, grid, dim3(kWideCols), 0, stream(), a, n, M, (int)groups);
+  else
+    hipLaunchKernelGGL(colsum_kernel, grid, dim3(kSumThreads), 0, stream(), a, n, M, (int)groups);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

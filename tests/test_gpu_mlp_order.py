@@ -1,6 +1,6 @@
 """Bias gradients add their rows in order, one after another from 0, bit for bit:
-sums of one matrix at the edges of the kernel's tiles (16 columns, 512 rows) and
-the ten first steps of a training run, whose gradients, parameters and outputs
+sums of one matrix at the edges of the kernels' tiles (16 columns, 512 rows; 256
+columns), on either side of the line between them, and the ten first steps of a training run, whose gradients, parameters and outputs
 follow from those sums."""
 import numpy as np
 import pytest
@@ -21,6 +21,7 @@ def _row_order(x):
 
 
 @pytest.mark.parametrize("M,N", [(1, 1), (2, 16), (3, 17), (64, 15), (65, 512), (511, 33), (512, 16), (513, 31),
+                                 (240, 300), (241, 300), (300, 8193), (480, 8193), (481, 8193), (245, 65553),
                                  (1023, 5), (1024, 512), (1025, 769), (2049, 48), (8192, 256)])
 def test_column_sums_add_the_rows_in_order(M, N):
     torch = _cuda()
