@@ -33,8 +33,8 @@ __device__ __forceinline__ float gelu_slope(float x) {
   return 0.5f * (1.0f + t) + 0.5f * x * dt;
 }
 
-// A workgroup owns a 64 x TN tile of C and walks K in steps of 128 G: each of its
-// G groups of 4 waves loads 128 of them, and every element of C is one chain of
+// A workgroup owns a 64 x TN tile of C and walks K in steps of KS G: each of its
+// G groups of 4 waves loads KS of them, and every element of C is one chain of
 // products in the order of k, whatever G is (activations are rounded to BF16
 // after the product: another order of its sum would move some of them by a whole
 // BF16 step).  A step's elements are requested during the products of the step
@@ -54,11 +54,19 @@ __device__ __forceinline__ float gelu_slope(float x) {
 // leave no room for a second.  With a tile more than that, 64 x 64 tiles by 4
 // waves are faster.  M x 512 x 769: M = 1024 (256 tiles) 7.5 us against 10.4,
 // M = 1536 (384) 12.9 against 10.6, M = 8192 46.9 against 24.1.
+// Those take steps of 64 where K is no more: half the loads and LDS, twice the
+// workgroups on a CU.  4096 x 4096 x 64 15.8 us (31.3 in steps of 128), 100000 x 256 x
+// 32 29 (48).  Products of 16 k or fewer and many tiles stay 1.2 to 1.5 times as long
+// as with 2-byte loads and steps of 16 (4096 x 4096 x 8 20 and 16 us).
 // Steps of 16 with 2-byte loads took 110 us at M = 1024; the eight products of a
 // training step at batch 1024 take 47 us (713), 4096 x 4096 x 4096 0.32 ms.
-constexpr int TM = 64, KS = 128, KPAD = 8;
-constexpr int kRowWords = (KS + KPAD) / 2;   // 32-bit words per LDS row
-__device__ __forceinline__ int lds_word(int r, int c) { return r * kRowWords + (c ^ ((r >> 3 & 7) << 3)); }
+constexpr int TM = 64, KPAD = 8;
+// 32-bit words per LDS row of KS elements (64 or 128)
+constexpr int row_words(int KS) { return (KS + KPAD) / 2; }
+template <int KS>
+__device__ __forceinline__ int lds_word(int r, int c) {
+  return r * row_words(KS) + (c ^ ((r >> 3 & (KS / 16 - 1)) << 3));
+}
 
 struct alignas(2) Elems8 {   // 8 elements at element alignment
   uint16_t v[8];
@@ -86,7 +94,7 @@ __device__ __forceinline__ uint4 drop(uint4 v, unsigned d) {
 // memory rows.  Each of a group's 256 threads holds kPieces pieces of 8 elements:
 // along k, or (two k per thread) along the rows.  Rows past the matrix may hold
 // anything, they reach no stored element; k past it is zero.
-template <int ROWS, bool CONTIG_K>
+template <int ROWS, int KS, bool CONTIG_K>
 struct Operand {
   static constexpr int kPieces = ROWS * KS / 8 / 256;
   static constexpr int kLanes = CONTIG_K ? KS / 8 : ROWS / 8;   // pieces along memory
@@ -144,18 +152,18 @@ struct Operand {
 #pragma unroll
       for (int i = 0; i < kPieces; ++i) {
         const int e = tid + 256 * i;
-        *reinterpret_cast<uint4 *>(lds + lds_word(e / kLanes, 4 * (e % kLanes))) = x[i];
+        *reinterpret_cast<uint4 *>(lds + lds_word<KS>(e / kLanes, 4 * (e % kLanes))) = x[i];
       }
     } else {
 #pragma unroll
       for (int i = 0; i < kPieces; i += 2) {
         const int e = tid + 256 * (i >> 1);
-        uint32_t *q = lds + lds_word(8 * (e % kLanes), e / kLanes);
+        uint32_t *q = lds + lds_word<KS>(8 * (e % kLanes), e / kLanes);
         const uint32_t a[4] = {x[i].x, x[i].y, x[i].z, x[i].w}, b[4] = {x[i + 1].x, x[i + 1].y, x[i + 1].z, x[i + 1].w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          q[(2 * j) * kRowWords] = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);       // low halves
-          q[(2 * j + 1) * kRowWords] = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);   // high halves
+          q[(2 * j) * row_words(KS)] = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);       // low halves
+          q[(2 * j + 1) * row_words(KS)] = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);   // high halves
         }
       }
     }
@@ -185,7 +193,7 @@ __device__ __forceinline__ unsigned xcd_order(unsigned blk, unsigned tiles) {
   return xcd * (tiles >> 3) + (xcd < rem ? xcd : rem) + (blk >> 3);
 }
 
-template <int TN, int G, bool TA, bool TB, End END>
+template <int TN, int G, int KS, bool TA, bool TB, End END>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsigned n0) {
   const unsigned M = g_.M, N = g_.N, K = g_.K;
   const uint16_t *__restrict__ A = g_.A, *__restrict__ B = g_.B;
@@ -194,7 +202,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsig
   const float *__restrict__ bias = g_.bias, *__restrict__ Z = g_.Z;
   const float beta = g_.beta;
   uint16_t *__restrict__ Cbf = g_.Cbf;
-  constexpr int kTileWords = (TM + TN) * kRowWords;
+  constexpr int kTileWords = (TM + TN) * row_words(KS);
   // 16 x 16 tiles of a multiplying wave, and those waves' place in the tile
   constexpr int NI = G == 1 ? 2 : 1, NJ = G == 1 ? TN / 32 : 1, kWavesN = TN / (16 * NJ);
   constexpr int kWaves = TM / (16 * NI) * kWavesN;
@@ -203,8 +211,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsig
   const int tid = threadIdx.x & 255, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = wave >> 2;
   const int wm = wave / kWavesN * 16 * NI, wn = wave % kWavesN * 16 * NJ;
-  Operand<TM, !TA> a{A, lda, M, K, m0, {}, {}};
-  Operand<TN, TB> b{B, ldb, N, K, n0, {}, {}};
+  Operand<TM, KS, !TA> a{A, lda, M, K, m0, {}, {}};
+  Operand<TN, KS, TB> b{B, ldb, N, K, n0, {}, {}};
   const int64_t adv_a = TA ? (int64_t)G * KS * lda : G * KS, adv_b = TB ? G * KS : (int64_t)G * KS * ldb;
   f32x4 acc[NI][NJ];
 #pragma unroll
@@ -224,7 +232,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsig
   for (unsigned k0 = 0; k0 < K; k0 += G * KS) {
     if (kg < K) {
       a.store(mine, tid);
-      b.store(mine + TM * kRowWords, tid);
+      b.store(mine + TM * row_words(KS), tid);
     }
     kg += G * KS;
     __syncthreads();
@@ -236,18 +244,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsig
 #pragma unroll
       for (int h = 0; h < G; ++h) {
         if (k0 + h * KS >= K) break;
-        const uint32_t *const ta = lds + h * kTileWords, *const tb = ta + TM * kRowWords;
+        const uint32_t *const ta = lds + h * kTileWords, *const tb = ta + TM * row_words(KS);
 #pragma unroll
         for (int q = 0; q < KS / 32; ++q) {
           bf16x8 fa[NI], fb[NJ];
 #pragma unroll
           for (int i = 0; i < NI; ++i)
             fa[i] =
-                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ta + lds_word(ar + 16 * i, kc + 16 * q)));
+                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ta + lds_word<KS>(ar + 16 * i, kc + 16 * q)));
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
             fb[j] =
-                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tb + lds_word(br + 16 * j, kc + 16 * q)));
+                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(tb + lds_word<KS>(br + 16 * j, kc + 16 * q)));
 #pragma unroll
           for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -287,10 +295,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsig
       }
 }
 
-template <int TN, int G, bool TA, bool TB, End END>
+template <int TN, int G, int KS, bool TA, bool TB, End END>
 __global__ __launch_bounds__(256 * G) void gemm_bf16_kernel(GemmArgs a) {
   const unsigned tile = xcd_order(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-  gemm_tile<TN, G, TA, TB, END>(a, tile / gridDim.x * TM, tile % gridDim.x * TN);
+  gemm_tile<TN, G, KS, TA, TB, END>(a, tile / gridDim.x * TM, tile % gridDim.x * TN);
 }
 
 // Up to kMany products A^T B (weight gradients) in one launch: none of a network's
@@ -308,21 +316,23 @@ __global__ __launch_bounds__(256 * G) void gemm_many_kernel(GemmSet s, int n) {
   for (int i = 1; i < n; ++i)
     if (tile >= s.first[i]) k = i;
   const unsigned t = tile - s.first[k], cols = s.cols[k];
-  gemm_tile<64, G, true, false, End::plain>(s.a[k], t / cols * TM, t % cols * 64);
+  gemm_tile<64, G, 128, true, false, End::plain>(s.a[k], t / cols * TM, t % cols * 64);
 }
 
-template <int TN, int G, bool TA, bool TB, End END>
+template <int TN, int G, int KS, bool TA, bool TB, End END>
 void launch_tiles(const GemmArgs &a) {
   const unsigned cols = (a.N + TN - 1) / TN, rows = (a.M + TM - 1) / TM;
-  hipLaunchKernelGGL((gemm_bf16_kernel<TN, G, TA, TB, END>), dim3(cols, rows), dim3(256 * G), 0, stream(), a);
+  hipLaunchKernelGGL((gemm_bf16_kernel<TN, G, KS, TA, TB, END>), dim3(cols, rows), dim3(256 * G), 0, stream(), a);
 }
 template <bool TA, bool TB, End END = End::plain>
 int launch_gemm(const GemmArgs &a) {
   const int64_t tiles = (((int64_t)a.M + TM - 1) / TM) * (((int64_t)a.N + 31) / 32);
   if (tiles <= device_cus())
-    launch_tiles<32, 4, TA, TB, END>(a);
+    launch_tiles<32, 4, 128, TA, TB, END>(a);
+  else if (a.K <= 64)
+    launch_tiles<64, 1, 64, TA, TB, END>(a);
   else
-    launch_tiles<64, 1, TA, TB, END>(a);
+    launch_tiles<64, 1, 128, TA, TB, END>(a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
