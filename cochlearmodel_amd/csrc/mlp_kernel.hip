@@ -53,15 +53,16 @@ __device__ __forceinline__ float gelu_slope(float x) {
 // a 16 x 16 tile each) as long as every tile has a CU of its own: 104 KiB of LDS
 // leave no room for a second.  With a tile more than that, 64 x 64 tiles by 4
 // waves are faster.  M x 512 x 769: M = 1024 (256 tiles) 7.5 us against 10.4,
-// M = 1536 (384) 12.9 against 10.6, M = 8192 46.9 against 24.1.
-// Those take steps of 64 where K is no more: half the loads and LDS, twice the
-// workgroups on a CU.  4096 x 4096 x 64 15.8 us (31.3 in steps of 128), 100000 x 256 x
-// 32 29 (48).  Products of 16 k or fewer and many tiles stay 1.2 to 1.5 times as long
-// as with 2-byte loads and steps of 16 (4096 x 4096 x 8 20 and 16 us).
+// M = 1536 (384) 12.9 against 10.4, M = 8192 46.9 against 23.2.
+// Those take one step of 32 or 64 where K is no more: fewer loads, less LDS and, with
+// no next step to hold, a quarter of the registers, so many more workgroups on a CU.
+// 4096 x 4096 x 8 14.8 us (20.3 in steps of 64 with a next step), x 32 14.0 (19.5), x 64
+// 15.1 (31.3 in steps of 128), 100000 x 256 x 32 17.9 (28.8); 2-byte loads and steps of 16
+// took 16.1, 19.3, 26.9 and 29.0.
 // Steps of 16 with 2-byte loads took 110 us at M = 1024; the eight products of a
 // training step at batch 1024 take 47 us (713), 4096 x 4096 x 4096 0.32 ms.
 constexpr int TM = 64, KPAD = 8;
-// 32-bit words per LDS row of KS elements (64 or 128)
+// 32-bit words per LDS row of KS elements (32, 64 or 128)
 constexpr int row_words(int KS) { return (KS + KPAD) / 2; }
 template <int KS>
 __device__ __forceinline__ int lds_word(int r, int c) {
@@ -96,7 +97,11 @@ __device__ __forceinline__ uint4 drop(uint4 v, unsigned d) {
 // anything, they reach no stored element; k past it is zero.
 template <int ROWS, int KS, bool CONTIG_K>
 struct Operand {
-  static constexpr int kPieces = ROWS * KS / 8 / 256;
+  static constexpr int kAll = ROWS * KS / 8 / 256;
+  // two k at a time and one piece per thread: half of the threads hold two, the
+  // others the same ones, which they do not store
+  static constexpr bool kTwice = !CONTIG_K && kAll == 1;
+  static constexpr int kPieces = kTwice ? 2 : kAll;
   static constexpr int kLanes = CONTIG_K ? KS / 8 : ROWS / 8;   // pieces along memory
   const uint16_t *p;
   int64_t ld;
@@ -105,10 +110,13 @@ struct Operand {
   uint4 x[kPieces];
 
   __device__ __forceinline__ unsigned row(int i, int tid) const {
-    return CONTIG_K ? r0 + (tid + 256 * i) / kLanes : r0 + 8 * ((tid + 256 * (i >> 1)) % kLanes);
+    return CONTIG_K ? r0 + (tid + 256 * i) / kLanes : r0 + 8 * (pair(i, tid) % kLanes);
   }
   __device__ __forceinline__ unsigned kofs(int i, int tid) const {
-    return CONTIG_K ? 8 * ((tid + 256 * i) % kLanes) : 2 * ((tid + 256 * (i >> 1)) / kLanes) + (i & 1);
+    return CONTIG_K ? 8 * ((tid + 256 * i) % kLanes) : 2 * (pair(i, tid) / kLanes) + (i & 1);
+  }
+  static __device__ __forceinline__ unsigned pair(int i, int tid) {
+    return kTwice ? tid & 127 : tid + 256 * (i >> 1);
   }
   __device__ __forceinline__ void start(unsigned k0, int tid) {
 #pragma unroll
@@ -121,6 +129,12 @@ struct Operand {
     if (k0 + KS <= K && (CONTIG_K || r0 + ROWS <= rows)) {
 #pragma unroll
       for (int i = 0; i < kPieces; ++i) x[i] = vec8(at[i]);
+    } else if (!CONTIG_K && r0 + ROWS <= rows) {   // whole lines, or none
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i) {
+        const unsigned r = row(i, tid), k = k0 + kofs(i, tid);
+        x[i] = k < K ? vec8(p + (int64_t)k * ld + r) : make_uint4(0, 0, 0, 0);
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < kPieces; ++i) {
@@ -154,7 +168,7 @@ struct Operand {
         const int e = tid + 256 * i;
         *reinterpret_cast<uint4 *>(lds + lds_word<KS>(e / kLanes, 4 * (e % kLanes))) = x[i];
       }
-    } else {
+    } else if (!kTwice || tid < 128) {
 #pragma unroll
       for (int i = 0; i < kPieces; i += 2) {
         const int e = tid + 256 * (i >> 1);
@@ -196,6 +210,7 @@ __device__ __forceinline__ unsigned xcd_order(unsigned blk, unsigned tiles) {
 template <int TN, int G, int KS, bool TA, bool TB, End END>
 __device__ __forceinline__ void gemm_tile(const GemmArgs &g_, unsigned m0, unsigned n0) {
   const unsigned M = g_.M, N = g_.N, K = g_.K;
+  if (KS < 128) __builtin_assume(K <= KS);   // one step
   const uint16_t *__restrict__ A = g_.A, *__restrict__ B = g_.B;
   const int lda = g_.lda, ldb = g_.ldb, ldc = g_.ldc;
   float *__restrict__ C = g_.C;
@@ -329,6 +344,8 @@ int launch_gemm(const GemmArgs &a) {
   const int64_t tiles = (((int64_t)a.M + TM - 1) / TM) * (((int64_t)a.N + 31) / 32);
   if (tiles <= device_cus())
     launch_tiles<32, 4, 128, TA, TB, END>(a);
+  else if (a.K <= 32)
+    launch_tiles<64, 1, 32, TA, TB, END>(a);
   else if (a.K <= 64)
     launch_tiles<64, 1, 64, TA, TB, END>(a);
   else
