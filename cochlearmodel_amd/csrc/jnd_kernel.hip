@@ -198,8 +198,8 @@ __device__ __forceinline__ float jnd_short(const JndWave &w, bool ai, double &ac
 template <bool SHORT>
 __global__ __launch_bounds__(SHORT ? CM_SECTIONS : 1024) void jnd_kernel(JndArgs a) {
   __shared__ float pre_lds[SHORT ? 1 : 4][SHORT ? 1 : 2 * kTileRows * 64];
-  __shared__ double mean_lds[2][CM_SECTIONS];
-  __shared__ float fisher_lds[CM_SECTIONS];
+  __shared__ double mean_lds[2][SHORT ? 1 : CM_SECTIONS];
+  __shared__ float fisher_lds[SHORT ? 1 : CM_SECTIONS];
   __shared__ float sh[CM_SECTIONS];
   const int iv = blockIdx.x, li = blockIdx.y, t = threadIdx.x;
   const int ref = a.ref_index[iv];
@@ -214,26 +214,34 @@ __global__ __launch_bounds__(SHORT ? CM_SECTIONS : 1024) void jnd_kernel(JndArgs
   if (a.calc_ai || a.calc_rms) {
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6), group = SHORT ? wave : wave >> 2, role = wave & 3;
     const int lane = t & 63, s = group * 64 + lane;
-    const JndWave w{a, a.lambda + c, a.lambda + r, node_stage, L, s, lane, stage, dAv, 1.0 / (double)dAv};
-    float accv;
+    const JndWave w{a, a.lambda + c, a.lambda + r, node_stage, L, s, lane, stage, dAv, a.calc_ai ? 1.0 / (double)dAv : 0.0};
+    float accv = 0.0f;
+    double acc_c = 0.0, acc_r = 0.0;   // sums of section t
     if constexpr (SHORT) {
-      fisher_lds[s] = jnd_short(w, a.calc_ai, mean_lds[0][s], mean_lds[1][s]);
-    } else if (role == 0) {
-      jnd_time<0>(w, pre_lds[group], a.calc_ai, accv);
-      fisher_lds[s] = accv;
-    } else if (role == 1) {
-      mean_lds[0][s] = jnd_time<1>(w, pre_lds[group], a.calc_ai, accv);
-    } else if (role == 2) {
-      mean_lds[1][s] = jnd_time<2>(w, pre_lds[group], a.calc_ai, accv);
+      accv = jnd_short(w, a.calc_ai, acc_c, acc_r);
     } else {
-      jnd_time<3>(w, pre_lds[group], a.calc_ai, accv);
+      if (role == 0) {
+        jnd_time<0>(w, pre_lds[group], a.calc_ai, accv);
+        fisher_lds[s] = accv;
+      } else if (role == 1) {
+        mean_lds[0][s] = jnd_time<1>(w, pre_lds[group], a.calc_ai, accv);
+      } else if (role == 2) {
+        mean_lds[1][s] = jnd_time<2>(w, pre_lds[group], a.calc_ai, accv);
+      } else {
+        jnd_time<3>(w, pre_lds[group], a.calc_ai, accv);
+      }
+      __syncthreads();
+      if (t < CM_SECTIONS) {
+        accv = fisher_lds[t];
+        acc_c = mean_lds[0][t];
+        acc_r = mean_lds[1][t];
+      }
     }
-    __syncthreads();
     const int64_t ms = ((int64_t)li * a.n_intervals + iv) * CM_SECTIONS + t;   // mean-rate layout
     float mr = 0.0f, dMR = 0.0f, mref = 0.0f;
     if (t < CM_SECTIONS) {
-      mr = (float)mean_lds[0][t] / (float)L;
-      mref = (float)mean_lds[1][t] / (float)L;
+      mr = (float)acc_c / (float)L;
+      mref = (float)acc_r / (float)L;
       a.mean_rate[ms] = mr;
       dMR = (mr - mref) / dAv;
       if (stage == 2) a.buffer[ms] = dMR;
@@ -244,7 +252,7 @@ __global__ __launch_bounds__(SHORT ? CM_SECTIONS : 1024) void jnd_kernel(JndArgs
     }
     if (t < CM_SECTIONS) {
       if (a.calc_ai) {
-        const float rs = 1.0f / __builtin_sqrtf(fisher_lds[t]);
+        const float rs = 1.0f / __builtin_sqrtf(accv);
         ai = (float)((double)(a.T / a.Tlength) * a.nIHC[t] / (double)(rs * rs));
         if (stage == 5) a.buffer[ms] = ai;
       }
@@ -286,16 +294,23 @@ __global__ void calc_dA_kernel(const float *input, float *dA, int n, int interva
 
 // Which bodies are short.  With w workgroups per CU, a tile's barriers are hidden
 // by other workgroups the better the fewer threads each has, so the longest short
-// body grows with w.  us for tiles and for short, Fisher and rate terms: 2
-// intervals of 8 rows 7.8 and 5.9, of 32 rows 8.0 and 10.1; 90 (w = 1.05) of 32
-// 14.8 and 10.9, of 64 20.5 and 24.8; 300 (3.5) of 64 41 and 30, of 256 100 and
-// 103; 700 (8.2) of 128 136 and 122, of 256 240 and 272; 2000 (23) of 512 1158 and
-// 1012.  Rates alone: 90 of 512 38 and 33, of 1024 79 and 83; 300 of 1024 194 and
-// 193, of 2000 364 and 376; 2000 of 2000 2222 and 2151; at w < 1 tiles always.
+// body grows with w; and a CU holds one workgroup of tiles at a time, so that just
+// above 3 per CU the fourth round costs tiles more.  us for tiles and for short,
+// Fisher and rate terms, each interval with another reference: 2 intervals of 8 rows
+// 7.8 and 5.9, of 32 rows 8.0 and 10.1; 90 (w = 1.05) of 32 14.8 and 10.9, of 80 25.5
+// and 33.4; 200 (2.3) of 80 40 and 35, of 96 40 and 41; 300 (3.5) of 96 53 and 44, of
+// 160 73 and 69, of 256 104 and 107; 500 (5.9) of 160 111 and 77, of 256 164 and 164;
+// 805 (9.4) of 256 270 and 289; 2000 (23) of 512 1158 and 1012.
+// Rates alone leave tiles two of four waves: 41 (0.5) of 8820 361 and 682; 100 (1.2) of
+// 700 68 and 56, of 8820 920 and 806 (with one reference for all, which stays in the
+// caches, 737 and 783); 200 of 8820 1587 and 1585 (1163 and 1133); 805 of 1500 1062
+// and 1069.
 static bool short_bodies(const cm::JndArgs &a) {
   const int64_t n = a.n_intervals, L = a.length_nodes, cus = cm::device_cus();
-  if (a.calc_ai) return L <= 16 || (3 * n > cus && (L - 24) * cus <= 20 * 3 * n);
-  return 3 * n > cus && L * cus <= 512 * 3 * n;
+  if (!a.calc_ai) return 3 * n > cus;
+  if (L <= 16) return true;
+  const int64_t over = (L - 24) * cus;
+  return 3 * n > cus && (over <= 25 * 3 * n || (n > cus && L <= 240 && over <= 36 * 3 * n));
 }
 
 extern "C" int cm_launch_jnd(const cm::JndArgs *a, hipStream_t stream) {

@@ -101,3 +101,12 @@ def test_stage_dumps(oracle, length):
                                    for i in range(n)])
             got, want = got[:, body], want[:, body]
         np.testing.assert_array_equal(got, want, err_msg=f"stage {k}")
+
+
+@pytest.mark.parametrize("n,length", [(100, 53), (100, 54), (256, 99), (256, 100), (257, 132), (257, 133), (300, 150),
+                                      (300, 151), (600, 240), (600, 241), (85, 600), (86, 700)])
+@pytest.mark.parametrize("ai,rms", [(1, 1), (0, 1)])
+def test_either_side_of_the_lines_by_rounds(oracle, n, length, ai, rms):
+    if length > 500 and ai:
+        pytest.skip("the line of rates alone")
+    test_either_side_of_the_line(oracle, n, length, ai, rms)
