@@ -62,12 +62,24 @@ class ToneBatch:
             self.ihc = stages.BatchedIHC(FS)
             self.fir_ivs, _ = stages.reference_intervals(self.rows, self.block, self.TB, self.DF)
             self.d_lambda = torch.empty((3, self.rows, SECTIONS), dtype=torch.float32, device=dev)
-            # an IHC/lambda AC/dS workspace of the caller's; the batch's own calls run
-            # in one pass and need none
             if d_scratch is not None and d_scratch.numel() < 2 * self.rows * SECTIONS:
                 raise ValueError("d_scratch holds fewer than 2 x rows x 256 floats")
-            self.d_scratch = d_scratch
+            self._scratch = d_scratch
         self.stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    @property
+    def d_scratch(self):
+        """An IHC/lambda AC/dS workspace of the batch's size, for a caller's own calls:
+        the one given, else allocated when it is first asked for.  The batch's calls
+        run in one pass and need none."""
+        if self._scratch is None:
+            self._scratch = self.torch.empty((2, self.rows, SECTIONS), dtype=self.torch.float32,
+                                             device=self.d_lambda.device)
+        return self._scratch
+
+    @d_scratch.setter
+    def d_scratch(self, scratch):
+        self._scratch = scratch
 
     def device_profiles(self, freqs, levels):
         """Another set of n tones' profiles, resident on the device, for
@@ -107,7 +119,7 @@ class ToneBatch:
             t["bm_ms"] = ms
         e2.record()
         if self.with_lambda:
-            self.ihc.run(self.d_speeds, self.rows, self.fir_ivs, d_lambda=self.d_lambda, d_scratch=self.d_scratch)
+            self.ihc.run(self.d_speeds, self.rows, self.fir_ivs, d_lambda=self.d_lambda, d_scratch=self._scratch)
         e3 = torch.cuda.Event(enable_timing=True)
         e3.record()
         e3.synchronize()

@@ -48,3 +48,13 @@ def test_tone_batches_hold_none():
     assert torch.cuda.memory_allocated() - before < 4.5 * tb.rows * 1024
     with pytest.raises(ValueError):
         batch.ToneBatch([500.0], [60.0], 0.2, d_scratch=torch.empty(8, device="cuda"))
+
+
+def test_tone_batches_give_one_when_asked():
+    torch = _cuda()
+    from cochlearmodel_amd import batch
+    tb = batch.ToneBatch([500.0], [60.0], 0.04)
+    ws = tb.d_scratch
+    assert ws.shape == (2, tb.rows, 256) and ws.dtype == torch.float32 and ws.is_cuda
+    assert tb.d_scratch is ws
+    assert batch.ToneBatch([2000.0], [40.0], 0.04, d_scratch=ws).d_scratch is ws
